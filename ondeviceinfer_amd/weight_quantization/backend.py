@@ -480,7 +480,8 @@ class CompressedLinearBackend:
             if self.name in FUSED_BACKENDS:
                 prepared = weights[prefix + '._prepared']
                 k, n = prepared.k, prepared.n
-                x = inputs.reshape(-1, k).contiguous()
+                flat = inputs.dim() == 2 and inputs.shape[1] == k
+                x = (inputs if flat else inputs.reshape(-1, k)).contiguous()
                 if self.marlin_max_rows_per_call <= 0 or x.shape[0] <= self.marlin_max_rows_per_call:
                     out = self._fused(x, prepared)
                 else:
@@ -488,7 +489,7 @@ class CompressedLinearBackend:
                     for start in range(0, x.shape[0], self.marlin_max_rows_per_call):
                         end = min(start + self.marlin_max_rows_per_call, x.shape[0])
                         self._fused(x[start:end], prepared, out[start:end])
-                return out.reshape(*inputs.shape[:-1], n)
+                return out if flat else out.reshape(*inputs.shape[:-1], n)
             weight = decode_weight(weights, name, group_size=self.group_size)
             self.explicit_dequant_bytes += weight.numel() * weight.element_size()
             if self.name == 'reference_w8a8':
