@@ -98,17 +98,18 @@ int wq_w4_decode_rows(const int32_t* weight_packed, const float* weight_scale,
 /* Workspace bytes wq_w4a16_linear can use for this shape (0 when it needs
  * none).  The workspace holds the arrival counters and fp32 partials of the
  * kernels that split a tile's k range over several workgroups: the decode
- * GEMV (m <= 4), the small-batch kernel (12 <= m <= 32 on n <= 18432) and the
- * deep-ring GEMM on the smallest prefill grids (m > 64 on narrow n).  The
- * counters sit in a fixed 16 KiB region at the start, so one buffer sized for
- * the largest shape serves every shape.  It must be zero-filled once before
- * first use; every call leaves the counters zeroed again, so it can be
- * reused by later calls (and graph replays) on the same stream.  Calls that
- * may run concurrently need separate workspaces.  With a NULL or smaller
- * workspace the linear runs without the split (the decode GEMV keeps each
- * tile in one workgroup: same result; at 12 <= m <= 32 the skinny kernels,
- * and the deep-ring GEMM over the whole k range: the same values up to fp32
- * summation order).  Replaces
+ * GEMV (m <= 4), the kernel of 5 to 64 rows and the deep-ring GEMM on the
+ * smallest prefill grids (m > 64 on narrow n).  The counters sit in a fixed
+ * 16 KiB region at the start, so one buffer sized for the largest shape
+ * serves every shape.  It must be zero-filled once before first use
+ * (5 <= m <= 64 uses counters only at 12 <= m <= 32 with n <= 18432,
+ * k <= 8192 and k % 512 == 0; elsewhere any scratch will do); every call
+ * leaves the counters zeroed again, so it can be reused by later calls (and
+ * graph replays) on the same stream.  Calls that may run concurrently need
+ * separate workspaces.  With a NULL or smaller workspace the linear runs
+ * without the split (the decode GEMV keeps each tile in one workgroup: same
+ * result; at 5 <= m <= 64 the skinny kernels, and the deep-ring GEMM over the
+ * whole k range: the same values up to fp32 summation order).  Replaces
  * marlin_make_workspace_new (backend.py:223). */
 int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t group_size, size_t* bytes);
 
@@ -204,7 +205,8 @@ int wq_w8_decode(const int8_t* qweight, const float* scale, int64_t n, int64_t k
                  uint16_t* weight, void* stream);
 
 /* Workspace bytes wq_w8a16_linear can use (same contract as
- * wq_w4a16_workspace_size).  Replaces the fp16 dequant scratch sizing of
+ * wq_w4a16_workspace_size: m <= 4 the decode GEMV, 5 <= m <= 64 the kernel
+ * of 5 to 64 rows).  Replaces the fp16 dequant scratch sizing of
  * QuantizedCpuWeightStore.max_dequant_elements (runtime/quantized.py:90-96),
  * with far less memory. */
 int wq_w8a16_workspace_size(int64_t m, int64_t n, int64_t k, size_t* bytes);

@@ -316,6 +316,11 @@ def shared_workspace(device: torch.device, nbytes: int, layout: tuple) -> torch.
     return buf
 
 
+def _counts_arrivals(m: int, n: int, k: int) -> bool:
+    """The 5-to-64-row W4 shapes whose split needs zeroed counters (``mid_counts`` in ``csrc/wq_mid.hip``)."""
+    return 12 <= m <= 32 and n <= 18432 and k <= 8192 and k % 512 == 0
+
+
 def w4a16_linear(x: torch.Tensor, tiles: torch.Tensor, meta: torch.Tensor, n: int, group_size: int,
                  out: torch.Tensor | None = None, workspace: torch.Tensor | None = None) -> torch.Tensor:
     """``y[m, n] = x[m, k] . dequant(W)^T`` on the repacked weight."""
@@ -331,10 +336,14 @@ def w4a16_linear(x: torch.Tensor, tiles: torch.Tensor, meta: torch.Tensor, n: in
         if out.data_ptr() % 16:
             raise ValueError('out must be 16-byte aligned')
     if workspace is None and (nbytes := w4a16_workspace_size(m, n, k, group_size)):
-        # M > 4, the small-batch kernel's and the deep-ring GEMM's split
-        # partials: their counters sit in a fixed region at the front and are
-        # zero after every call, so all such shapes share one buffer.
-        workspace = shared_workspace(device, nbytes, ('w4a16', m, n, k, group_size) if m <= 4 else ('w4a16-split',))
+        if 4 < m <= 64 and not _counts_arrivals(m, n, k):
+            # Split partials only (no counters): any scratch of this call's own.
+            workspace = x.new_empty(nbytes, dtype=torch.uint8)
+        else:
+            # M > 4, counted splits and the deep-ring GEMM's: their counters
+            # sit in a fixed region at the front and are zero after every
+            # call, so all such shapes share one buffer.
+            workspace = shared_workspace(device, nbytes, ('w4a16', m, n, k, group_size) if m <= 4 else ('w4a16-split',))
     ws_ptr, ws_bytes = None, 0
     if workspace is not None:
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
@@ -604,8 +613,11 @@ def w8a16_linear(x: torch.Tensor, qweight, scale: torch.Tensor, bias: torch.Tens
         out = torch.empty((m, n), dtype=torch.float16, device=device)
     else:
         _check(out, torch.float16, (m, n), 'out')
-    if workspace is None and m <= 4:
-        workspace = shared_workspace(device, w8a16_workspace_size(m, n, k), ('w8a16', m, n, k))
+    if workspace is None and m <= 64 and (nbytes := w8a16_workspace_size(m, n, k)):
+        if m <= 4:
+            workspace = shared_workspace(device, nbytes, ('w8a16', m, n, k))
+        else:   # split partials only (no counters): any scratch of this call's own
+            workspace = x.new_empty(nbytes, dtype=torch.uint8)
     ws_ptr, ws_bytes = None, 0
     if workspace is not None:
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()

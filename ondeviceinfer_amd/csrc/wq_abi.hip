@@ -18,7 +18,8 @@ void set_error(const char* fmt, ...) {
 }
 
 size_t gemv_workspace_bytes(bool w4, int64_t m, int64_t n, int64_t k);
-size_t w4_batch_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t g);
+size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
+size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
                      half_t* y, void* ws, size_t ws_bytes, hipStream_t s);
 int launch_w8_skinny(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
@@ -85,9 +86,9 @@ extern "C" int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t 
   if (int st = linear_shape_check(m, n, k)) return st;
   WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");
   size_t need = gemv_workspace_bytes(true, m, n, k);
-  const size_t batch = w4_batch_workspace_bytes(m, n, k, group_size);
+  const size_t mid = w4_mid_workspace_bytes(m, n, k);
   const size_t gemm = m > kSkinnyMaxM && k <= kGemmMaxK ? w4_gemm_workspace_bytes(m, n, k) : 0;
-  if (batch > need) need = batch;
+  if (mid > need) need = mid;
   if (gemm > need) need = gemm;
   *bytes = need;
   return WQ_OK;
@@ -96,7 +97,10 @@ extern "C" int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t 
 extern "C" int wq_w8a16_workspace_size(int64_t m, int64_t n, int64_t k, size_t* bytes) {
   if (int st = linear_shape_check(m, n, k)) return st;
   WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");
-  *bytes = k % kW8BlockK == 0 ? gemv_workspace_bytes(false, m, n, k) : 0;
+  size_t need = k % kW8BlockK == 0 ? gemv_workspace_bytes(false, m, n, k) : 0;
+  const size_t mid = w8_mid_workspace_bytes(m, n, k);
+  if (mid > need) need = mid;
+  *bytes = need;
   return WQ_OK;
 }
 
@@ -325,7 +329,7 @@ extern "C" int wq_w8a16_linear_tiled(const uint16_t* x, int64_t m, int64_t k, co
 // Allocation-free W4A16 linear (wq_w4a16_linear_noalloc).
 //
 // The k-split counters and fp32 partials of the split kernels (decode GEMV,
-// small-batch kernel, deep-ring GEMM) live in this file-scope device array
+// 5-to-64-row kernel, deep-ring GEMM) live in this file-scope device array
 // instead of a caller workspace.  Each GPU holds its own copy for the life of
 // the process.  Host code never passes `scratch` itself to a kernel: the name
 // is only a host-side handle, so every use goes through the device address
@@ -402,7 +406,7 @@ extern "C" int wq_w4a16_linear_noalloc(const uint16_t* x, int64_t m, int64_t k, 
   if (int st = linear_shape_check(m, n, k)) return st;
   if (m == 0) return wq_w4a16_linear(x, m, k, tiles, meta, n, group_size, y, nullptr, 0, stream);
   // The same sizing as wq_w4a16_workspace_size: every split plan (decode
-  // GEMV, small-batch kernel, deep-ring GEMM) fits kSplitWorkspaceMaxBytes,
+  // GEMV, 5-to-64-row kernel, deep-ring GEMM) fits kSplitWorkspaceMaxBytes,
   // so this runs the plan a caller workspace would.
   size_t need = 0;
   if (int st = wq_w4a16_workspace_size(m, n, k, group_size, &need)) return st;

@@ -89,7 +89,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int
 constexpr int kNtPolicy = 2;   // non-temporal: data streamed once
 
 // Workspace layout shared by every kernel that splits a tile's k range over
-// workgroups (decode GEMV, small-batch kernel, deep-ring GEMM): uint32
+// workgroups (decode GEMV, 5-to-64-row kernel, deep-ring GEMM): uint32
 // arrival counters in this fixed region at the start, then that kernel's
 // fp32 partials.  Every call leaves the counters it used at zero, and no
 // kernel's partials reach into the region, so one buffer can serve all the

@@ -921,8 +921,10 @@ int launch_w4_gemv_flat(const half_t* x, int M, int K, const uint4_t* tiles, con
 
 }  // namespace
 
-int launch_w4_batch(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
-                    void* ws, size_t ws_bytes, hipStream_t st);
+int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
+                  void* ws, size_t ws_bytes, hipStream_t st);
+int launch_w8_mid(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
+                  half_t* y, void* ws, size_t ws_bytes, hipStream_t st, int tiled);
 
 int launch_w4_gemv_fused(const half_t* x, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
                          int x_mode, const half_t* norm_w, const float* sumsq_in, int sumsq_count, float eps,
@@ -964,8 +966,8 @@ int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const 
     int rc = launch_w4_gemv_flat(x, M, K, tiles, meta, N, G, y, ws, ws_bytes, s);
     if (rc != kNotApplicable) return rc;
   } else {
-    // 12 <= M <= 32 on narrow N: activations shared in LDS (wq_batch.hip).
-    int rc = launch_w4_batch(x, M, K, tiles, meta, N, G, y, ws, ws_bytes, s);
+    // Activations shared in LDS (wq_mid.hip).
+    int rc = launch_w4_mid(x, M, K, tiles, meta, N, G, y, ws, ws_bytes, s);
     if (rc != kNotApplicable) return rc;
   }
   const int mc = (M + 15) / 16;
@@ -987,6 +989,9 @@ int launch_w8_skinny(const half_t* x, int M, int K, const int8_t* q, const half_
                      half_t* y, void* ws, size_t ws_bytes, hipStream_t s, int tiled) {
   if (M <= kGemvFlatMaxM) {
     int rc = launch_gemv_flat<WFmt::W8>(x, M, K, q, scale, bias, N, tiled, y, ws, ws_bytes, s);
+    if (rc != kNotApplicable) return rc;
+  } else {
+    int rc = launch_w8_mid(x, M, K, q, scale, bias, N, y, ws, ws_bytes, s, tiled);
     if (rc != kNotApplicable) return rc;
   }
   const int mc = (M + 15) / 16;

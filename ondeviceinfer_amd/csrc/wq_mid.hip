@@ -1,0 +1,477 @@
+// Batches of 5 to 64 rows: W4A16 and W8A16 linears whose activations are
+// staged once per workgroup in LDS and shared by its tile waves.
+//
+// Bound: a weight stream (HBM) as long as the activations stay cheap.  The
+// skinny kernels give every wave its own copy of the activation fragments, so
+// at M = 49..64 a wave moves 16 KiB of x from L2 for every 2 KiB of W4
+// weights; here a workgroup moves M * 256 B of x per 128-k block once for its
+// eight 16-row tiles.  Workgroup (g, s) = 8 waves owns tile group g (128
+// rows of W) over the k range s of S:
+//  * wave (p, h) takes the tile pair p (two tiles, so that an x fragment read
+//    from LDS feeds two MFMAs; one tile per wave would make the LDS reads the
+//    bound) and the 128-k blocks of parity h, which halves the number of
+//    barriers per block; the two parities meet in LDS at the end;
+//  * a stage is two blocks: its x goes buffer -> LDS (rows past M read as
+//    zero, 16-byte chunk c of row r at slot c ^ (r & 15)), its weights straight
+//    into registers, D - 1 stages ahead (D = 3, and 2 where 48 or 64 rows fill
+//    the LDS and the registers: a deeper ring measured no faster there);
+//  * per block the skinny kernels' arithmetic: W4 the exact fp16 (q - z) on
+//    MFMA 16x16x32, then the group scale times the block sum added in fp32;
+//    INT8 the exact fp16 q, the row scale applied to the final sum.
+// Few tile groups leave compute units idle, so the k range is split until
+// about one workgroup per compute unit runs (mid_splits); each split stores
+// its fp32 partials with device-coherent stores and a second small launch
+// adds them in split order.  Against a last-arriver sum inside this kernel
+// (arrival counters, as the deep-ring GEMM) that is 0.3-0.8 us slower at some
+// W4 shapes and 0.4-4 us faster at N = 1024 and on INT8, and it needs no
+// zeroed counters, so any scratch of the call's own will do.  The short W4
+// shapes of 12 to 32 rows keep the last arriver (mid_counts): they finish
+// before the host has queued a second launch (fused QKV M = 24 called from
+// Python 11.5 us against 13.3).
+// MI355X, graphs of distinct weights, us, previous kernel -> this one:
+//   W4 17408->5120  M = 8 / 24 / 40 / 56   20.2 / 35.1 / 48.9 / 64.3 -> 15.0 / 17.3 / 20.8 / 24.0
+//   W4 5120->7168   M = 24 / 40 / 56       12.4 / 17.9 / 22.8 -> 11.7 / 14.0 / 16.0
+//   W4 5120->17408  M = 8 / 24 / 40 / 56   22.2 / 27.2 / 39.6 / 55.4 -> 17.6 / 20.6 / 22.9 / 30.2
+//   INT8 17408->5120  M = 8 / 24 / 56      31.5 / 36.5 / 65.6 -> 19.4 / 20.9 / 28.9
+//   INT8 5120->17408  M = 8 / 24 / 56      25.4 / 36.1 / 70.1 -> 20.7 / 25.9 / 31.7
+// i.e. 46 MB of W4 weights at M = 8 in 15.0 us (3.1 TB/s) and 89 MB of INT8
+// weights in 20.7 us (4.3 TB/s); what remains is about 6 us of launch, first
+// load and partial sum, then 0.75 us (M <= 16) to 1.3 us (M = 64, bound by
+// issue: 32 MFMAs, 120 VALU and 20 LDS operations per wave) a stage.
+#include "wq_common.h"
+#include "wq_status.h"
+
+namespace wq {
+namespace {
+
+enum class MFmt { W4, W8 };
+
+constexpr int kMidWaves = 8;
+constexpr int kMidTilesPerWave = 2;
+constexpr int kMidGroupTiles = 4 * kMidTilesPerWave;   // tiles per workgroup
+// Largest k: 64 rows of x stay inside the 31-bit buffer range.
+constexpr int64_t kMidMaxK = 1 << 23;
+static_assert(1152 / kMidGroupTiles <= kSplitMaxCounters, "one counter per tile group");
+constexpr int kMidSumDepth = 8;                        // split partials requested at once by the final sum
+
+template <int N>
+__device__ __forceinline__ void mid_wait_vm() {
+  static_assert(N >= 0 && N <= 63, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+// The MC fragments of one k-step (16 rows apart inside a stage), read and
+// waited for in one asm block.
+template <int MC>
+__device__ __forceinline__ void mid_read(uint4_t (&f)[MC], uint32_t a) {
+  if constexpr (MC == 1)
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(f[0]) : "v"(a));
+  else if constexpr (MC == 2)
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]) : "v"(a));
+  else if constexpr (MC == 3)
+    asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:4096\n\tds_read_b128 %2, %3 offset:8192\n\t"
+                 "s_waitcnt lgkmcnt(0)" : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]) : "v"(a));
+  else
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:4096\n\tds_read_b128 %2, %4 offset:8192\n\t"
+                 "ds_read_b128 %3, %4 offset:12288\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]) : "v"(a));
+}
+
+// Columns n0 .. n0 + 3 of row m (N % 8 == 0 for W4; INT8 takes any N and
+// stores the quad at once when row m keeps 8-byte alignment).
+template <MFmt F>
+__device__ __forceinline__ void mid_store(float4_t s, int m, int n0, int M, int N, const void* __restrict__ wmeta,
+                                          const half_t* __restrict__ bias, half_t* __restrict__ y) {
+  if (m >= M || n0 >= N) return;
+  half4_t o;
+  if constexpr (F == MFmt::W4) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = (half_t)s[v];
+    *reinterpret_cast<half4_t*>(y + (size_t)m * N + n0) = o;
+  } else {
+    const half_t* scale = reinterpret_cast<const half_t*>(wmeta);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int n = min(n0 + v, N - 1);
+      float r = s[v] * (float)scale[n];
+      if (bias) r += (float)bias[n];
+      o[v] = (half_t)r;
+    }
+    if ((N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+      *reinterpret_cast<half4_t*>(y + (size_t)m * N + n0) = o;
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (n0 + v < N) y[(size_t)m * N + n0 + v] = o[v];
+    }
+  }
+}
+
+// One wave's weights of one 128-k block.
+template <MFmt F>
+struct MidRegs;
+template <>
+struct MidRegs<MFmt::W4> {
+  uint4_t w[kMidTilesPerWave];
+  uint2_t s[kMidTilesPerWave];
+  uint32_t z[kMidTilesPerWave];
+};
+template <>
+struct MidRegs<MFmt::W8> {
+  uint4_t a[kMidTilesPerWave], b[kMidTilesPerWave];
+};
+
+template <MFmt F, int MC, int D, int MINW>
+__global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
+    const half_t* __restrict__ x, int M, int K, const void* __restrict__ wsrc, const void* __restrict__ wmeta, int N,
+    int bpg, const half_t* __restrict__ bias, half_t* __restrict__ y, float4_t* ws_part, uint32_t* ws_cnt, int tiled) {
+  constexpr int NT = kMidTilesPerWave;
+  constexpr int kSubBytes = MC * 16 * 256;      // one 128-k block of x
+  constexpr int kStageBytes = 2 * kSubBytes;
+  constexpr int kLoads = MC + (F == MFmt::W4 ? 3 : 2) * NT;   // per wave and stage
+  constexpr int kUnits = 4 * NT * MC;           // 1 KiB accumulator units of the workgroup
+  static_assert(D >= 2 && (D - 2) * kLoads <= 63, "ring depth");
+  static_assert(kUnits * 1024 <= D * kStageBytes, "the parity sum reuses the ring");
+  __shared__ __attribute__((aligned(1024))) uint8_t xs[D * kStageBytes];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p = wave & 3, h = wave >> 2;
+  const int i = lane & 15, kb = lane >> 4;
+  const int ntile = (N + 15) >> 4;
+  const int nblk = K / kW4BlockK, nst = (nblk + 1) >> 1;
+  const int group = blockIdx.x, split = blockIdx.y, S = gridDim.y;
+  const int st_lo = (split * nst) / S, nloc = ((split + 1) * nst) / S - st_lo;
+  const int tile0 = (group * 4 + p) * NT;
+  constexpr uint32_t kPastEnd = 0x80000000u;
+
+  uint32_t xvo[MC];
+#pragma unroll
+  for (int j = 0; j < MC; ++j) {
+    const int rr = 4 * (p * MC + j) + (lane >> 4);
+    xvo[j] = (uint32_t)(rr * K * 2 + ((lane & 15) ^ (rr & 15)) * 16);
+  }
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, (int64_t)M * K * 2);
+
+  const int ngrp = F == MFmt::W4 ? nblk / bpg : 0;
+  __amdgpu_buffer_rsrc_t rw, rm;
+  if constexpr (F == MFmt::W4) {
+    rw = buf_rsrc(reinterpret_cast<const uint8_t*>(wsrc) + (size_t)tile0 * nblk * 1024,
+                  (int64_t)(ntile - tile0) * nblk * 1024);
+    rm = buf_rsrc(reinterpret_cast<const uint8_t*>(wmeta) + (size_t)tile0 * ngrp * kW4MetaBytes,
+                  (int64_t)(ntile - tile0) * ngrp * kW4MetaBytes);
+  } else {
+    rw = tiled ? buf_rsrc(reinterpret_cast<const int8_t*>(wsrc) + (size_t)tile0 * nblk * kW8TileBlockBytes,
+                          (int64_t)(ntile - tile0) * nblk * kW8TileBlockBytes)
+               : buf_rsrc(reinterpret_cast<const int8_t*>(wsrc) + (size_t)tile0 * 16 * K, (int64_t)(N - tile0 * 16) * K);
+    rm = rw;
+  }
+  // Stages are requested in order, so the next block, its group and the
+  // group's remainder advance by two blocks a stage (no division per stage).
+  int nx = 2 * st_lo + h;
+  const int nx_end = min(2 * (st_lo + nloc), nblk);
+  int gq = F == MFmt::W4 ? nx / bpg : 0, gr = F == MFmt::W4 ? nx - gq * bpg : 0;
+  const int gq2 = F == MFmt::W4 ? 2 / bpg : 0, gr2 = F == MFmt::W4 ? 2 - gq2 * bpg : 0;
+  const uint32_t wvo = F == MFmt::W4 || tiled ? (uint32_t)lane * 16 : (uint32_t)(i * K + 16 * kb);
+  const uint32_t wstep = F == MFmt::W4 ? 1024 : tiled ? kW8TileBlockBytes : kW8BlockK;
+  const uint32_t wtile = F == MFmt::W4 ? (uint32_t)nblk * 1024 : tiled ? (uint32_t)nblk * kW8TileBlockBytes : (uint32_t)(16 * K);
+  auto fetch = [&](int st, MidRegs<F>& r) {
+    const bool live = nx < nx_end;
+    const uint32_t xo = live ? (uint32_t)nx * 256 : kPastEnd;
+#pragma unroll
+    for (int j = 0; j < MC; ++j)
+      lds_load16(rx, xvo[j], xo, xs + st * kStageBytes + h * kSubBytes + (p * MC + j) * 1024);
+    const uint32_t wo = live ? (uint32_t)nx * wstep : kPastEnd;
+    if constexpr (F == MFmt::W4) {
+      const uint32_t mo = live ? (uint32_t)(gq * kW4MetaBytes) : kPastEnd;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        r.w[t] = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo, wo + t * wtile, kNtPolicy);
+        r.s[t] = __builtin_bit_cast(uint2_t, __builtin_amdgcn_raw_buffer_load_b64(rm, (uint32_t)kb * 8, mo + t * ngrp * kW4MetaBytes, 0));
+        r.z[t] = __builtin_amdgcn_raw_buffer_load_b32(rm, 32 + (uint32_t)(i >> 3) * 4, mo + t * ngrp * kW4MetaBytes, 0);
+      }
+      gq += gq2;
+      gr += gr2;
+      if (gr >= bpg) {
+        gr -= bpg;
+        ++gq;
+      }
+    } else {
+      const uint32_t p1 = tiled ? kW8TileBlockBytes / 2 : 64;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        r.a[t] = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo, wo + t * wtile, kNtPolicy);
+        r.b[t] = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo + p1, wo + t * wtile, kNtPolicy);
+      }
+    }
+    nx += 2;
+  };
+
+  float4_t acc[NT][MC];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mc = 0; mc < MC; ++mc) acc[t][mc] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const uint32_t xs_base = (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)xs) +
+                           (uint32_t)(h * kSubBytes + i * 256);
+
+  auto block = [&](int st, const MidRegs<F>& r) {
+    float4_t cg[NT][MC];
+    uint32_t c_lo[NT], c_hi[NT];
+    if constexpr (F == MFmt::W4) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        w4_zero_consts((r.z[t] >> (4 * (i & 7))) & 0xFu, c_lo[t], c_hi[t]);
+#pragma unroll
+        for (int mc = 0; mc < MC; ++mc) cg[t][mc] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    const uint32_t base = xs_base + (uint32_t)(st * kStageBytes);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      uint4_t f[MC];
+      // k-step w's 16-byte chunk of this lane, at slot chunk ^ row (row & 15 = i)
+      const int c = F == MFmt::W4 ? 4 * kb + w : 2 * kb + (w & 1) + 8 * (w >> 1);
+      mid_read<MC>(f, base + (uint32_t)((c ^ i) * 16));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        half8_t a;
+        if constexpr (F == MFmt::W4) {
+          const uint32_t word = w == 0 ? r.w[t].x : w == 1 ? r.w[t].y : w == 2 ? r.w[t].z : r.w[t].w;
+          a = w4_word_to_h8(word, c_lo[t], c_hi[t]);
+        } else {
+          const uint4_t& v = w < 2 ? r.a[t] : r.b[t];
+          a = (w & 1) == 0 ? i8x8_to_h8(v.x, v.y) : i8x8_to_h8(v.z, v.w);
+        }
+#pragma unroll
+        for (int mc = 0; mc < MC; ++mc) {
+          if constexpr (F == MFmt::W4) cg[t][mc] = mfma16(a, __builtin_bit_cast(half8_t, f[mc]), cg[t][mc]);
+          else acc[t][mc] = mfma16(a, __builtin_bit_cast(half8_t, f[mc]), acc[t][mc]);
+        }
+      }
+    }
+    if constexpr (F == MFmt::W4) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const half4_t s4 = __builtin_bit_cast(half4_t, r.s[t]);
+#pragma unroll
+        for (int mc = 0; mc < MC; ++mc)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[t][mc][v] += (float)s4[v] * cg[t][mc][v];
+      }
+    }
+  };
+
+  MidRegs<F> wr[D];
+#pragma unroll
+  for (int j = 0; j < D - 1; ++j) {
+    fetch(j, wr[j]);
+    __builtin_amdgcn_sched_barrier(0);   // loads stay in stage order: the waits below count them
+  }
+  mid_wait_vm<(D - 2) * kLoads>();
+  __builtin_amdgcn_s_barrier();
+  int base = 0;
+  do {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      fetch((u + D - 1) % D, wr[(u + D - 1) % D]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (base + u < nloc) block(u, wr[u]);
+      mid_wait_vm<(D - 2) * kLoads>();
+      __builtin_amdgcn_s_barrier();
+    }
+    base += D;
+  } while (base < nloc);
+  mid_wait_vm<0>();            // the run-out's empty copies have landed ...
+  __builtin_amdgcn_s_barrier();   // ... everyone's: the ring is dead
+
+  // Unit (p, t, mc) at 1 KiB granules: the odd-block waves hand theirs over.
+  float4_t* red = reinterpret_cast<float4_t*>(xs);
+  if (h == 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int mc = 0; mc < MC; ++mc) red[((p * NT + t) * MC + mc) * 64 + lane] = acc[t][mc];
+  }
+  __syncthreads();
+  if (h == 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int mc = 0; mc < MC; ++mc) {
+        const int unit = (p * NT + t) * MC + mc;
+        const float4_t s = acc[t][mc] + red[unit * 64 + lane];
+        if (S == 1) mid_store<F>(s, mc * 16 + i, (group * kMidGroupTiles + p * NT + t) * 16 + 4 * kb, M, N, wmeta, bias, y);
+        else coherent_store16(ws_part, (uint32_t)(((group * S + split) * kUnits + unit) * 1024 + lane * 16),
+                              __builtin_bit_cast(uint4_t, s));
+      }
+  }
+  if constexpr (F == MFmt::W4 && MC <= 2) {
+    if (ws_cnt == nullptr) return;   // uniform: S == 1, or mid_sum_kernel adds the partials
+    // The last of the group's S workgroups to arrive adds the partials, in
+    // split order, and stores y.
+    __builtin_amdgcn_s_waitcnt(0);   // this wave's partials are acknowledged
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();                 // ... and every wave's; the sums above are read
+    uint32_t* arrival = reinterpret_cast<uint32_t*>(xs);
+    if (threadIdx.x == 0)
+      *arrival = __hip_atomic_fetch_add(&ws_cnt[group], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*arrival != (uint32_t)(S - 1)) return;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    static_assert(kUnits == MC * kMidWaves, "MC units per wave");
+    constexpr int Q = 8 / MC;        // splits of each unit requested at once
+    float4_t sum[MC];
+    for (int s0 = 0; s0 < S; s0 += Q) {
+      float4_t v[MC][Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q)   // past the last split: that split again, not added
+#pragma unroll
+        for (int u = 0; u < MC; ++u)
+          v[u][q] = __builtin_bit_cast(
+              float4_t, coherent_load16(ws_part, (uint32_t)(((group * S + min(s0 + q, S - 1)) * kUnits + wave +
+                                                             u * kMidWaves) * 1024 + lane * 16)));
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (s0 + q < S)
+#pragma unroll
+          for (int u = 0; u < MC; ++u) sum[u] = s0 + q == 0 ? v[u][q] : sum[u] + v[u][q];
+    }
+#pragma unroll
+    for (int u = 0; u < MC; ++u) {
+      const int unit = wave + u * kMidWaves;
+      mid_store<F>(sum[u], (unit % MC) * 16 + i, (group * kMidGroupTiles + unit / MC) * 16 + 4 * kb, M, N, wmeta, bias, y);
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(&ws_cnt[group], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The S partials of every unit, in split order.  One wave per unit, all of a
+// lane's loads (up to six) in flight at once.
+template <MFmt F, int MC>
+__global__ __launch_bounds__(256) void mid_sum_kernel(const float4_t* __restrict__ part, int S, int M, int N,
+                                                      const void* __restrict__ wmeta, const half_t* __restrict__ bias,
+                                                      half_t* __restrict__ y) {
+  constexpr int kUnits = kMidGroupTiles * MC;
+  constexpr int Q = 5;   // partials after the first requested at once
+  const int lane = threadIdx.x & 63, i = lane & 15, kb = lane >> 4;
+  const int gu = blockIdx.x * 4 + (threadIdx.x >> 6);   // group * kUnits + unit
+  const int group = gu / kUnits, unit = gu % kUnits;
+  const int m = (unit % MC) * 16 + i, n0 = (group * kMidGroupTiles + unit / MC) * 16 + 4 * kb;
+  if (m >= M || n0 >= N) return;
+  const float4_t* q = part + ((size_t)group * S * kUnits + unit) * 64 + lane;
+  float4_t s = q[0];
+  for (int s0 = 1; s0 < S; s0 += Q) {
+    float4_t v[Q];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) v[j] = q[(size_t)min(s0 + j, S - 1) * kUnits * 64];   // past the last: not added
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+      if (s0 + j < S) s += v[j];
+  }
+  mid_store<F>(s, m, n0, M, N, wmeta, bias, y);
+}
+
+// Splits of the k range (two-block stages) over workgroups: one workgroup per
+// compute unit (256) for up to 128 tile groups, at most 2/5 of a split per
+// stage (shorter ranges are all start-up: N = 1024, K = 5120 8 splits of 2.5
+// stages).  Beyond 128 groups the grid covers more than half of the machine by
+// itself and the splits only even out its rounds: three up to 170 groups (408
+// workgroups on the gate / up shape), two above.  INT8 at M <= 32 keeps the
+// whole range up to 170 groups: its 96 KiB of weights in flight per workgroup
+// saturate memory from 136 compute units (5120->17408 M = 8 20.7 us against
+// 23.2 with three splits), which W4's half does not (18.4 against 17.4).
+int mid_splits(bool w4, int64_t M, int64_t N, int64_t K) {
+  const int mc = (int)((M + 15) / 16);
+  const int64_t groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles, nst = (K / kW4BlockK + 1) / 2;
+  int64_t s = groups <= 128 ? 256 / groups : groups > 170 ? 2 : !w4 && mc <= 2 ? 1 : 3;
+  if (s > nst * 2 / 5) s = nst * 2 / 5;
+  if (s > 16) s = 16;
+  while (s > 1 && kSplitCounterBytes + (size_t)(groups * s) * kMidGroupTiles * mc * 1024 > kSplitWorkspaceMaxBytes) --s;
+  return s < 1 ? 1 : (int)s;
+}
+
+// The shapes this file takes, from both sides' measurements.  W4: from 12
+// rows on, below 2048 tiles (there the deep-ring GEMM stays ahead: fused
+// gate_up M = 24 / 56 36 / 50 us against 38 / 59), and from 5 rows where the
+// k chain is long or N is wide (17408->5120 M = 8 20.2 -> 15.0 us, 5120->17408
+// 22.2 -> 17.6; fused QKV M = 8 8.2 against 10.2 the other way).  At 33 to 35
+// rows short chains stay on the skinny kernels: their workspace query answers
+// 0 bytes just past 32 rows, which callers may rely on.  INT8: everything but
+// narrow N at M <= 16 (N = 1024 M = 8 6.6 us against 8.6).
+bool mid_takes(bool w4, int64_t M, int64_t N, int64_t K) {
+  if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return false;
+  const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
+  if (!w4) return M > 16 || ntile >= 128;
+  if (ntile >= 2048) return false;
+  if (M < 12) return nblk >= 64 || ntile >= 1024;
+  return nblk >= 64 || M < 33 || M > 35;
+}
+
+// Whether the last arriver sums (W4, mid_kernel's ws_cnt): 12 to 32 rows on up
+// to 1152 tiles and k chains of 4 to 64 blocks (a multiple of four), the
+// shapes whose workspace carried zeroed counters before this kernel.
+bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
+  const int64_t nblk = K / kW4BlockK;
+  return w4 && M >= 12 && M <= 32 && (N + 15) / 16 <= 1152 && nblk <= 64 && nblk % 4 == 0;
+}
+
+size_t mid_ws_bytes(bool w4, int64_t M, int64_t N, int64_t K) {
+  if (!mid_takes(w4, M, N, K)) return 0;
+  const int s = mid_splits(w4, M, N, K);
+  if (s <= 1) return 0;
+  const int64_t groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles;
+  return kSplitCounterBytes + (size_t)(groups * s) * kMidGroupTiles * ((M + 15) / 16) * 1024;
+}
+
+template <MFmt F, int MC, int D, int MINW>
+int launch_mid(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* bias,
+               half_t* y, void* ws, int S, int tiled, hipStream_t st) {
+  const int groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles;
+  // The partials start past the counter region that other split kernels keep
+  // at zero in a shared workspace.
+  float4_t* part = S > 1 ? reinterpret_cast<float4_t*>(reinterpret_cast<uint8_t*>(ws) + kSplitCounterBytes) : nullptr;
+  uint32_t* cnt = S > 1 && mid_counts(F == MFmt::W4, M, N, K) ? reinterpret_cast<uint32_t*>(ws) : nullptr;
+  hipLaunchKernelGGL((mid_kernel<F, MC, D, MINW>), dim3((unsigned)groups, (unsigned)S), dim3(64 * kMidWaves), 0, st, x,
+                     M, K, w, meta, N, bpg, bias, y, part, cnt, tiled);
+  if (S > 1 && cnt == nullptr)
+    hipLaunchKernelGGL((mid_sum_kernel<F, MC>), dim3((unsigned)(groups * kMidGroupTiles * MC / 4)), dim3(256), 0, st,
+                       part, S, M, N, meta, bias, y);
+  return check_launch(F == MFmt::W4 ? "w4_mid" : "w8_mid");
+}
+
+// Returns -1 (not taken) when the shape is not this file's or its splits need
+// more workspace than given; the caller then runs the skinny kernels.
+template <MFmt F>
+int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* bias,
+                    half_t* y, void* ws, size_t ws_bytes, int tiled, hipStream_t st) {
+  constexpr bool w4 = F == MFmt::W4;
+  if (!mid_takes(w4, M, N, K)) return -1;
+  const size_t need = mid_ws_bytes(w4, M, N, K);
+  if (need > 0 && (ws == nullptr || ws_bytes < need)) return -1;
+  const int S = mid_splits(w4, M, N, K);
+  switch ((M + 15) / 16) {
+    case 1: return launch_mid<F, 1, 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
+    case 2: return launch_mid<F, 2, 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
+    case 3: return launch_mid<F, 3, w4 ? 2 : 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
+    default: return launch_mid<F, 4, 2, 2>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
+  }
+}
+
+}  // namespace
+
+size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(true, m, n, k); }
+size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(false, m, n, k); }
+
+int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
+                  void* ws, size_t ws_bytes, hipStream_t st) {
+  return launch_mid_auto<MFmt::W4>(x, M, K, tiles, meta, N, G / kW4BlockK, nullptr, y, ws, ws_bytes, 0, st);
+}
+
+int launch_w8_mid(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
+                  half_t* y, void* ws, size_t ws_bytes, hipStream_t st, int tiled) {
+  return launch_mid_auto<MFmt::W8>(x, M, K, q, scale, N, 1, bias, y, ws, ws_bytes, tiled, st);
+}
+
+}  // namespace wq

@@ -1,0 +1,104 @@
+"""GPU parity of the 5-to-64-row linears (wq_mid.hip) against the CPU oracle at
+the edges of its 16-row chunks, tile groups, stages and splits.
+
+Bars as in test_gpu_parity.py (``oracle.qdq.parity_ok``); the two INT8 layouts
+run the same plan and must give the same bits."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qdq, synth
+from ondeviceinfer_amd import _native
+from ondeviceinfer_amd.weight_quantization import backend as wq
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (5, 16, 17, 33, 36, 48, 49, 64)   # both ends of the 16-row chunks (33..35: skinny on short chains)
+
+
+def dev(a, device):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(device)
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def check_parity(actual, expected, label):
+    m = qdq.parity_metrics(actual, expected)
+    print(label, {k: (round(v, 8) if isinstance(v, float) else v) for k, v in m.items()}, flush=True)
+    assert qdq.parity_ok(m), (label, m)
+
+
+# (n, k, group, symmetric): one block (the odd parity idle); a partial last tile
+# group (1000 rows = 63 tiles) over 31 blocks, and over 66 with groups of 384 =
+# three blocks (stages start inside a group); whole groups of 256 blocks wide;
+# 1088 tiles (three splits); 1600 tiles (two splits).
+@pytest.mark.parametrize('n,k,g,sym', [(512, 128, 128, False), (1000, 3968, 128, False), (1000, 8448, 384, True),
+                                       (2048, 2560, 256, False), (17408, 1280, 128, False),
+                                       (25600, 1280, 128, True)])
+def test_w4_mid_matches_oracle(gpu, n, k, g, sym):
+    name = 'p.weight'
+    weights, x = synth.w4_case(n, k, max(ROWS), seed=n % 89 + k, group_size=g, symmetric=sym, name=name)
+    layer = {key: dev(v, gpu) for key, v in weights.items()}
+    backend = wq.CompressedLinearBackend('marlin', group_size=g)
+    backend.prepare(layer, name)
+    w32 = qdq.decode_weight(weights, name, group_size=g).astype(np.float32)
+    for m in ROWS:
+        y = host(backend.linear(dev(x[:m], gpu), layer, name))
+        check_parity(y, (x[:m].astype(np.float32) @ w32.T).astype(np.float16), f'w4 mid n={n} k={k} g={g} m={m}')
+
+
+@pytest.mark.parametrize('n,k', [(512, 128), (1001, 3968), (2050, 8448), (17408, 1280), (34816, 640)])
+def test_w8_mid_matches_oracle_in_both_layouts(gpu, n, k):
+    _, q, s, x = synth.int8_case(n, k, max(ROWS), seed=n % 97 + k)
+    qd, sd = dev(q, gpu), dev(s, gpu)
+    tiles = _native.w8_repack(qd)
+    w32 = qdq.dequantize_linear_weight(q, s).astype(np.float32)
+    bias = (np.random.default_rng(k).standard_normal(n) * 0.1).astype(np.float16)
+    for m in ROWS:
+        xd = dev(x[:m], gpu)
+        y = _native.w8a16_linear(xd, tiles, sd, bias=dev(bias, gpu))
+        assert torch.equal(y, _native.w8a16_linear(xd, qd, sd, bias=dev(bias, gpu)))
+        expected = (x[:m].astype(np.float32) @ w32.T + bias.astype(np.float32)).astype(np.float16)
+        check_parity(host(y), expected, f'w8 mid n={n} k={k} m={m}')
+
+
+def test_mid_splits_run_on_two_streams_at_once_and_under_capture(gpu):
+    """Every call brings its own partials: calls on two streams that overlap,
+    and replays of two captured graphs, equal the calls made one by one; a
+    workspace too small for the splits runs the skinny kernels within the bar."""
+    gen = torch.Generator(device=gpu).manual_seed(3)
+    w = wq.CompressedLinearBackend('w8a16')
+    layer = {'p.weight': torch.randint(-127, 128, (5120, 5120), generator=gen, device=gpu).to(torch.int8),
+             'p.weight_scale': torch.rand(5120, 1, generator=gen, device=gpu) * 1e-3 + 1e-4}
+    w.prepare(layer, 'p.weight')
+    xs = [torch.randn(40, 5120, generator=gen, device=gpu).half() for _ in range(2)]
+    refs = [w.linear(x, layer, 'p.weight').clone() for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    outs = [[], []]
+    for _ in range(8):
+        for s, x, o in zip(streams, xs, outs):
+            with torch.cuda.stream(s):
+                o.append(w.linear(x, layer, 'p.weight'))
+    torch.cuda.synchronize()
+    for o, ref in zip(outs, refs):
+        assert all(torch.equal(y, ref) for y in o)
+    graphs, ys = [], []
+    for s, x in zip(streams, xs):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            ys.append(w.linear(x, layer, 'p.weight'))
+        graphs.append(g)
+    for _ in range(3):
+        for g, s, y in zip(graphs, streams, ys):
+            with torch.cuda.stream(s):
+                y.zero_()
+                g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, ref) for y, ref in zip(ys, refs))
+    p = layer['p._prepared']
+    small = _native.w8a16_linear(xs[0], p.qweight, p.scale, workspace=torch.empty(16, dtype=torch.uint8, device=gpu))
+    check_parity(host(small), host(refs[0]).astype(np.float32), 'skinny fallback')
