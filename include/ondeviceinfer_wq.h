@@ -292,6 +292,16 @@ int wq_w8a8_linear(const int8_t* qx, const float* x_scale, int64_t m, int64_t k,
 int wq_w8a8_linear_tiled(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const void* tiles,
                          const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y, void* stream);
 
+/* wq_w8a8_linear (tiled == 0) / wq_w8a8_linear_tiled (tiled != 0) with a
+ * workspace of wq_w8a8_workspace_size bytes (any scratch, no zero-filling;
+ * NULL or smaller: the kernels without the split) for the int32 partials of
+ * the kernel that splits the k range at 5 <= m <= 255.  Same results, bit for
+ * bit.  The reference's call has no workspace (backend.py:254). */
+int wq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k, size_t* bytes);
+int wq_w8a8_linear_ws(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const void* weight,
+                      int32_t tiled, const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

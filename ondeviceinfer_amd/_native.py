@@ -72,6 +72,8 @@ _SIGNATURES = {
     'wq_w8a16_linear': [_P, _I64, _I64, _P, _P, _I64, _P, _P, _P, ctypes.c_size_t, _P],
     'wq_w8a8_quantize': [_P, _I64, _I64, _P, _P, _P],
     'wq_w8a8_linear': [_P, _P, _I64, _I64, _P, _P, _I64, _P, _P, _P],
+    'wq_w8a8_workspace_size': [_I64, _I64, _I64, _SIZE_P],
+    'wq_w8a8_linear_ws': [_P, _P, _I64, _I64, _P, ctypes.c_int32, _P, _I64, _P, _P, _P, ctypes.c_size_t, _P],
     'wq_w8_quantize': [_P, _I64, _I64, _P, _P, _P, _P],
     # include/ondeviceinfer_decode.h
     'wq_add_rmsnorm': [_P, _P, _P, _I64, _I64, ctypes.c_float, _P, _P, _P],
@@ -640,11 +642,18 @@ def w8a8_quantize(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return qx, scale
 
 
+@functools.lru_cache(maxsize=1024)   # a pure function of the shape, asked for on every call
+def w8a8_workspace_size(m: int, n: int, k: int) -> int:
+    b = ctypes.c_size_t()
+    _call('wq_w8a8_workspace_size', m, n, k, ctypes.byref(b))
+    return b.value
+
+
 def w8a8_linear(qx: torch.Tensor, x_scale: torch.Tensor, qweight, w_scale: torch.Tensor,
                 bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """``y = fp16(float(qx . qweight^T) * x_scale[m] * w_scale[n] (+ bias))``,
-    int32 accumulation on the int8 matrix cores; ``qweight`` row-major INT8
-    (``wq_w8a8_linear``) or ``W8Tiles`` (``wq_w8a8_linear_tiled``)."""
+    int32 accumulation on the int8 matrix cores; ``qweight`` row-major INT8 or
+    ``W8Tiles`` (``wq_w8a8_linear_ws``)."""
     n, kw, q, tiled = _w8_weight(qweight)
     device = _require_gpu(qx, x_scale, q, w_scale, bias, out)
     if qx.dtype != torch.int8 or qx.dim() != 2:
@@ -662,8 +671,11 @@ def w8a8_linear(qx: torch.Tensor, x_scale: torch.Tensor, qweight, w_scale: torch
         out = torch.empty((m, n), dtype=torch.float16, device=device)
     else:
         _check(out, torch.float16, (m, n), 'out')
-    _call('wq_w8a8_linear_tiled' if tiled else 'wq_w8a8_linear', _ptr(qx), _ptr(x_scale.contiguous()), m, k, _ptr(q), _ptr(w_scale.contiguous()), n,
-          _ptr(None if bias is None else bias.contiguous()), _ptr(out), _stream(device))
+    # The splits' partials (m <= 255): this call's own scratch.
+    nbytes = w8a8_workspace_size(m, n, k) if 4 < m < 256 else 0
+    workspace = qx.new_empty(nbytes, dtype=torch.uint8) if nbytes else None
+    _call('wq_w8a8_linear_ws', _ptr(qx), _ptr(x_scale.contiguous()), m, k, _ptr(q), tiled, _ptr(w_scale.contiguous()), n,
+          _ptr(None if bias is None else bias.contiguous()), _ptr(out), _ptr(workspace), nbytes, _stream(device))
     return out
 
 

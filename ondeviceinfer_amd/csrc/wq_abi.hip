@@ -18,6 +18,8 @@ void set_error(const char* fmt, ...) {
 }
 
 size_t gemv_workspace_bytes(bool w4, int64_t m, int64_t n, int64_t k);
+int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
+                  void* ws, size_t ws_bytes, hipStream_t st);
 size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
@@ -118,6 +120,12 @@ extern "C" int wq_w4a16_linear(const uint16_t* x, int64_t m, int64_t k, const vo
              WQ_ERR_INVALID_ARGUMENT, "x, tiles and y must be 16-byte aligned and meta 8-byte aligned");
   const half_t* xh = reinterpret_cast<const half_t*>(x);
   half_t* yh = reinterpret_cast<half_t*>(y);
+  if (m > 4 && m <= kSkinnyMaxM) {   // activations shared in LDS (wq_mid.hip), where it takes the shape
+    const int rc = launch_w4_mid(xh, (int)m, (int)k, reinterpret_cast<const uint4_t*>(tiles),
+                                 reinterpret_cast<const uint8_t*>(meta), (int)n, (int)group_size, yh, workspace,
+                                 workspace_bytes, as_stream(stream));
+    if (rc != -1) return rc;
+  }
   if (w4_gemm_small_fits(m, n) && k <= kGemmMaxK)
     return launch_w4_gemm_small(xh, (int)m, (int)k, reinterpret_cast<const uint4_t*>(tiles),
                                 reinterpret_cast<const uint8_t*>(meta), (int)n, (int)group_size, yh, as_stream(stream));

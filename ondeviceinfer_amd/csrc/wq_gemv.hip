@@ -921,8 +921,6 @@ int launch_w4_gemv_flat(const half_t* x, int M, int K, const uint4_t* tiles, con
 
 }  // namespace
 
-int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
-                  void* ws, size_t ws_bytes, hipStream_t st);
 int launch_w8_mid(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
                   half_t* y, void* ws, size_t ws_bytes, hipStream_t st, int tiled);
 
@@ -964,10 +962,6 @@ int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const 
                      half_t* y, void* ws, size_t ws_bytes, hipStream_t s) {
   if (M <= kGemvFlatMaxM) {
     int rc = launch_w4_gemv_flat(x, M, K, tiles, meta, N, G, y, ws, ws_bytes, s);
-    if (rc != kNotApplicable) return rc;
-  } else {
-    // Activations shared in LDS (wq_mid.hip).
-    int rc = launch_w4_mid(x, M, K, tiles, meta, N, G, y, ws, ws_bytes, s);
     if (rc != kNotApplicable) return rc;
   }
   const int mc = (M + 15) / 16;

@@ -5,40 +5,41 @@
 // skinny kernels give every wave its own copy of the activation fragments, so
 // at M = 49..64 a wave moves 16 KiB of x from L2 for every 2 KiB of W4
 // weights; here a workgroup moves M * 256 B of x per 128-k block once for its
-// eight 16-row tiles.  Workgroup (g, s) = 8 waves owns tile group g (128
-// rows of W) over the k range s of S:
+// 2 P 16-row tiles (P = 4 or 5).  Workgroup (g, s) = 2 P waves owns tile group
+// g over the k range s of S (both from mid_split):
 //  * wave (p, h) takes the tile pair p (two tiles, so that an x fragment read
-//    from LDS feeds two MFMAs; one tile per wave would make the LDS reads the
-//    bound) and the 128-k blocks of parity h, which halves the number of
-//    barriers per block; the two parities meet in LDS at the end;
+//    from LDS feeds two MFMAs) and the 128-k blocks of parity h, which halves
+//    the number of barriers per block; the two parities meet in LDS at the end;
 //  * a stage is two blocks: its x goes buffer -> LDS (rows past M read as
 //    zero, 16-byte chunk c of row r at slot c ^ (r & 15)), its weights straight
 //    into registers, D - 1 stages ahead (D = 3, and 2 where 48 or 64 rows fill
-//    the LDS and the registers: a deeper ring measured no faster there);
+//    the LDS and the registers: a deeper ring measured no faster there, nor
+//    did x staged through registers with the LDS reads one k-step ahead);
 //  * per block the skinny kernels' arithmetic: W4 the exact fp16 (q - z) on
 //    MFMA 16x16x32, then the group scale times the block sum added in fp32;
 //    INT8 the exact fp16 q, the row scale applied to the final sum.
-// Few tile groups leave compute units idle, so the k range is split until
-// about one workgroup per compute unit runs (mid_splits); each split stores
-// its fp32 partials with device-coherent stores and a second small launch
-// adds them in split order.  Against a last-arriver sum inside this kernel
-// (arrival counters, as the deep-ring GEMM) that is 0.3-0.8 us slower at some
-// W4 shapes and 0.4-4 us faster at N = 1024 and on INT8, and it needs no
-// zeroed counters, so any scratch of the call's own will do.  The short W4
-// shapes of 12 to 32 rows keep the last arriver (mid_counts): they finish
-// before the host has queued a second launch (fused QKV M = 24 called from
-// Python 11.5 us against 13.3).
-// MI355X, graphs of distinct weights, us, previous kernel -> this one:
-//   W4 17408->5120  M = 8 / 24 / 40 / 56   20.2 / 35.1 / 48.9 / 64.3 -> 15.0 / 17.3 / 20.8 / 24.0
-//   W4 5120->7168   M = 24 / 40 / 56       12.4 / 17.9 / 22.8 -> 11.7 / 14.0 / 16.0
-//   W4 5120->17408  M = 8 / 24 / 40 / 56   22.2 / 27.2 / 39.6 / 55.4 -> 17.6 / 20.6 / 22.9 / 30.2
-//   INT8 17408->5120  M = 8 / 24 / 56      31.5 / 36.5 / 65.6 -> 19.4 / 20.9 / 28.9
-//   INT8 5120->17408  M = 8 / 24 / 56      25.4 / 36.1 / 70.1 -> 20.7 / 25.9 / 31.7
-// i.e. 46 MB of W4 weights at M = 8 in 15.0 us (3.1 TB/s) and 89 MB of INT8
-// weights in 20.7 us (4.3 TB/s); what remains is about 6 us of launch, first
-// load and partial sum, then 0.75 us (M <= 16) to 1.3 us (M = 64, bound by
-// issue: 32 MFMAs, 120 VALU and 20 LDS operations per wave) a stage.
+// Each split stores its fp32 partials with device-coherent stores (0.1-0.8 us
+// ahead of plain and non-temporal ones) and a second small launch adds them
+// in split order.  Against a last-arriver sum inside this kernel (arrival
+// counters, as the deep-ring GEMM) that is 0.3-0.8 us slower at some W4 shapes
+// and 0.4-4 us faster at N = 1024 and on INT8, and it needs no zeroed counters,
+// so any scratch of the call's own will do.  The short W4 shapes of 12 to 32
+// rows keep the last arriver (mid_counts): they finish before the host has
+// queued a second launch (fused QKV M = 24 called from Python 11.5 us against
+// 13.3).
+// MI355X, graphs of distinct weights, us, previous kernels -> this one:
+//   W4 17408->5120    M = 8 / 24 / 40 / 56   20.5 / 35.8 / 49.7 / 65.1 -> 16.5 / 18.6 / 22.1 / 25.7
+//   W4 5120->7168     M = 24 / 40 / 56       13.0 / 18.1 / 23.2 -> 11.8 / 14.4 / 16.7
+//   W4 5120->17408    M = 8 / 24 / 40 / 56   22.5 / 27.5 / 40.0 / 56.2 -> 18.5 / 20.8 / 24.2 / 28.1
+//   W4 5120->34816    M = 8 / 24 / 40 / 56   27.9 / 35.9 / 49.3 / 50.6 -> 26.7 / 30.6 / 35.2 / 41.2
+//   INT8 17408->5120  M = 8 / 24 / 56        32.0 / 37.2 / 66.2 -> 20.4 / 21.7 / 30.6
+//   INT8 5120->17408  M = 8 / 24 / 56        25.5 / 36.4 / 71.3 -> 22.0 / 24.4 / 30.9
+//   INT8 5120->34816  M = 8 / 24 / 56        41.1 / 59.0 / 118 -> 33.4 / 35.8 / 47.1
+// i.e. 93 MB of W4 weights at M = 8 in 26.7 us (3.5 TB/s) and 178 MB of INT8
+// in 33.4 us (5.3 TB/s); what remains is about 6 us of launch, first load and
+// partial sum, then 16 B per cycle and compute unit of weights and x.
 #include "wq_common.h"
+#include "wq_mid_plan.h"
 #include "wq_status.h"
 
 namespace wq {
@@ -46,13 +47,9 @@ namespace {
 
 enum class MFmt { W4, W8 };
 
-constexpr int kMidWaves = 8;
-constexpr int kMidTilesPerWave = 2;
-constexpr int kMidGroupTiles = 4 * kMidTilesPerWave;   // tiles per workgroup
 // Largest k: 64 rows of x stay inside the 31-bit buffer range.
 constexpr int64_t kMidMaxK = 1 << 23;
-static_assert(1152 / kMidGroupTiles <= kSplitMaxCounters, "one counter per tile group");
-constexpr int kMidSumDepth = 8;                        // split partials requested at once by the final sum
+static_assert(1152 / (4 * kMidTilesPerWave) <= kSplitMaxCounters, "one counter per tile group");
 
 template <int N>
 __device__ __forceinline__ void mid_wait_vm() {
@@ -122,28 +119,28 @@ struct MidRegs<MFmt::W8> {
   uint4_t a[kMidTilesPerWave], b[kMidTilesPerWave];
 };
 
-template <MFmt F, int MC, int D, int MINW>
-__global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
+template <MFmt F, int P, int MC, int D, int MINW>
+__global__ __launch_bounds__(128 * P, MINW) void mid_kernel(
     const half_t* __restrict__ x, int M, int K, const void* __restrict__ wsrc, const void* __restrict__ wmeta, int N,
     int bpg, const half_t* __restrict__ bias, half_t* __restrict__ y, float4_t* ws_part, uint32_t* ws_cnt, int tiled) {
   constexpr int NT = kMidTilesPerWave;
   constexpr int kSubBytes = MC * 16 * 256;      // one 128-k block of x
   constexpr int kStageBytes = 2 * kSubBytes;
-  constexpr int kLoads = MC + (F == MFmt::W4 ? 3 : 2) * NT;   // per wave and stage
-  constexpr int kUnits = 4 * NT * MC;           // 1 KiB accumulator units of the workgroup
-  static_assert(D >= 2 && (D - 2) * kLoads <= 63, "ring depth");
+  constexpr int kWLoads = (F == MFmt::W4 ? 3 : 2) * NT;   // weight loads per wave and stage
+  constexpr int kUnits = P * NT * MC;           // 1 KiB accumulator units of the workgroup
+  static_assert(D >= 2 && (D - 2) * (MC + kWLoads) <= 63, "ring depth");
   static_assert(kUnits * 1024 <= D * kStageBytes, "the parity sum reuses the ring");
   __shared__ __attribute__((aligned(1024))) uint8_t xs[D * kStageBytes];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int p = wave & 3, h = wave >> 2;
+  const int h = wave >= P ? 1 : 0, p = wave - h * P;
   const int i = lane & 15, kb = lane >> 4;
   const int ntile = (N + 15) >> 4;
   const int nblk = K / kW4BlockK, nst = (nblk + 1) >> 1;
   const int group = blockIdx.x, split = blockIdx.y, S = gridDim.y;
   const int st_lo = (split * nst) / S, nloc = ((split + 1) * nst) / S - st_lo;
-  const int tile0 = (group * 4 + p) * NT;
+  const int tile0 = (group * P + p) * NT;
   constexpr uint32_t kPastEnd = 0x80000000u;
 
   uint32_t xvo[MC];
@@ -179,9 +176,11 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
   auto fetch = [&](int st, MidRegs<F>& r) {
     const bool live = nx < nx_end;
     const uint32_t xo = live ? (uint32_t)nx * 256 : kPastEnd;
+    if (P == 4 || p < 4) {   // four of the P waves of a parity copy its x
 #pragma unroll
-    for (int j = 0; j < MC; ++j)
-      lds_load16(rx, xvo[j], xo, xs + st * kStageBytes + h * kSubBytes + (p * MC + j) * 1024);
+      for (int j = 0; j < MC; ++j)
+        lds_load16(rx, xvo[j], xo, xs + st * kStageBytes + h * kSubBytes + (p * MC + j) * 1024);
+    }
     const uint32_t wo = live ? (uint32_t)nx * wstep : kPastEnd;
     if constexpr (F == MFmt::W4) {
       const uint32_t mo = live ? (uint32_t)(gq * kW4MetaBytes) : kPastEnd;
@@ -269,8 +268,12 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
     fetch(j, wr[j]);
     __builtin_amdgcn_sched_barrier(0);   // loads stay in stage order: the waits below count them
   }
-  mid_wait_vm<(D - 2) * kLoads>();
-  __builtin_amdgcn_s_barrier();
+  auto wait = [&]() {   // the next stage has landed: this wave's part, then everyone's
+    if (P == 4 || p < 4) mid_wait_vm<(D - 2) * (MC + kWLoads)>();
+    else mid_wait_vm<(D - 2) * kWLoads>();
+    __builtin_amdgcn_s_barrier();
+  };
+  wait();
   int base = 0;
   do {
 #pragma unroll
@@ -278,8 +281,7 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
       fetch((u + D - 1) % D, wr[(u + D - 1) % D]);
       __builtin_amdgcn_sched_barrier(0);
       if (base + u < nloc) block(u, wr[u]);
-      mid_wait_vm<(D - 2) * kLoads>();
-      __builtin_amdgcn_s_barrier();
+      wait();
     }
     base += D;
   } while (base < nloc);
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
       for (int mc = 0; mc < MC; ++mc) {
         const int unit = (p * NT + t) * MC + mc;
         const float4_t s = acc[t][mc] + red[unit * 64 + lane];
-        if (S == 1) mid_store<F>(s, mc * 16 + i, (group * kMidGroupTiles + p * NT + t) * 16 + 4 * kb, M, N, wmeta, bias, y);
+        if (S == 1) mid_store<F>(s, mc * 16 + i, (tile0 + t) * 16 + 4 * kb, M, N, wmeta, bias, y);
         else coherent_store16(ws_part, (uint32_t)(((group * S + split) * kUnits + unit) * 1024 + lane * 16),
                               __builtin_bit_cast(uint4_t, s));
       }
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
     __syncthreads();
     if (*arrival != (uint32_t)(S - 1)) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    static_assert(kUnits == MC * kMidWaves, "MC units per wave");
+    static_assert(kUnits == MC * 2 * P, "MC units per wave");
     constexpr int Q = 8 / MC;        // splits of each unit requested at once
     float4_t sum[MC];
     for (int s0 = 0; s0 < S; s0 += Q) {
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
         for (int u = 0; u < MC; ++u)
           v[u][q] = __builtin_bit_cast(
               float4_t, coherent_load16(ws_part, (uint32_t)(((group * S + min(s0 + q, S - 1)) * kUnits + wave +
-                                                             u * kMidWaves) * 1024 + lane * 16)));
+                                                             u * 2 * P) * 1024 + lane * 16)));
 #pragma unroll
       for (int q = 0; q < Q; ++q)
         if (s0 + q < S)
@@ -340,8 +342,8 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
     }
 #pragma unroll
     for (int u = 0; u < MC; ++u) {
-      const int unit = wave + u * kMidWaves;
-      mid_store<F>(sum[u], (unit % MC) * 16 + i, (group * kMidGroupTiles + unit / MC) * 16 + 4 * kb, M, N, wmeta, bias, y);
+      const int unit = wave + u * 2 * P;
+      mid_store<F>(sum[u], (unit % MC) * 16 + i, (group * P * NT + unit / MC) * 16 + 4 * kb, M, N, wmeta, bias, y);
     }
     if (threadIdx.x == 0) __hip_atomic_store(&ws_cnt[group], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -349,16 +351,17 @@ __global__ __launch_bounds__(64 * kMidWaves, MINW) void mid_kernel(
 
 // The S partials of every unit, in split order.  One wave per unit, all of a
 // lane's loads (up to six) in flight at once.
-template <MFmt F, int MC>
-__global__ __launch_bounds__(256) void mid_sum_kernel(const float4_t* __restrict__ part, int S, int M, int N,
+template <MFmt F, int P, int MC>
+__global__ __launch_bounds__(256) void mid_sum_kernel(const float4_t* __restrict__ part, int S, int groups, int M, int N,
                                                       const void* __restrict__ wmeta, const half_t* __restrict__ bias,
                                                       half_t* __restrict__ y) {
-  constexpr int kUnits = kMidGroupTiles * MC;
+  constexpr int kUnits = P * kMidTilesPerWave * MC;
   constexpr int Q = 5;   // partials after the first requested at once
   const int lane = threadIdx.x & 63, i = lane & 15, kb = lane >> 4;
   const int gu = blockIdx.x * 4 + (threadIdx.x >> 6);   // group * kUnits + unit
+  if (gu >= groups * kUnits) return;   // the last workgroup's spare waves
   const int group = gu / kUnits, unit = gu % kUnits;
-  const int m = (unit % MC) * 16 + i, n0 = (group * kMidGroupTiles + unit / MC) * 16 + 4 * kb;
+  const int m = (unit % MC) * 16 + i, n0 = (group * P * kMidTilesPerWave + unit / MC) * 16 + 4 * kb;
   if (m >= M || n0 >= N) return;
   const float4_t* q = part + ((size_t)group * S * kUnits + unit) * 64 + lane;
   float4_t s = q[0];
@@ -373,38 +376,30 @@ __global__ __launch_bounds__(256) void mid_sum_kernel(const float4_t* __restrict
   mid_store<F>(s, m, n0, M, N, wmeta, bias, y);
 }
 
-// Splits of the k range (two-block stages) over workgroups: one workgroup per
-// compute unit (256) for up to 128 tile groups, at most 2/5 of a split per
-// stage (shorter ranges are all start-up: N = 1024, K = 5120 8 splits of 2.5
-// stages).  Beyond 128 groups the grid covers more than half of the machine by
-// itself and the splits only even out its rounds: three up to 170 groups (408
-// workgroups on the gate / up shape), two above.  INT8 at M <= 32 keeps the
-// whole range up to 170 groups: its 96 KiB of weights in flight per workgroup
-// saturate memory from 136 compute units (5120->17408 M = 8 20.7 us against
-// 23.2 with three splits), which W4's half does not (18.4 against 17.4).
-int mid_splits(bool w4, int64_t M, int64_t N, int64_t K) {
+// Tile groups and k splits (two-block stages) of a shape.
+MidSplit mid_plan(bool w4, int64_t M, int64_t N, int64_t K) {
   const int mc = (int)((M + 15) / 16);
-  const int64_t groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles, nst = (K / kW4BlockK + 1) / 2;
-  int64_t s = groups <= 128 ? 256 / groups : groups > 170 ? 2 : !w4 && mc <= 2 ? 1 : 3;
-  if (s > nst * 2 / 5) s = nst * 2 / 5;
-  if (s > 16) s = 16;
-  while (s > 1 && kSplitCounterBytes + (size_t)(groups * s) * kMidGroupTiles * mc * 1024 > kSplitWorkspaceMaxBytes) --s;
-  return s < 1 ? 1 : (int)s;
+  return mid_split((N + 15) / 16, (K / kW4BlockK + 1) / 2, w4 ? 2 * (1024 + kW4MetaBytes) : 2 * kW8TileBlockBytes,
+                   2 * mc * 16 * 256, 1, mc);
 }
 
 // The shapes this file takes, from both sides' measurements.  W4: from 12
-// rows on, below 2048 tiles (there the deep-ring GEMM stays ahead: fused
-// gate_up M = 24 / 56 36 / 50 us against 38 / 59), and from 5 rows where the
-// k chain is long or N is wide (17408->5120 M = 8 20.2 -> 15.0 us, 5120->17408
-// 22.2 -> 17.6; fused QKV M = 8 8.2 against 10.2 the other way).  At 33 to 35
+// rows on, and from 5 rows where the k chain is long or N is wide (17408->5120
+// M = 8 20.5 -> 16.5 us, 5120->17408 22.5 -> 18.5; fused QKV M = 8 8.2 against
+// 10.2 the other way); from 2048 tiles on only chains of at least 32 blocks
+// (shorter ones keep the skinny kernels and, above 16 rows, the deep-ring
+// GEMM, whose rows equal those of longer batches bit for bit).  At 33 to 35
 // rows short chains stay on the skinny kernels: their workspace query answers
-// 0 bytes just past 32 rows, which callers may rely on.  INT8: everything but
-// narrow N at M <= 16 (N = 1024 M = 8 6.6 us against 8.6).
+// 0 bytes just past 32 rows, which callers may rely on.  INT8: from 33 rows on,
+// and weights of at least 10000 tile blocks (20 MB; 5120->1024 M = 8 6.6 us
+// against 8.6, 2048->4040 5.2 against 8.2 the other way) or, from 17 rows,
+// chains of at least 32 blocks (5120->1024 M = 24 12.9 -> 9.3 us, 2048->4040
+// 8.2 against 9.1).
 bool mid_takes(bool w4, int64_t M, int64_t N, int64_t K) {
   if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return false;
   const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
-  if (!w4) return M > 16 || ntile >= 128;
-  if (ntile >= 2048) return false;
+  if (!w4) return M > 32 || ntile * nblk >= 10000 || (M > 16 && nblk >= 32);
+  if (ntile >= 2048) return nblk >= 32;
   if (M < 12) return nblk >= 64 || ntile >= 1024;
   return nblk >= 64 || M < 33 || M > 35;
 }
@@ -419,26 +414,32 @@ bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
 
 size_t mid_ws_bytes(bool w4, int64_t M, int64_t N, int64_t K) {
   if (!mid_takes(w4, M, N, K)) return 0;
-  const int s = mid_splits(w4, M, N, K);
-  if (s <= 1) return 0;
-  const int64_t groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles;
-  return kSplitCounterBytes + (size_t)(groups * s) * kMidGroupTiles * ((M + 15) / 16) * 1024;
+  return mid_partial_bytes(mid_plan(w4, M, N, K), 1, (int)((M + 15) / 16));
 }
 
-template <MFmt F, int MC, int D, int MINW>
+template <MFmt F, int P, int MC, int D, int MINW>
 int launch_mid(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* bias,
-               half_t* y, void* ws, int S, int tiled, hipStream_t st) {
-  const int groups = ((N + 15) / 16 + kMidGroupTiles - 1) / kMidGroupTiles;
-  // The partials start past the counter region that other split kernels keep
-  // at zero in a shared workspace.
-  float4_t* part = S > 1 ? reinterpret_cast<float4_t*>(reinterpret_cast<uint8_t*>(ws) + kSplitCounterBytes) : nullptr;
-  uint32_t* cnt = S > 1 && mid_counts(F == MFmt::W4, M, N, K) ? reinterpret_cast<uint32_t*>(ws) : nullptr;
-  hipLaunchKernelGGL((mid_kernel<F, MC, D, MINW>), dim3((unsigned)groups, (unsigned)S), dim3(64 * kMidWaves), 0, st, x,
+               half_t* y, void* ws, const MidSplit& m, int tiled, hipStream_t st) {
+  float4_t* part = m.s > 1 ? reinterpret_cast<float4_t*>(reinterpret_cast<uint8_t*>(ws) + kSplitCounterBytes) : nullptr;
+  uint32_t* cnt = m.s > 1 && mid_counts(F == MFmt::W4, M, N, K) ? reinterpret_cast<uint32_t*>(ws) : nullptr;
+  hipLaunchKernelGGL((mid_kernel<F, P, MC, D, MINW>), dim3((unsigned)m.groups, (unsigned)m.s), dim3(128 * P), 0, st, x,
                      M, K, w, meta, N, bpg, bias, y, part, cnt, tiled);
-  if (S > 1 && cnt == nullptr)
-    hipLaunchKernelGGL((mid_sum_kernel<F, MC>), dim3((unsigned)(groups * kMidGroupTiles * MC / 4)), dim3(256), 0, st,
-                       part, S, M, N, meta, bias, y);
+  if (m.s > 1 && cnt == nullptr)
+    hipLaunchKernelGGL((mid_sum_kernel<F, P, MC>), dim3((unsigned)((m.groups * P * kMidTilesPerWave * MC + 3) / 4)),
+                       dim3(256), 0, st, part, m.s, (int)m.groups, M, N, meta, bias, y);
   return check_launch(F == MFmt::W4 ? "w4_mid" : "w8_mid");
+}
+
+template <MFmt F, int P>
+int launch_mid_p(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* bias,
+                 half_t* y, void* ws, const MidSplit& m, int tiled, hipStream_t st) {
+  constexpr int kMin = P == 4 ? 4 : 3;   // waves per SIMD: two workgroups of eight waves, or one of ten
+  switch ((M + 15) / 16) {
+    case 1: return launch_mid<F, P, 1, 3, kMin>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
+    case 2: return launch_mid<F, P, 2, 3, kMin>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
+    case 3: return launch_mid<F, P, 3, F == MFmt::W4 ? 2 : 3, kMin>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
+    default: return launch_mid<F, P, 4, 2, P == 4 ? 2 : 3>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
+  }
 }
 
 // Returns -1 (not taken) when the shape is not this file's or its splits need
@@ -450,13 +451,9 @@ int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* me
   if (!mid_takes(w4, M, N, K)) return -1;
   const size_t need = mid_ws_bytes(w4, M, N, K);
   if (need > 0 && (ws == nullptr || ws_bytes < need)) return -1;
-  const int S = mid_splits(w4, M, N, K);
-  switch ((M + 15) / 16) {
-    case 1: return launch_mid<F, 1, 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
-    case 2: return launch_mid<F, 2, 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
-    case 3: return launch_mid<F, 3, w4 ? 2 : 3, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
-    default: return launch_mid<F, 4, 2, 2>(x, M, K, w, meta, N, bpg, bias, y, ws, S, tiled, st);
-  }
+  const MidSplit m = mid_plan(w4, M, N, K);
+  return m.p == 4 ? launch_mid_p<F, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st)
+                  : launch_mid_p<F, 5>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
 }
 
 }  // namespace

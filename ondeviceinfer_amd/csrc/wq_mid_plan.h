@@ -1,0 +1,80 @@
+// Work split of the shared-activation kernels (wq_mid.hip: 5 to 64 rows;
+// wq_w8a8.hip: up to 255 rows), host only.
+#pragma once
+
+#include "wq_common.h"
+
+namespace wq {
+
+constexpr int kMidTilesPerWave = 2;   // 16-row tiles per wave
+
+// Tile groups of 2 P tiles (P wave pairs per workgroup), S k splits.
+struct MidSplit {
+  int p, s;
+  int64_t groups;
+};
+
+inline int64_t mid_groups(int64_t ntile, int p) {
+  return (ntile + p * kMidTilesPerWave - 1) / (p * kMidTilesPerWave);
+}
+
+// Split partials: one 1 KiB unit per tile, 16-row chunk and split, behind the
+// counter region (which other split kernels keep at zero in a shared
+// workspace).
+inline size_t mid_partial_bytes(const MidSplit& m, int64_t nz, int mc) {
+  return m.s <= 1 ? 0 : kSplitCounterBytes + (size_t)(m.groups * nz * m.s) * m.p * kMidTilesPerWave * mc * 1024;
+}
+
+// The (P, S) of least estimated time.  Timing-only copies of the kernels
+// showed what bounds them: leaving out the MFMAs or the LDS reads changes
+// nothing, leaving out the x copies their share of the bytes, so a compute
+// unit takes in about 35 KB/us whatever it holds (16 B per cycle; one
+// workgroup of 72 or 128 KiB in flight or two alike), and all of them
+// together what memory gives, about 5.5 MB/us.  Hence
+//   rounds of workgroups over 256 compute units x bytes per workgroup / 35 KB
+//   (at least the whole weight / 5.5 MB; a tenth of it on top, so that of two
+//   splits at that bound the finer one wins)
+//   + the partial sums: their launch 1.5 us, a second round of loads beyond
+//   six splits 1 us, their bytes out and back at 4 MB/us.
+// P = 4 or 5: eight or ten tiles a workgroup.  Ten is for grids of more than
+// 128 groups of eight, whose rounds it can even out: 5120->34816 (2176 tiles)
+// takes 218 workgroups in one round instead of 272 in two (W8A8 M = 48 48.3 ->
+// 34.9 us, INT8 M = 40 54 -> 41.8, W4 M = 40 43 -> 35.7), 5120->17408 in two
+// splits the same (W8A8 M = 48 27.6 -> 24.7 us).  On narrow N ten waves lost to
+// eight at the same bytes (W4 17408->5120 M = 8, seven splits: 18.2 us against
+// 15.0 with eight waves in six).
+// Beyond 64 rows ten waves' registers would spill.
+// w_tile / x_stage: bytes of one tile's weights and of the workgroup's x in one
+// stage; nst stages; nz row blocks; mc 16-row chunks.
+inline MidSplit mid_split(int64_t ntile, int64_t nst, double w_tile, double x_stage, int64_t nz, int mc) {
+  MidSplit best{4, 1, mid_groups(ntile, 4)};
+  double best_us = 1e30;
+  const int most = mc <= 4 && mid_groups(ntile, 4) * nz > 128 ? 5 : 4;
+  for (int p = 4; p <= most; ++p) {
+    MidSplit m{p, 1, mid_groups(ntile, p)};
+    for (m.s = 1; m.s <= 16 && m.s * 5 <= nst * 3; ++m.s) {
+      if (mid_partial_bytes(m, nz, mc) > kSplitWorkspaceMaxBytes) break;
+      const double rounds = (double)((m.groups * nz * m.s + 255) / 256);
+      const double stages = (double)((nst + m.s - 1) / m.s);
+      const double fill = rounds * stages * (p * kMidTilesPerWave * w_tile + x_stage) / 35e3;
+      const double stream = (double)ntile * (double)nst * w_tile / 5.5e6;
+      double us = (fill > stream ? fill : stream) + 0.1 * fill;
+      if (m.s > 1) us += (m.s > 6 ? 2.5 : 1.5) + 2.0 * (double)mid_partial_bytes(m, nz, mc) / 4e6;
+      if (us < best_us) {
+        best_us = us;
+        best = m;
+      }
+    }
+    if (nst * 3 < 5) {   // a single stage: the loop above has no S to try
+      m.s = 1;
+      const double us = (double)((m.groups * nz + 255) / 256) * (p * kMidTilesPerWave * w_tile + x_stage);
+      if (p == 4 || us < best_us) {
+        best_us = us;
+        best = m;
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace wq

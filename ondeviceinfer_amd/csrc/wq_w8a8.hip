@@ -10,6 +10,7 @@
 // the A operand (rows n), activations the B operand (columns m).
 #include "ondeviceinfer_wq.h"
 #include "wq_common.h"
+#include "wq_mid_plan.h"
 #include "wq_status.h"
 
 #include <math.h>
@@ -32,36 +33,83 @@ __device__ __forceinline__ float wave_max_abs(float v) {
   return v;
 }
 
-// One workgroup per row of x [M, K] (K % 8 == 0): absmax in fp32,
-// scale = max(absmax, 1e-12) / 127, q = clamp(rint(x / scale), -127, 127)
-// with an IEEE divide and round-half-even, as the reference's W8A8 oracle
-// (backend.py:258-261).
-__global__ __launch_bounds__(256) void w8a8_quantize_kernel(const half_t* __restrict__ x, int K,
-                                                            int8_t* __restrict__ q, float* __restrict__ scale) {
-  __shared__ float part[4];
+// clamp(rint(v / s), -127, 127) of eight values, packed; rs = RN(1 / s).  The
+// quotient of one row's values by one s: Markstein's correction of v * rs
+// (IBM J. Res. Dev. 34, 1990), a remainder by fma and a corrected quotient,
+// applied twice, which rounds like the IEEE divide (the first leaves a
+// faithful quotient, the second the nearest) in five operations a value
+// instead of the divide's dozen.  v and s are normal or v is zero, |v| <= 127 s,
+// so no step over- or underflows.  MARKSTEIN = false is the plain divide.
+template <bool MARKSTEIN>
+__device__ __forceinline__ uint2_t w8a8_codes8(half8_t v, float s, float rs) {
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float a = (float)v[e];
+    float d;
+    if constexpr (MARKSTEIN) {
+      d = a * rs;
+      d = __builtin_fmaf(__builtin_fmaf(-d, s, a), rs, d);
+      d = __builtin_fmaf(__builtin_fmaf(-d, s, a), rs, d);
+    } else {
+      d = a / s;
+    }
+    const float r = fminf(fmaxf(rintf(d), -127.0f), 127.0f);
+    w[e >> 2] |= (uint32_t)(uint8_t)(int8_t)(int)r << (8 * (e & 3));
+  }
+  return uint2_t{w[0], w[1]};
+}
+
+// One workgroup of T threads per row of x [M, K] (K % 8 == 0): absmax in
+// fp32, scale = max(absmax, 1e-12) / 127, q = clamp(rint(x / scale), -127, 127)
+// with the IEEE quotient and round-half-even, as the reference's W8A8 oracle
+// (backend.py:258-261).  With C > 0 the row (at most C chunks of 8 per thread)
+// stays in registers between the two steps; C == 0 reads it again (longer
+// rows).  Bound: at 2048 rows of 5120 by issue (the divide), at few rows by
+// the chain load -> reduce -> store, hence 1024 threads per row there.
+template <int T, int C>
+__global__ __launch_bounds__(T) void w8a8_quantize_kernel(const half_t* __restrict__ x, int K, int8_t* __restrict__ q,
+                                                          float* __restrict__ scale) {
+  __shared__ float part[T / 64];
   const size_t base = (size_t)blockIdx.x * K;
   const int nc = K >> 3;
+  half8_t v[C > 0 ? C : 1];
   float mx = 0.f;
-  for (int c = threadIdx.x; c < nc; c += 256) {
-    const half8_t v = ld_h8(x + base + 8 * c);
+  auto absmax = [&](half8_t h) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf((float)v[e]));
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf((float)h[e]));
+  };
+  if constexpr (C > 0) {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int c = threadIdx.x + j * T;
+      v[j] = c < nc ? ld_h8(x + base + 8 * c) : half8_t{};
+    }
+#pragma unroll
+    for (int j = 0; j < C; ++j) absmax(v[j]);
+  } else {
+    for (int c = threadIdx.x; c < nc; c += T) absmax(ld_h8(x + base + 8 * c));
   }
   mx = wave_max_abs(mx);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) mx = fmaxf(mx, part[w]);
   const float s = fmaxf(mx, 1e-12f) / 127.0f;
   if (threadIdx.x == 0) scale[blockIdx.x] = s;
-  for (int c = threadIdx.x; c < nc; c += 256) {
-    const half8_t v = ld_h8(x + base + 8 * c);
-    uint32_t w[2] = {0u, 0u};
+  const float rs = 1.0f / s;
+  const bool finite = s < __builtin_inff();   // an infinite row: the plain divide's 0 and NaN
+  auto put = [&](int c, half8_t h) {
+    *reinterpret_cast<uint2_t*>(q + base + 8 * c) = finite ? w8a8_codes8<true>(h, s, rs) : w8a8_codes8<false>(h, s, rs);
+  };
+  if constexpr (C > 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float r = fminf(fmaxf(rintf((float)v[e] / s), -127.0f), 127.0f);
-      w[e >> 2] |= (uint32_t)(uint8_t)(int8_t)(int)r << (8 * (e & 3));
+    for (int j = 0; j < C; ++j) {
+      const int c = threadIdx.x + j * T;
+      if (c < nc) put(c, v[j]);
     }
-    *reinterpret_cast<uint2_t*>(q + base + 8 * c) = uint2_t{w[0], w[1]};
+  } else {
+    for (int c = threadIdx.x; c < nc; c += T) put(c, ld_h8(x + base + 8 * c));
   }
 }
 
@@ -351,6 +399,298 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(const int8_t* __restr
   }
 }
 
+// Batches of 5 to 255 rows: the activation tile of a workgroup shared in LDS
+// and the k range split over workgroups, as the fp16 kernel of 5 to 64 rows
+// (wq_mid.hip), on the int8 matrix cores.
+//
+// Bound: the weight stream, at the rate a compute unit takes bytes in
+// (wq_mid_plan.h).  The GEMM below takes 32-row tiles at these M, so it reads
+// the weights once per 32 rows with one 128-k block in flight; here a workgroup
+// covers up to 128 rows (MC chunks of 16) of its 2 P 16-row weight tiles.  Its
+// 2 P waves (p, h) take the tile pair p and two of the four 128-k blocks of a
+// stage (h), weights straight into registers and x buffer -> LDS D - 1 stages
+// ahead; the two halves meet in LDS, S > 1 k ranges through int32 partials that
+// a second launch adds and scales.  The sums are exact integers, so every plan
+// gives the same bits.
+// MI355X, graphs of distinct weights, us with the quantizer, before -> now:
+//   17408->5120  M = 8 / 24 / 56 / 96 / 200   37.4 / 62.2 / 62.8 / 62.9 / 71.8 -> 24.4 / 25.8 / 29.9 / 34.1 / 48.3
+//   5120->17408  M = 8 / 24 / 56              27.2 / 32.2 / 37.6 -> 24.7 / 26.2 / 30.7
+//   5120->34816  M = 8 / 24 / 56              45.4 / 44.5 / 67.5 -> 36.4 / 38.1 / 43.6
+//   5120->5120   M = 16 / 56 / 96             17.1 / 23.9 / 24.1 -> 14.7 / 19.4 / 20.9
+// i.e. 178 MB of weights at M = 8 in 32 us without the quantizer (5.6 TB/s).
+constexpr int kM8Tiles = kMidTilesPerWave;
+constexpr int kM8MaxM = 255;   // from 256 rows the GEMM takes 128-row tiles
+
+// The MC fragments of one k-step (16 rows apart in a stage), read and waited
+// for in one asm block (see i8_lds_read_off for why asm).
+template <int MC>
+__device__ __forceinline__ void m8_read(uint4_t (&f)[MC], uint32_t a) {
+  if constexpr (MC == 1)
+    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(f[0]) : "v"(a));
+  else if constexpr (MC == 2)
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]) : "v"(a));
+  else if constexpr (MC == 3)
+    asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:2048\n\tds_read_b128 %2, %3 offset:4096\n\t"
+                 "s_waitcnt lgkmcnt(0)" : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]) : "v"(a));
+  else if constexpr (MC == 4)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\tds_read_b128 %2, %4 offset:4096\n\t"
+                 "ds_read_b128 %3, %4 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]) : "v"(a));
+  else if constexpr (MC == 6)
+    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:2048\n\tds_read_b128 %2, %6 offset:4096\n\t"
+                 "ds_read_b128 %3, %6 offset:6144\n\tds_read_b128 %4, %6 offset:8192\n\tds_read_b128 %5, %6 offset:10240\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]) : "v"(a));
+  else
+    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:2048\n\tds_read_b128 %2, %8 offset:4096\n\t"
+                 "ds_read_b128 %3, %8 offset:6144\n\tds_read_b128 %4, %8 offset:8192\n\tds_read_b128 %5, %8 offset:10240\n\t"
+                 "ds_read_b128 %6, %8 offset:12288\n\tds_read_b128 %7, %8 offset:14336\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]), "=&v"(f[6]), "=&v"(f[7])
+                 : "v"(a));
+}
+
+// As w8a8_store, the four columns n0 .. n0 + 3 at once where row m keeps
+// 8-byte alignment.
+__device__ __forceinline__ void m8_store(int4v_t s, int m, int n0, int M, int N, const float* __restrict__ sx,
+                                         const float* __restrict__ sw, const half_t* __restrict__ bias,
+                                         half_t* __restrict__ y) {
+#pragma clang fp contract(off)
+  if (m >= M || n0 >= N) return;
+  half4_t o;
+  const float xs = sx[m];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int n = min(n0 + v, N - 1);
+    float r = (float)s[v] * xs * sw[n];
+    if (bias) r += (float)bias[n];
+    o[v] = (half_t)r;
+  }
+  if ((N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+    *reinterpret_cast<half4_t*>(y + (size_t)m * N + n0) = o;
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (n0 + v < N) y[(size_t)m * N + n0 + v] = o[v];
+  }
+}
+
+template <int P, int MC, int D>
+__global__ __launch_bounds__(128 * P, P == 4 ? 2 : 3) void w8a8_mid_kernel(
+    const int8_t* __restrict__ qx, const float* __restrict__ sx, int M, int K, const int8_t* __restrict__ qw,
+    const float* __restrict__ sw, const half_t* __restrict__ bias, int N, half_t* __restrict__ y, int4v_t* ws_part,
+    W8Layout wl8) {
+  constexpr int NT = kM8Tiles;
+  constexpr int kSubBytes = MC * 16 * kI8RowBytes;   // x of one 128-k block
+  constexpr int kStageBytes = 4 * kSubBytes;
+  constexpr int kUnits = P * NT * MC;
+  static_assert(kUnits * 1024 <= D * kStageBytes && (D - 2) * (MC + 4 * NT) <= 63, "ring");
+  __shared__ __attribute__((aligned(1024))) uint8_t xs[D * kStageBytes];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = wave >= P ? 1 : 0, p = wave - h * P;
+  const int i = lane & 15, kb = lane >> 4;
+  const int ntile = (N + 15) >> 4, nblk = K / kI8Blk, nst = (nblk + 3) >> 2;
+  const int group = blockIdx.x, split = blockIdx.y, S = gridDim.y;
+  const int st_lo = (split * nst) / S, nloc = ((split + 1) * nst) / S - st_lo;
+  const int tile0 = (group * P + p) * NT;
+  const int m0 = blockIdx.z * (MC * 16);
+  constexpr uint32_t kPastEnd = 0x80000000u;
+
+  // A stage is four 128-k blocks, 2h and 2h + 1 this wave's.  x instruction
+  // J = p MC + j of the parity's 4 MC: block J / (2 MC), rows 8 (J % (2 MC)) ..
+  uint32_t xvo[MC];
+#pragma unroll
+  for (int j = 0; j < MC; ++j) {
+    const int J = p * MC + j, sub = J / (2 * MC), rr = 8 * (J % (2 * MC)) + (lane >> 3);
+    xvo[j] = (uint32_t)(rr * K + 16 * i8_swz(rr, lane & 7) + sub * kI8Blk);
+  }
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(qx + (size_t)m0 * K, (int64_t)(M - m0) * K);
+  const __amdgpu_buffer_rsrc_t rw =
+      wl8.tiled ? buf_rsrc(qw + (size_t)tile0 * nblk * kW8TileBlockBytes, (int64_t)(ntile - tile0) * nblk * kW8TileBlockBytes)
+                : buf_rsrc(qw + (size_t)tile0 * 16 * K, (int64_t)(N - tile0 * 16) * K);
+  const uint32_t wvo = wl8.tiled ? (uint32_t)lane * 16 : (uint32_t)(i * K + 16 * kb);
+  const uint32_t wstep = (uint32_t)wl8.block_bytes(), p1 = (uint32_t)wl8.piece1();
+  const uint32_t wtile = wl8.tiled ? (uint32_t)nblk * kW8TileBlockBytes : (uint32_t)(16 * K);
+  int nx = 4 * st_lo + 2 * h;
+  const int nx_end = min(4 * (st_lo + nloc), nblk);
+  struct Regs { uint4_t w[2][NT][2]; };
+  auto fetch = [&](int st, Regs& r) {
+    // x of a block past the range: the second block of an odd tail reads the
+    // next row's bytes (or past the buffer) and meets zero weights.
+    const uint32_t xo = nx < nx_end ? (uint32_t)nx * kI8Blk : kPastEnd;
+    if (P == 4 || p < 4) {   // four of the P waves of a half copy its x
+#pragma unroll
+      for (int j = 0; j < MC; ++j)
+        lds_load16(rx, xvo[j], xo, xs + st * kStageBytes + h * 2 * kSubBytes + (p * MC + j) * 1024);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint32_t wo = nx + b < nx_end ? (uint32_t)(nx + b) * wstep : kPastEnd;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        r.w[b][t][0] = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo, wo + t * wtile, kNtPolicy);
+        r.w[b][t][1] = __builtin_amdgcn_raw_buffer_load_b128(rw, wvo + p1, wo + t * wtile, kNtPolicy);
+      }
+    }
+    nx += 4;
+  };
+  int4v_t acc[NT][MC];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mc = 0; mc < MC; ++mc) acc[t][mc] = int4v_t{0, 0, 0, 0};
+  const uint32_t xs_base = (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)xs) +
+                           (uint32_t)(h * 2 * kSubBytes + i * kI8RowBytes);
+  auto stage_math = [&](int st, const Regs& r) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int step = 0; step < 2; ++step) {
+        uint4_t f[MC];
+        m8_read<MC>(f, xs_base + (uint32_t)(st * kStageBytes + b * kSubBytes + i8_swz(i, 4 * step + kb) * 16));
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int mc = 0; mc < MC; ++mc) acc[t][mc] = mfma_i8(r.w[b][t][step], f[mc], acc[t][mc]);
+      }
+  };
+  Regs wr[D];
+#pragma unroll
+  for (int j = 0; j < D - 1; ++j) {
+    fetch(j, wr[j]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto wait = [&]() {
+    constexpr int W = (D - 2) * (MC + 4 * NT), W2 = (D - 2) * 4 * NT;
+    if (P == 4 || p < 4) __builtin_amdgcn_s_waitcnt((W & 0xF) | ((W >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+    else __builtin_amdgcn_s_waitcnt((W2 & 0xF) | ((W2 >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+    __builtin_amdgcn_s_barrier();
+  };
+  wait();   // stage 0 landed (this wave's part, then everyone's)
+  int base = 0;
+  do {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      fetch((u + D - 1) % D, wr[(u + D - 1) % D]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (base + u < nloc) stage_math(u, wr[u]);
+      wait();
+    }
+    base += D;
+  } while (base < nloc);
+  __builtin_amdgcn_s_waitcnt(0);   // the run-out's empty copies
+  __builtin_amdgcn_s_barrier();    // ... everyone's: the ring is dead
+  int4v_t* red = reinterpret_cast<int4v_t*>(xs);
+  if (h == 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int mc = 0; mc < MC; ++mc) red[((p * NT + t) * MC + mc) * 64 + lane] = acc[t][mc];
+  }
+  __syncthreads();
+  if (h == 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int mc = 0; mc < MC; ++mc) {
+        const int unit = (p * NT + t) * MC + mc;
+        const int4v_t s = acc[t][mc] + red[unit * 64 + lane];
+        if (S == 1) m8_store(s, m0 + mc * 16 + i, (tile0 + t) * 16 + 4 * kb, M, N, sx, sw, bias, y);
+        else coherent_store16(ws_part, (uint32_t)((((blockIdx.z * gridDim.x + group) * S + split) * kUnits + unit) * 1024 + lane * 16),
+                              __builtin_bit_cast(uint4_t, s));
+      }
+  }
+}
+
+// The S partials of every unit, one wave per unit, then the scaling.
+template <int P, int MC>
+__global__ __launch_bounds__(256) void w8a8_mid_sum_kernel(const int4v_t* __restrict__ part, int S, int groups, int nz, int M, int N,
+                                                           const float* __restrict__ sx, const float* __restrict__ sw,
+                                                           const half_t* __restrict__ bias, half_t* __restrict__ y) {
+  constexpr int kUnits = P * kM8Tiles * MC, Q = 5;
+  const int lane = threadIdx.x & 63, i = lane & 15, kb = lane >> 4;
+  const int gu = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (gu >= nz * groups * kUnits) return;   // the last workgroup's spare waves
+  const int zg = gu / kUnits, unit = gu % kUnits, group = zg % groups;
+  const int m = (zg / groups) * (MC * 16) + (unit % MC) * 16 + i, n0 = (group * P * kM8Tiles + unit / MC) * 16 + 4 * kb;
+  if (m >= M || n0 >= N) return;
+  const int4v_t* q = part + ((size_t)zg * S * kUnits + unit) * 64 + lane;
+  int4v_t s = q[0];
+  for (int s0 = 1; s0 < S; s0 += Q) {
+    int4v_t v[Q];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) v[j] = q[(size_t)min(s0 + j, S - 1) * kUnits * 64];
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+      if (s0 + j < S) s += v[j];
+  }
+  m8_store(s, m, n0, M, N, sx, sw, bias, y);
+}
+
+struct M8Plan {
+  int mc, nz, d;   // 16-row chunks, row blocks, ring depth; mc == 0: not taken
+  MidSplit m;
+  size_t bytes() const { return mid_partial_bytes(m, nz, mc); }
+};
+
+// Row blocks: one up to 128 rows (the weights are read once), except two on
+// narrow N with short k chains, where the rows give the parallelism that more
+// splits would (5120^2 M = 96: 15.2 us for two blocks in three splits, 16.9
+// for one in six).  Depth: three stages while a compute unit holds one
+// workgroup, two (two workgroups fit) beyond.  Not taken: M <= 4, and M <= 16
+// where the GEMV is as fast (short, narrow shapes: N = 1024 M = 8 5.9 us
+// against 8.9; 5120^2 M = 8 10.5 against 10.7; 2048->4040 M = 16 / 40, with the
+// quantizer, 7.8 / 12.4 against 11.9 / 13.8; 3328->13000 M = 96 24.2 against
+// 26.3); above 128 rows the shapes whose
+// GEMM grid already fills the machine (N = 17408 M = 200 53 us against 58).
+M8Plan m8_plan(int64_t M, int64_t N, int64_t K) {
+  M8Plan p{0, 1, 2, {4, 1, 0}};
+  const int64_t ntile = (N + 15) / 16, nblk = K / kI8Blk, g8 = (ntile + 7) / 8;
+  if (M <= 4 || M > kM8MaxM || K % kI8Blk != 0 || K > (1 << 23)) return p;
+  const bool long_k = nblk >= 64;
+  if (nblk < 20 && ntile * nblk < 10000) return p;
+  if (M <= 16 && !long_k && g8 < 128 && !(M > 8 && g8 >= 32 && ntile * nblk >= 10000)) return p;
+  if (M > 64 && M <= 128 && nblk < 32 && g8 > 64 && g8 <= 128) return p;
+  if (M > 128 && !long_k && (g8 < 40 || (g8 > 128 && g8 < 256))) return p;
+  if (M > 128 || (!long_k && g8 <= 64 && M > (g8 <= 16 ? 32 : 48))) p.nz = 2;
+  const int mc = (int)((M + 16 * p.nz - 1) / (16 * p.nz));
+  p.mc = mc <= 4 ? mc : mc <= 6 ? 6 : 8;
+  p.m = mid_split(ntile, (nblk + 3) / 4, 4 * kW8TileBlockBytes, 4.0 * p.mc * 16 * kI8RowBytes, p.nz, p.mc);
+  p.d = p.m.groups * p.nz * p.m.s <= 256 && p.mc < 8 ? 3 : 2;
+  return p;
+}
+
+template <int P, int MC, int D>
+int launch_m8(const int8_t* qx, const float* sx, int M, int K, const int8_t* qw, const float* sw, const half_t* bias,
+              int N, half_t* y, const M8Plan& p, void* ws, W8Layout wl8, hipStream_t st) {
+  int4v_t* part = p.m.s > 1 ? reinterpret_cast<int4v_t*>(reinterpret_cast<uint8_t*>(ws) + kSplitCounterBytes) : nullptr;
+  hipLaunchKernelGGL((w8a8_mid_kernel<P, MC, D>), dim3((unsigned)p.m.groups, (unsigned)p.m.s, (unsigned)p.nz),
+                     dim3(128 * P), 0, st, qx, sx, M, K, qw, sw, bias, N, y, part, wl8);
+  if (p.m.s > 1)
+    hipLaunchKernelGGL((w8a8_mid_sum_kernel<P, MC>), dim3((unsigned)((p.nz * p.m.groups * P * kM8Tiles * MC + 3) / 4)),
+                       dim3(256), 0, st, part, p.m.s, (int)p.m.groups, p.nz, M, N, sx, sw, bias, y);
+  return check_launch("w8a8_mid");
+}
+
+template <int P>
+int launch_m8_plan(const int8_t* qx, const float* sx, int M, int K, const int8_t* qw, const float* sw,
+                   const half_t* bias, int N, half_t* y, const M8Plan& p, void* ws, W8Layout wl8, hipStream_t st) {
+  switch (p.mc * 10 + p.d) {
+    case 12: return launch_m8<P, 1, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 13: return launch_m8<P, 1, 3>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 22: return launch_m8<P, 2, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 23: return launch_m8<P, 2, 3>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 32: return launch_m8<P, 3, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 33: return launch_m8<P, 3, 3>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 42: return launch_m8<P, 4, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 43: return launch_m8<P, 4, 3>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    case 62: return launch_m8<4, 6, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);   // P = 4 beyond mc = 4
+    case 63: return launch_m8<4, 6, 3>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+    default: return launch_m8<4, 8, 2>(qx, sx, M, K, qw, sw, bias, N, y, p, ws, wl8, st);
+  }
+}
+
 constexpr int kW8A8GemvMaxM = 16;
 // Largest k of the W8A8 GEMM: its x and weight offsets are 32-bit (127 rows
 // of k bytes, 64 weight rows of k bytes); longer rows run the GEMV kernel 16
@@ -368,15 +708,26 @@ extern "C" int wq_w8a8_quantize(const uint16_t* x, int64_t m, int64_t k, int8_t*
   WQ_REQUIRE(m > 0 && m <= 0x7fffffff && k > 0 && k % 8 == 0 && k <= (1 << 26), WQ_ERR_INVALID_ARGUMENT,
              "need m >= 0 and 0 < k, k %% 8 == 0 (k = %lld)", (long long)k);
   WQ_REQUIRE(((uintptr_t)x | (uintptr_t)qx) % 16 == 0, WQ_ERR_INVALID_ARGUMENT, "x and qx must be 16-byte aligned");
-  hipLaunchKernelGGL(w8a8_quantize_kernel, dim3((unsigned)m), dim3(256), 0, as_stream(stream),
-                     reinterpret_cast<const half_t*>(x), (int)k, qx, x_scale);
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)m), dim3(threads), 0, as_stream(stream),
+                       reinterpret_cast<const half_t*>(x), (int)k, qx, x_scale);
+  };
+  const int64_t nc = k / 8;
+  if (m <= 512 && nc > 256 && nc <= 3 * 1024) {   // few rows: one round of loads over 16 waves
+    if (nc <= 1024) launch(w8a8_quantize_kernel<1024, 1>, 1024);
+    else launch(w8a8_quantize_kernel<1024, 3>, 1024);
+  } else if (nc <= 256) launch(w8a8_quantize_kernel<256, 1>, 256);
+  else if (nc <= 3 * 256) launch(w8a8_quantize_kernel<256, 3>, 256);
+  else if (nc <= 9 * 256) launch(w8a8_quantize_kernel<256, 9>, 256);
+  else launch(w8a8_quantize_kernel<256, 0>, 256);
   return check_launch("w8a8_quantize");
 }
 
 namespace {
 
 int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const int8_t* qweight,
-                     const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y, void* stream, int tiled) {
+                     const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y, void* ws, size_t ws_bytes,
+                     void* stream, int tiled) {
   if (m == 0 || n == 0) return WQ_OK;
   WQ_REQUIRE(qx && x_scale && qweight && w_scale && y, WQ_ERR_INVALID_ARGUMENT, "null pointer argument");
   WQ_REQUIRE(m > 0 && n > 0 && k > 0 && m <= 0x7fffffff && n <= 0x7fffffff && k <= (1 << 26),
@@ -389,6 +740,10 @@ int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t 
   const half_t* b = reinterpret_cast<const half_t*>(bias);
   half_t* yy = reinterpret_cast<half_t*>(y);
   const int64_t nsteps = k / kI8Step, ntile = (n + 15) / 16;
+  const M8Plan plan = m8_plan(m, n, k);
+  if (plan.mc > 0 && (plan.m.s == 1 || (ws != nullptr && ws_bytes >= plan.bytes())))
+    return (plan.m.p == 4 ? launch_m8_plan<4> : launch_m8_plan<5>)(qx, x_scale, (int)m, (int)k, qweight, w_scale, b,
+                                                                  (int)n, yy, plan, ws, wl8, as_stream(stream));
   if (m > kW8A8GemvMaxM && k % kI8Blk == 0 && k <= kW8A8GemmMaxK) {
     // GEMM: 128-row x tiles for long batches, 32-row ones otherwise; four
     // weight tiles per wave while that still leaves a full machine of
@@ -429,12 +784,29 @@ int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t 
 
 }  // namespace
 
+extern "C" int wq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k, size_t* bytes) {
+  WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");
+  WQ_REQUIRE(m >= 0 && n > 0 && k > 0 && m <= 0x7fffffff && n <= 0x7fffffff && k <= (1 << 26), WQ_ERR_INVALID_ARGUMENT,
+             "m, n, k out of range");
+  const M8Plan p = m8_plan(m, n, k);
+  *bytes = p.mc > 0 ? p.bytes() : 0;
+  return WQ_OK;
+}
+
 extern "C" int wq_w8a8_linear(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const int8_t* qweight,
                               const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y, void* stream) {
-  return w8a8_linear_impl(qx, x_scale, m, k, qweight, w_scale, n, bias, y, stream, 0);
+  return w8a8_linear_impl(qx, x_scale, m, k, qweight, w_scale, n, bias, y, nullptr, 0, stream, 0);
 }
 
 extern "C" int wq_w8a8_linear_tiled(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const void* tiles,
                                     const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y, void* stream) {
-  return w8a8_linear_impl(qx, x_scale, m, k, reinterpret_cast<const int8_t*>(tiles), w_scale, n, bias, y, stream, 1);
+  return w8a8_linear_impl(qx, x_scale, m, k, reinterpret_cast<const int8_t*>(tiles), w_scale, n, bias, y, nullptr, 0,
+                          stream, 1);
+}
+
+extern "C" int wq_w8a8_linear_ws(const int8_t* qx, const float* x_scale, int64_t m, int64_t k, const void* weight,
+                                 int32_t tiled, const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
+  return w8a8_linear_impl(qx, x_scale, m, k, reinterpret_cast<const int8_t*>(weight), w_scale, n, bias, y, workspace,
+                          workspace_bytes, stream, tiled ? 1 : 0);
 }
