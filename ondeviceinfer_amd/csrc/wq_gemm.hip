@@ -401,7 +401,6 @@ __global__ __launch_bounds__(256, 2) void wq_gemm_kernel(const half_t* __restric
 // order and stores y, so the result does not depend on arrival order.  The
 // counters sit in a fixed region at the start of the workspace and are back
 // at zero after every call.
-constexpr int kDeepMaxTiles = kSplitMaxCounters;          // (bx, by) tiles with a counter
 constexpr size_t kDeepCounterBytes = kSplitCounterBytes;
 
 template <GFmt F, int NT, int MT, int D>
@@ -643,54 +642,93 @@ int launch_gemm_deep(const half_t* x, int M, int K, const void* w, const void* m
   return check_launch(F == GFmt::W4 ? "w4_gemm_deep" : "w8_gemm_deep");
 }
 
-// Workgroups from which the prefill GEMM takes 256-wide n slices of 128-row
-// tiles (NT = 4, MT = 8): 384, three quarters of the 512 resident slots (the
-// 128-row grid at 448 workgroups ran the fused QKV at M = 2048 in 137 us
-// against 155 us for 64-row tiles, 5120^2 at M = 3072 (480) in 143 against
-// 171 us, down 458 against 565 us; at 320, 5120^2 at M = 2048, the 64-row
-// grid stays ahead, 118 against 129 us; same bits on every grid).
-constexpr long kWideGrid = 384;
+// The prefill grids: 64 NT columns x 16 MT rows per workgroup.
+enum class Grid { k4x8, k4x4, k2x8, k2x4, k1x4, kDeep };
 
-// Grids: 256-wide n slices of 128-row tiles (NT = 4, MT = 8) from kWideGrid
-// workgroups on.  Otherwise W4 takes the most work per
-// workgroup that still gives at least 384 workgroups: 128-wide slices of
-// 64-row tiles (NT = 2, MT = 4), then 64-wide slices (NT = 1), then 64-wide
-// slices of 32-row tiles on the deep ring (NT = 1, MT = 2, D = 4: three
-// blocks in flight; D = 6 was 2-15 % slower once the block math ran at raised
-// priority, e.g. 5120^2 at M = 65 17.4 against 20.4 us, q/o at M = 128 23.5
-// against 25.0 us, same bits).  The
-// narrow shapes gain most (k_proj 5120->1024: M = 2048 46.7 -> 38.0 us,
-// M = 512 37.4 -> 21.8 us; down 17408->5120 at M = 128 101 -> 77 us; 5120^2
-// at M = 2048 155 -> 127 us).  INT8 tiles take the same grids (5120^2 at
-// M = 2048 190 -> 159 us, k_proj at M = 512 48 -> 22 us); row-major INT8,
-// whose weight loads are 16 rows x 64 B, loses from two tiles per wave and
-// keeps 64-wide slices of 64-row (M <= 256) or 128-row tiles.
-// Whether launch_gemm_auto runs the deep ring on 32-row tiles for this shape.
+// Whether the deep ring on 32-row tiles may serve this shape: every plain grid
+// of narrower slices is below 384 workgroups (three quarters of the 512
+// resident slots of 128-row tiles).  Its k split keeps the shapes this rule
+// gives it (deep_splits).
+constexpr long kFullGrid = 384;
+
 bool gemm_takes_deep(long M, long N, bool w4_or_tiles) {
   const long ntile = (N + 15) / 16, mblk = (M + 127) / 128, mb64 = (M + 63) / 64;
-  if (((ntile + 15) / 16) * mblk >= kWideGrid || !w4_or_tiles) return false;
-  constexpr long kMinGrid = 384;
-  return ((ntile + 7) / 8) * mb64 < kMinGrid && ((ntile + 3) / 4) * mb64 < kMinGrid;
+  if (((ntile + 15) / 16) * mblk >= kFullGrid || !w4_or_tiles) return false;
+  return ((ntile + 7) / 8) * mb64 < kFullGrid && ((ntile + 3) / 4) * mb64 < kFullGrid;
+}
+
+// The grid of least estimated time for W4 weights or INT8 tiles (every grid
+// gives the same bits).  On MI355X a grid takes c rounds of 256 workgroups, c
+// = ceil(workgroups / 256), at a cost per round that hardly depends on how
+// many of a compute unit's workgroups run side by side, only on the tile:
+// K = 5120, us per round over M = 100..1500 on N = 5120..34816:
+//          4x8   4x4   2x8   2x4   1x4   deep 1x2
+//   W4     68    41.5  40    22    13.9  11.7
+//   INT8   77    48    45.5  24.5  14.3  12.6
+// A single round leaves each SIMD one wave, with nothing beside its load waits
+// (4x8 W4 92 us instead of 68; narrow tiles about twice), and an odd round of
+// 128-row tiles, two of which share a compute unit, runs its last one alone.
+// So rows padded to the tile and rounds left partly empty decide: fused gate_up
+// M = 400 4x8 pads to 512 rows in three rounds, 197 us, 4x4 to 448 in four, 170;
+// 17408->5120 M = 1500 2x4 takes four rounds, 290 us, 2x8 two, 265; 5120^2
+// M = 200 deep 34.4 us, 1x4 31.2; INT8 17408->5120 M = 200 deep 133 us, 1x4 84.
+// The widest tile keeps a 3 % lead: it reads the least through L2.
+struct GridCost {
+  Grid grid;
+  int nt, mt;
+  float w4, w8, alone;   // us per round (K = 5120), factor of a single round
+};
+constexpr GridCost kGridCosts[] = {{Grid::k4x8, 4, 8, 66.0f, 74.7f, 1.4f}, {Grid::k4x4, 4, 4, 41.5f, 48.0f, 1.4f},
+                                   {Grid::k2x8, 2, 8, 40.0f, 45.5f, 1.4f}, {Grid::k2x4, 2, 4, 22.0f, 24.5f, 1.6f},
+                                   {Grid::k1x4, 1, 4, 13.9f, 14.3f, 2.2f}, {Grid::kDeep, 1, 2, 11.7f, 12.6f, 1.9f}};
+
+// allow_deep / min_nt: the grids the caller can use (the fused epilogues have
+// no deep ring, and SiluPair pairs tiles within a wave).
+Grid gemm_grid(long M, long N, bool w4, bool allow_deep, int min_nt) {
+  const long ntile = (N + 15) / 16;
+  Grid best = Grid::k2x4;
+  float best_us = 1e30f;
+  for (const GridCost& g : kGridCosts) {
+    if ((g.grid == Grid::kDeep && !allow_deep) || g.nt < min_nt) continue;
+    const long wgs = ((ntile + 4 * g.nt - 1) / (4 * g.nt)) * ((M + 16 * g.mt - 1) / (16 * g.mt));
+    const long c = (wgs + 255) / 256;
+    float rounds = (float)c;
+    if (c == 1) rounds = g.alone;
+    else if (g.mt == 8 && (c & 1)) rounds += 0.15f;
+    const float us = rounds * (w4 ? g.w4 : g.w8);
+    if (us < best_us) {
+      best_us = us;
+      best = g.grid;
+    }
+  }
+  return best;
 }
 
 template <GFmt F>
 int launch_gemm_auto(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg,
                      const half_t* bias, half_t* y, hipStream_t s, int w8_tiled, void* ws = nullptr,
                      size_t ws_bytes = 0) {
-  const long ntile = (N + 15) / 16, mblk = (M + 127) / 128;
-  if (((ntile + 15) / 16) * mblk >= kWideGrid) return launch_gemm<F, 4, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
   if (F == GFmt::W4 || w8_tiled) {
-    constexpr long kMinGrid = 384;
-    const long mb64 = (M + 63) / 64;
-    if (((ntile + 7) / 8) * mb64 >= kMinGrid)
-      return launch_gemm<F, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
-    if (((ntile + 3) / 4) * mb64 >= kMinGrid)
-      return launch_gemm<F, 1, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
-    return launch_gemm_deep<F, 1, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled, ws, ws_bytes);
-  } else {
-    if (M <= 256) return launch_gemm<F, 1, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
-    return launch_gemm<F, 1, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+    const bool deep = gemm_takes_deep(M, N, true);
+    // The deep ring's k split, where there is one and its workspace, beats
+    // every whole-k grid of these shapes.
+    const bool split = F == GFmt::W4 && deep && bias == nullptr && ws != nullptr && deep_splits<1, 2>(M, N, K) > 1 &&
+                       ws_bytes >= deep_ws_bytes<1, 2>(M, N, K);
+    switch (split ? Grid::kDeep : gemm_grid(M, N, F == GFmt::W4, deep, 1)) {
+      case Grid::k4x8: return launch_gemm<F, 4, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k4x4: return launch_gemm<F, 4, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k2x8: return launch_gemm<F, 2, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k2x4: return launch_gemm<F, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k1x4: return launch_gemm<F, 1, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      default: return launch_gemm_deep<F, 1, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled, ws, ws_bytes);
+    }
   }
+  // Row-major INT8, whose weight loads are 16 rows x 64 B, loses 10-25 % from
+  // two tiles per wave: 64-wide slices below a full 128 x 256 grid.
+  const long ntile = (N + 15) / 16, mblk = (M + 127) / 128;
+  if (((ntile + 15) / 16) * mblk >= kFullGrid) return launch_gemm<F, 4, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+  if (M <= 256) return launch_gemm<F, 1, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+  return launch_gemm<F, 1, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
 }
 
 }  // namespace
@@ -707,51 +745,56 @@ size_t w4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return deep_ws_bytes<1, 2>((int)M, (int)N, (int)K);
 }
 
-// The grid launch_gemm_auto picks for a W4 (or INT8-tile) shape, when it is a wq_gemm_kernel
-// grid that can carry a fused epilogue: 1 = NT 4 / MT 8, 2 = NT 2 / MT 4,
-// 3 = NT 1 / MT 4 (Residual only: SiluPair pairs tiles within a wave); 0
-// otherwise.  SiluPair also needs the up tiles' offsets (nh + NT tiles of
-// block_bytes per 128-k block from a wave's first tile) inside the 31-bit
-// buffer range.
+// Whether a W4 (or INT8-tile) shape has a fused epilogue: 0 where the deep
+// ring may serve it; mode 1 (SiluPair) also needs gate and up tiles within one
+// wave (N % 32 == 0, and 128-wide slices that fill the machine) and the up
+// tiles' offsets (nh + NT tiles of block_bytes per 128-k block from a wave's
+// first tile) inside the 31-bit buffer range.
 int gemm_epi_plan(int64_t M, int64_t N, int64_t K, int mode, int64_t block_bytes) {
   const long ntile = (N + 15) / 16, mblk = (M + 127) / 128, mb64 = (M + 63) / 64;
-  int plan = 0;
-  if (((ntile + 15) / 16) * mblk >= kWideGrid) plan = 1;
-  else if (((ntile + 7) / 8) * mb64 >= 384) plan = 2;
-  else if (((ntile + 3) / 4) * mb64 >= 384) plan = 3;
+  if (gemm_takes_deep(M, N, true)) return 0;
   if (mode == 1) {
-    if (plan == 3 || N % 32 != 0) return 0;
+    if ((((ntile + 15) / 16) * mblk < kFullGrid && ((ntile + 7) / 8) * mb64 < kFullGrid) || N % 32 != 0) return 0;
     if ((ntile / 2 + 4) * (K / kW4BlockK) * block_bytes > 0x7fffffffL) return 0;
   }
-  return plan;
+  return 1;
 }
 
+namespace {
+
+template <GFmt F, Epi EP>
+int launch_gemm_epi(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* res,
+                    half_t* y, hipStream_t s) {
+  constexpr int tiled = F == GFmt::W8;
+  switch (gemm_grid(M, N, F == GFmt::W4, false, EP == Epi::SiluPair ? 2 : 1)) {
+    case Grid::k4x8: return launch_gemm<F, 4, 8, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k4x4: return launch_gemm<F, 4, 4, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k2x8: return launch_gemm<F, 2, 8, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k2x4: return launch_gemm<F, 2, 4, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    default:
+      if constexpr (EP == Epi::Residual)
+        return launch_gemm<F, 1, 4, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+      else
+        return fail(WQ_ERR_UNSUPPORTED, "GEMM epilogue: no grid pairs gate and up tiles");
+  }
+}
+
+}  // namespace
+
 // W4 prefill GEMM with a fused epilogue (mode 1 SiluPair, 2 Residual); the
-// caller has checked w4_gemm_epi_plan.
+// caller has checked gemm_epi_plan.
 int launch_w4_gemm_epi(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
                        int mode, const half_t* res, half_t* y, hipStream_t s) {
   const int bpg = G / kW4BlockK;
-  switch (gemm_epi_plan(M, N, K, mode, 1024) * 2 + (mode == 1 ? 0 : 1)) {
-    case 2: return launch_gemm<GFmt::W4, 4, 8, Epi::SiluPair>(x, M, K, tiles, meta, N, bpg, nullptr, y, s, 0);
-    case 3: return launch_gemm<GFmt::W4, 4, 8, Epi::Residual>(x, M, K, tiles, meta, N, bpg, nullptr, y, s, 0, res);
-    case 4: return launch_gemm<GFmt::W4, 2, 4, Epi::SiluPair>(x, M, K, tiles, meta, N, bpg, nullptr, y, s, 0);
-    case 5: return launch_gemm<GFmt::W4, 2, 4, Epi::Residual>(x, M, K, tiles, meta, N, bpg, nullptr, y, s, 0, res);
-    case 7: return launch_gemm<GFmt::W4, 1, 4, Epi::Residual>(x, M, K, tiles, meta, N, bpg, nullptr, y, s, 0, res);
-    default: return fail(WQ_ERR_UNSUPPORTED, "w4 GEMM epilogue: shape has no fused-epilogue grid");
-  }
+  return mode == 1 ? launch_gemm_epi<GFmt::W4, Epi::SiluPair>(x, M, K, tiles, meta, N, bpg, nullptr, y, s)
+                   : launch_gemm_epi<GFmt::W4, Epi::Residual>(x, M, K, tiles, meta, N, bpg, res, y, s);
 }
 
 // The same for INT8 tiles (scale: fp16 per output row).
 int launch_w8_gemm_epi(const half_t* x, int M, int K, const int8_t* tiles, const half_t* scale, int N, int mode,
                        const half_t* res, half_t* y, hipStream_t s) {
-  switch (gemm_epi_plan(M, N, K, mode, kW8TileBlockBytes) * 2 + (mode == 1 ? 0 : 1)) {
-    case 2: return launch_gemm<GFmt::W8, 4, 8, Epi::SiluPair>(x, M, K, tiles, scale, N, 1, nullptr, y, s, 1);
-    case 3: return launch_gemm<GFmt::W8, 4, 8, Epi::Residual>(x, M, K, tiles, scale, N, 1, nullptr, y, s, 1, res);
-    case 4: return launch_gemm<GFmt::W8, 2, 4, Epi::SiluPair>(x, M, K, tiles, scale, N, 1, nullptr, y, s, 1);
-    case 5: return launch_gemm<GFmt::W8, 2, 4, Epi::Residual>(x, M, K, tiles, scale, N, 1, nullptr, y, s, 1, res);
-    case 7: return launch_gemm<GFmt::W8, 1, 4, Epi::Residual>(x, M, K, tiles, scale, N, 1, nullptr, y, s, 1, res);
-    default: return fail(WQ_ERR_UNSUPPORTED, "INT8 GEMM epilogue: shape has no fused-epilogue grid");
-  }
+  return mode == 1 ? launch_gemm_epi<GFmt::W8, Epi::SiluPair>(x, M, K, tiles, scale, N, 1, nullptr, y, s)
+                   : launch_gemm_epi<GFmt::W8, Epi::Residual>(x, M, K, tiles, scale, N, 1, res, y, s);
 }
 
 // Wide N at 16 < M <= 64: the deep ring keeps three weight blocks per wave in
