@@ -88,6 +88,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int
 
 constexpr int kNtPolicy = 2;   // non-temporal: data streamed once
 
+// Activation rows in LDS, 16 chunks of 16 bytes: lane (i, kb) of a
+// 16x16x32 fragment read takes slot (2 kb + (w & 1) + 8 (w >> 1)) ^ i of row i
+// in k-step w.  ds_read_b128 serves lanes of neighbouring kb together, whose
+// slots have to differ below 128 bytes: with 4 kb + w, the order of the W4
+// tiles, half of the LDS cycles were bank conflicts, with this order none are (W4
+// 5120^2 M = 700 45.9 -> 45.4 us, fused gate_up M = 4096 1213 -> 1204).
+__device__ __forceinline__ int frag_slot(int i, int kb, int w) { return (2 * kb + (w & 1) + 8 * (w >> 1)) ^ i; }
+
+// The chunk of row r that slot s holds: W4 tiles take k = 32 kb + 8 w (chunk
+// 4 kb + w) in step w, INT8 tiles chunk 2 kb + (w & 1) + 8 (w >> 1).
+template <bool W4>
+__device__ __forceinline__ int slot_chunk(int r, int s) {
+  const int f = s ^ (r & 15);
+  return W4 ? 4 * ((f >> 1) & 3) + 2 * (f >> 3) + (f & 1) : f;
+}
+
 // Workspace layout shared by every kernel that splits a tile's k range over
 // workgroups (decode GEMV, 5-to-64-row kernel, deep-ring GEMM): uint32
 // arrival counters in this fixed region at the start, then that kernel's

@@ -5,8 +5,8 @@
 // workgroup); all four waves share a BM = 16*MT slice of M.  Per 128-k block:
 //  * the activation tile x[BM, 128] is copied buffer -> LDS with
 //    buffer_load_dwordx4 ... lds (no register staging) into a two-stage ring;
-//    16-byte chunk c of row r sits at slot c ^ (r & 15), so the sixteen rows
-//    a B-fragment read touches fall in sixteen different bank groups;
+//    row r's 16-byte chunks sit at slots turned by r & 15 (frag_slot), so a
+//    B-fragment read has no bank conflicts;
 //  * each wave loads its weight tiles straight from HBM into registers one
 //    block ahead (the W4 tile layout already is the MFMA A-fragment order)
 //    and dequantizes them there, one tile at a time;
@@ -55,9 +55,6 @@ struct WRegs<GFmt::W8, NT> {
   uint4_t a[NT], b[NT];
 };
 
-// LDS slot (16-byte chunk index inside a 256-byte row) of chunk c in row r.
-__device__ __forceinline__ int swz(int r, int c) { return c ^ (r & 15); }
-
 // The MT B-fragments of one k-step: fragment mt is row mt*16 + i of the
 // stage, so its address is a per-lane base plus the immediate mt*16 rows
 // (no address arithmetic per read).  Inline asm for the reason given at
@@ -92,12 +89,9 @@ __device__ __forceinline__ void gemm_block(const uint8_t* stage, const WRegs<F, 
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    // chunk of this k-step inside the 128-k block, matching the fragment
-    const int c = F == GFmt::W4 ? 4 * kb + w : 2 * kb + (w & 1) + 8 * (w >> 1);
-    // row r = mt*16 + i holds chunk c at slot c ^ (r & 15) = c ^ i
     uint4_t b[MT];
     lds_read_frags<MT>(b, (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)stage) +
-                              (uint32_t)(i * kRowBytes + (c ^ i) * 16));
+                              (uint32_t)(i * kRowBytes + frag_slot(i, kb, w) * 16));
     auto dequant = [&](int t) -> half8_t {
       if constexpr (F == GFmt::W4) {
         uint32_t c_lo, c_hi;
@@ -268,7 +262,7 @@ __global__ __launch_bounds__(256, 2) void wq_gemm_kernel(const half_t* __restric
 
   // Activation copy for block `blk` into stage `st`: instruction J of the
   // workgroup fills rows 4J..4J+3; lane L lands in row 4J + L/16, slot L%16,
-  // so it fetches chunk (L%16) ^ (row & 15) of that row.  The buffer ends at
+  // so it fetches chunk slot_chunk(row, L%16) of that row.  The buffer ends at
   // row M, so rows past it land as zeros.  With kInstrPerWave a multiple of
   // 4, row & 15 depends only on j & 3 and the lane: four lane offsets.
   static_assert(kInstrPerWave % 4 == 0, "x copy layout");
@@ -276,7 +270,7 @@ __global__ __launch_bounds__(256, 2) void wq_gemm_kernel(const half_t* __restric
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int rl = 4 * q + (lane >> 4);   // row & 15 of instruction j with j & 3 == q
-    xvo[q] = (uint32_t)((lane >> 4) * K * 2 + swz(rl, lane & 15) * 16);
+    xvo[q] = (uint32_t)((lane >> 4) * K * 2 + slot_chunk<F == GFmt::W4>(rl, lane & 15) * 16);
   }
   const half_t* xw = x + (size_t)m0 * K;
   const int64_t x_bytes = (int64_t)(M - m0) * K * 2;
@@ -437,7 +431,7 @@ __global__ __launch_bounds__(256) void wq_gemm_deep_kernel(const half_t* __restr
 #pragma unroll
   for (int j = 0; j < kInstrPerWave; ++j) {
     const int J = wave * kInstrPerWave + j;
-    xvo[j] = (uint32_t)((lane >> 4) * K * 2 + swz(4 * J + (lane >> 4), lane & 15) * 16);
+    xvo[j] = (uint32_t)((lane >> 4) * K * 2 + slot_chunk<F == GFmt::W4>(4 * J + (lane >> 4), lane & 15) * 16);
   }
   const half_t* xw = x + (size_t)m0 * K;
   const int64_t x_bytes = (int64_t)(M - m0) * K * 2;

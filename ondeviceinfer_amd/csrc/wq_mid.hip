@@ -11,7 +11,7 @@
 //    from LDS feeds two MFMAs) and the 128-k blocks of parity h, which halves
 //    the number of barriers per block; the two parities meet in LDS at the end;
 //  * a stage is two blocks: its x goes buffer -> LDS (rows past M read as
-//    zero, 16-byte chunk c of row r at slot c ^ (r & 15)), its weights straight
+//    zero, chunks at the slots of frag_slot), its weights straight
 //    into registers, D - 1 stages ahead (D = 3, and 2 where 48 or 64 rows fill
 //    the LDS and the registers: a deeper ring measured no faster there, nor
 //    did x staged through registers with the LDS reads one k-step ahead);
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(128 * P, MINW) void mid_kernel(
 #pragma unroll
   for (int j = 0; j < MC; ++j) {
     const int rr = 4 * (p * MC + j) + (lane >> 4);
-    xvo[j] = (uint32_t)(rr * K * 2 + ((lane & 15) ^ (rr & 15)) * 16);
+    xvo[j] = (uint32_t)(rr * K * 2 + slot_chunk<F == MFmt::W4>(rr, lane & 15) * 16);
   }
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, (int64_t)M * K * 2);
 
@@ -230,9 +230,7 @@ __global__ __launch_bounds__(128 * P, MINW) void mid_kernel(
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       uint4_t f[MC];
-      // k-step w's 16-byte chunk of this lane, at slot chunk ^ row (row & 15 = i)
-      const int c = F == MFmt::W4 ? 4 * kb + w : 2 * kb + (w & 1) + 8 * (w >> 1);
-      mid_read<MC>(f, base + (uint32_t)((c ^ i) * 16));
+      mid_read<MC>(f, base + (uint32_t)(frag_slot(i, kb, w) * 16));
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         half8_t a;
