@@ -275,6 +275,11 @@ __device__ __forceinline__ half4_t i8x4_to_h4(uint32_t w) {
   return r;
 }
 
+// Bytes 2 j, 2 j + 1 of one word (i8x4_to_h4's pairs).
+__device__ __forceinline__ half2_t i8_pair(uint32_t w, int j) {
+  return as_h2(__builtin_amdgcn_perm(w ^ 0x80808080u, 0x64646464u, j ? 0x00070006u : 0x00050004u)) + as_h2(0xE480E480u);
+}
+
 __device__ __forceinline__ half8_t i8x8_to_h8(uint32_t w0, uint32_t w1) {
   half8_t r;
   r.s0123 = i8x4_to_h4(w0);

@@ -65,12 +65,27 @@ __device__ __forceinline__ uint4_t lds_read16_off(uint32_t a) {
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "i"(OFF));
   return v;
 }
-template <int MT, int MTI = 0>
+template <int MT, int LO, int HI>
 __device__ __forceinline__ void lds_read_frags(uint4_t (&b)[MT], uint32_t a) {
-  if constexpr (MTI < MT) {
-    b[MTI] = lds_read16_off<MTI * 16 * kRowBytes>(a);
-    lds_read_frags<MT, MTI + 1>(b, a);
+  if constexpr (LO < HI) {
+    b[LO] = lds_read16_off<LO * 16 * kRowBytes>(a);
+    lds_read_frags<MT, LO + 1, HI>(b, a);
   }
+}
+// Wait until at most LEFT of the LDS reads issued are outstanding, tied to the
+// fragments [LO, HI) it completes so that no use moves above it.
+template <int MT, int LO, int HI, int LEFT>
+__device__ __forceinline__ void lds_wait_frags(uint4_t (&b)[MT]) {
+  static_assert(HI - LO >= 1 && HI - LO <= 4, "fragment count");
+  if constexpr (HI - LO == 1)
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[LO]) : "i"(LEFT));
+  else if constexpr (HI - LO == 2)
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[LO]), "+v"(b[LO + 1]) : "i"(LEFT));
+  else if constexpr (HI - LO == 3)
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]) : "i"(LEFT));
+  else
+    asm volatile("s_waitcnt lgkmcnt(%4)"
+                 : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]), "+v"(b[LO + 3]) : "i"(LEFT));
 }
 
 // One 128-k block of a wave's NT x MT tile: per 32-k step, MT B-fragments
@@ -83,34 +98,27 @@ __device__ __forceinline__ void lds_read_frags(uint4_t (&b)[MT], uint32_t a) {
 // its block math wins issue over one that is setting up its next block
 // (M = 4096, same box: fused QKV 281.8 -> 275.2 us, gate 656 -> 644 us,
 // k_proj 54.3 -> 49.6 us together with the load order of wq_gemm_kernel).
-template <GFmt F, int NT, int MT>
-__device__ __forceinline__ void gemm_block(const uint8_t* stage, const WRegs<F, NT>& cur, int i, int kb,
-                                           float4_t (&acc)[NT][MT]) {
+template <int NT, int MT>
+__device__ __forceinline__ void gemm_block_w4(const uint8_t* stage, const WRegs<GFmt::W4, NT>& cur, int i, int kb,
+                                              float4_t (&acc)[NT][MT]) {
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     uint4_t b[MT];
-    lds_read_frags<MT>(b, (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)stage) +
+    lds_read_frags<MT, 0, MT>(b, (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)stage) +
                               (uint32_t)(i * kRowBytes + frag_slot(i, kb, w) * 16));
     auto dequant = [&](int t) -> half8_t {
-      if constexpr (F == GFmt::W4) {
-        uint32_t c_lo, c_hi;
-        w4_zero_consts((cur.z[t] >> (4 * (i & 7))) & 0xFu, c_lo, c_hi);
-        const half2_t s2 = as_h2((uint32_t)cur.s[t] * 0x00010001u);
-        const uint32_t word = w == 0 ? cur.w[t].x : w == 1 ? cur.w[t].y : w == 2 ? cur.w[t].z : cur.w[t].w;
-        return w4_word_to_h8_scaled(word, c_lo, c_hi, s2);
-      } else {
-        return w == 0 ? i8x8_to_h8(cur.a[t].x, cur.a[t].y)
-             : w == 1 ? i8x8_to_h8(cur.a[t].z, cur.a[t].w)
-             : w == 2 ? i8x8_to_h8(cur.b[t].x, cur.b[t].y)
-                      : i8x8_to_h8(cur.b[t].z, cur.b[t].w);
-      }
+      uint32_t c_lo, c_hi;
+      w4_zero_consts((cur.z[t] >> (4 * (i & 7))) & 0xFu, c_lo, c_hi);
+      const half2_t s2 = as_h2((uint32_t)cur.s[t] * 0x00010001u);
+      const uint32_t word = w == 0 ? cur.w[t].x : w == 1 ? cur.w[t].y : w == 2 ? cur.w[t].z : cur.w[t].w;
+      return w4_word_to_h8_scaled(word, c_lo, c_hi, s2);
     };
     half8_t a = dequant(0);
-    lds_wait_first_half<MT>(b);
+    lds_wait_frags<MT, 0, MT / 2, MT - MT / 2>(b);
 #pragma unroll
     for (int mt = 0; mt < MT / 2; ++mt) acc[0][mt] = mfma16(a, __builtin_bit_cast(half8_t, b[mt]), acc[0][mt]);
-    lds_wait_rest<MT>(b);
+    lds_wait_frags<MT, MT / 2, MT, 0>(b);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const half8_t a_next = t + 1 < NT ? dequant(t + 1) : a;
@@ -121,6 +129,75 @@ __device__ __forceinline__ void gemm_block(const uint8_t* stage, const WRegs<F, 
     }
   }
   __builtin_amdgcn_s_setprio(0);
+}
+
+// The same block for INT8 weights, with the order of issue fixed: each pair of
+// converted weights (three VALU operations) sits between two MFMAs, and the
+// next k-step's fragment reads go out as the last tile is done with the
+// current ones, so one wave by itself keeps the matrix cores fed past the
+// block's first reads.  Left to the compiler, a k-step began with two tiles'
+// conversions and its reads, with no MFMA beside them (MI355X, us before ->
+// now: 17408->5120 M = 700 / 1500 162 -> 153 / 263 -> 257, fused gate_up M =
+// 200 / 4096 131 -> 126 / 1371 -> 1343, 5120^2 M = 100 24.2 -> 22.6).  W4
+// gained nothing from it (0 to 3 % slower: a pair is four dependent
+// operations) and keeps the form above.
+template <int NT, int MT>
+__device__ __forceinline__ void gemm_block_w8(const uint8_t* stage, const WRegs<GFmt::W8, NT>& cur, int i, int kb,
+                                              float4_t (&acc)[NT][MT]) {
+  __builtin_amdgcn_s_setprio(1);
+  constexpr int H = MT / 2;
+  const uint32_t row = (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)stage) + (uint32_t)(i * kRowBytes);
+  auto addr = [&](int w) { return row + (uint32_t)(frag_slot(i, kb, w) * 16); };
+  // Elements 2 j, 2 j + 1 of tile t's fragment of k-step w.
+  auto piece = [&](int t, int w, int j) -> half2_t {
+    const uint4_t& v = w < 2 ? cur.a[t] : cur.b[t];
+    return i8_pair((w & 1) ? (j < 2 ? v.z : v.w) : (j < 2 ? v.x : v.y), j & 1);
+  };
+  auto pack = [](half2_t (&p)[4]) -> half8_t {
+    half8_t r;
+    r.s01 = p[0]; r.s23 = p[1]; r.s45 = p[2]; r.s67 = p[3];
+    return r;
+  };
+  uint4_t b[MT];
+  lds_read_frags<MT, 0, MT>(b, addr(0));
+  half2_t nx[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) nx[j] = piece(0, 0, j);
+  half8_t a = pack(nx);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    lds_wait_frags<MT, 0, H, MT - H>(b);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int tn = t + 1 < NT ? t + 1 : 0, wn = t + 1 < NT ? w : w + 1;
+      const bool last = t == NT - 1 && w < 3;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        if (t == 0 && mt == H) {   // NT == 1: the next step's first H reads are behind these
+          if (NT == 1 && w < 3) lds_wait_frags<MT, H, MT, H>(b);
+          else lds_wait_frags<MT, H, MT, 0>(b);
+        }
+        acc[t][mt] = mfma16(a, __builtin_bit_cast(half8_t, b[mt]), acc[t][mt]);
+        if (wn < 4) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if ((MT >= 4 ? j : j * MT / 4) == mt) nx[j] = piece(tn, wn, j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (last && mt == H - 1) lds_read_frags<MT, 0, H>(b, addr(w + 1));
+        if (last && mt == MT - 1) lds_read_frags<MT, H, MT>(b, addr(w + 1));
+      }
+      a = pack(nx);
+    }
+  }
+  __builtin_amdgcn_s_setprio(0);
+}
+
+template <GFmt F, int NT, int MT>
+__device__ __forceinline__ void gemm_block(const uint8_t* stage, const WRegs<F, NT>& cur, int i, int kb,
+                                           float4_t (&acc)[NT][MT]) {
+  if constexpr (F == GFmt::W4) gemm_block_w4<NT, MT>(stage, cur, i, kb, acc);
+  else gemm_block_w8<NT, MT>(stage, cur, i, kb, acc);
 }
 
 // Epilogue: lane holds D[n = 4*kb + v][m = i] of every (tile, m-subtile).
