@@ -342,12 +342,12 @@ __global__ __launch_bounds__(256, 2) void wq_gemm_kernel(const half_t* __restric
   // so it fetches chunk slot_chunk(row, L%16) of that row.  The buffer ends at
   // row M, so rows past it land as zeros.  With kInstrPerWave a multiple of
   // 4, row & 15 depends only on j & 3 and the lane: four lane offsets.
-  static_assert(kInstrPerWave % 4 == 0, "x copy layout");
-  uint32_t xvo[4];
+  constexpr int kXvo = kInstrPerWave % 4 == 0 ? 4 : kInstrPerWave;
+  uint32_t xvo[kXvo];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int rl = 4 * q + (lane >> 4);   // row & 15 of instruction j with j & 3 == q
-    xvo[q] = (uint32_t)((lane >> 4) * K * 2 + slot_chunk<F == GFmt::W4>(rl, lane & 15) * 16);
+  for (int q = 0; q < kXvo; ++q) {
+    const int r = 4 * (wave * kInstrPerWave + q) + (lane >> 4);
+    xvo[q] = (uint32_t)((lane >> 4) * K * 2 + slot_chunk<F == GFmt::W4>(r, lane & 15) * 16);
   }
   const half_t* xw = x + (size_t)m0 * K;
   const int64_t x_bytes = (int64_t)(M - m0) * K * 2;
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256, 2) void wq_gemm_kernel(const half_t* __restric
 #pragma unroll
     for (int j = 0; j < kInstrPerWave; ++j) {
       const int J = wave * kInstrPerWave + j;
-      lds_load16(r, xvo[j & 3], (uint32_t)(4 * J * K * 2), xs + st * kStageBytes + J * 1024);
+      lds_load16(r, xvo[j % kXvo], (uint32_t)(4 * J * K * 2), xs + st * kStageBytes + J * 1024);
     }
   };
 
@@ -714,7 +714,7 @@ int launch_gemm_deep(const half_t* x, int M, int K, const void* w, const void* m
 }
 
 // The prefill grids: 64 NT columns x 16 MT rows per workgroup.
-enum class Grid { k4x8, k4x4, k2x8, k2x4, k1x4, kDeep };
+enum class Grid { k4x8, k4x7, k4x6, k4x4, k2x8, k2x6, k2x5, k2x4, k1x4, kDeep };
 
 // Whether the deep ring on 32-row tiles may serve this shape: every plain grid
 // of narrower slices is below 384 workgroups (three quarters of the 512
@@ -733,25 +733,34 @@ bool gemm_takes_deep(long M, long N, bool w4_or_tiles) {
 // = ceil(workgroups / 256), at a cost per round that hardly depends on how
 // many of a compute unit's workgroups run side by side, only on the tile:
 // K = 5120, us per round over M = 100..1500 on N = 5120..34816:
-//          4x8   4x4   2x8   2x4   1x4   deep 1x2
+//          4x8   4x4   2x8   2x4   1x4   deep 1x2   (4x6, 4x7, 2x5, 2x6 in between)
 //   W4     68    41.5  40    22    13.9  11.7
 //   INT8   77    48    45.5  24.5  14.3  12.6
 // A single round leaves each SIMD one wave, with nothing beside its load waits
-// (4x8 W4 92 us instead of 68; narrow tiles about twice), and an odd round of
-// 128-row tiles, two of which share a compute unit, runs its last one alone.
-// So rows padded to the tile and rounds left partly empty decide: fused gate_up
-// M = 400 4x8 pads to 512 rows in three rounds, 197 us, 4x4 to 448 in four, 170;
-// 17408->5120 M = 1500 2x4 takes four rounds, 290 us, 2x8 two, 265; 5120^2
-// M = 200 deep 34.4 us, 1x4 31.2; INT8 17408->5120 M = 200 deep 133 us, 1x4 84.
+// (4x8 W4 92 us instead of 68; narrow tiles about 1.75 times and more), and an
+// odd round of 112- or 128-row tiles, two of which share a compute unit, runs
+// its last one alone.  So rows padded to the tile and rounds left partly empty
+// decide, and the tile heights in between give a ragged M a grid that does
+// neither (us, W4 / INT8):
+//   17408->5120 M = 777   2x4 (520 workgroups, three rounds) 199 / 221 -> 2x5 (400, two) 175 / 163
+//   17408->5120 M = 1500  2x4 (960, four) 290 / 280 -> 2x8 (480, two) 264 / 257
+//   5120^2 M = 777        64 / 73 -> 2x5 56 / 57;  M = 1000  72 / 87 -> 66 / 67
+//   fused QKV M = 1500    128 / 149 -> 119 / 123 (4x6)
+//   fused gate_up M = 777 4x8 271 / 309 -> 4x7 254 / 281;  M = 400  197 / 205 -> 172 / 184 (4x6)
+//   5120->17408 M = 200   67 / 79 -> 59 / 61 (2x5)
+//   5120^2 M = 200        deep 34.4 / 37 -> 1x4 30 / 31; INT8 17408->5120 133 -> 95
 // The widest tile keeps a 3 % lead: it reads the least through L2.
 struct GridCost {
   Grid grid;
   int nt, mt;
   float w4, w8, alone;   // us per round (K = 5120), factor of a single round
 };
-constexpr GridCost kGridCosts[] = {{Grid::k4x8, 4, 8, 66.0f, 74.7f, 1.4f}, {Grid::k4x4, 4, 4, 41.5f, 48.0f, 1.4f},
-                                   {Grid::k2x8, 2, 8, 40.0f, 45.5f, 1.4f}, {Grid::k2x4, 2, 4, 22.0f, 24.5f, 1.6f},
-                                   {Grid::k1x4, 1, 4, 13.9f, 14.3f, 2.2f}, {Grid::kDeep, 1, 2, 11.7f, 12.6f, 1.9f}};
+constexpr GridCost kGridCosts[] = {
+    {Grid::k4x8, 4, 8, 66.0f, 74.7f, 1.4f}, {Grid::k4x7, 4, 7, 60.0f, 68.0f, 1.4f},
+    {Grid::k4x6, 4, 6, 53.8f, 61.4f, 1.4f}, {Grid::k4x4, 4, 4, 41.5f, 48.0f, 1.4f},
+    {Grid::k2x8, 2, 8, 40.0f, 45.5f, 1.4f}, {Grid::k2x6, 2, 6, 31.0f, 35.0f, 1.7f},
+    {Grid::k2x5, 2, 5, 27.0f, 30.5f, 1.75f}, {Grid::k2x4, 2, 4, 22.0f, 24.5f, 1.75f},
+    {Grid::k1x4, 1, 4, 13.9f, 14.3f, 2.2f}, {Grid::kDeep, 1, 2, 11.7f, 12.6f, 1.9f}};
 
 // allow_deep / min_nt: the grids the caller can use (the fused epilogues have
 // no deep ring, and SiluPair pairs tiles within a wave).
@@ -765,7 +774,7 @@ Grid gemm_grid(long M, long N, bool w4, bool allow_deep, int min_nt) {
     const long c = (wgs + 255) / 256;
     float rounds = (float)c;
     if (c == 1) rounds = g.alone;
-    else if (g.mt == 8 && (c & 1)) rounds += 0.15f;
+    else if (g.mt >= 7 && (c & 1)) rounds += 0.15f;
     const float us = rounds * (w4 ? g.w4 : g.w8);
     if (us < best_us) {
       best_us = us;
@@ -787,8 +796,12 @@ int launch_gemm_auto(const half_t* x, int M, int K, const void* w, const void* m
                        ws_bytes >= deep_ws_bytes<1, 2>(M, N, K);
     switch (split ? Grid::kDeep : gemm_grid(M, N, F == GFmt::W4, deep, 1)) {
       case Grid::k4x8: return launch_gemm<F, 4, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k4x7: return launch_gemm<F, 4, 7>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k4x6: return launch_gemm<F, 4, 6>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k4x4: return launch_gemm<F, 4, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k2x8: return launch_gemm<F, 2, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k2x6: return launch_gemm<F, 2, 6>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
+      case Grid::k2x5: return launch_gemm<F, 2, 5>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k2x4: return launch_gemm<F, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k1x4: return launch_gemm<F, 1, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       default: return launch_gemm_deep<F, 1, 2, 4>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled, ws, ws_bytes);
@@ -839,8 +852,12 @@ int launch_gemm_epi(const half_t* x, int M, int K, const void* w, const void* me
   constexpr int tiled = F == GFmt::W8;
   switch (gemm_grid(M, N, F == GFmt::W4, false, EP == Epi::SiluPair ? 2 : 1)) {
     case Grid::k4x8: return launch_gemm<F, 4, 8, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k4x7: return launch_gemm<F, 4, 7, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k4x6: return launch_gemm<F, 4, 6, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     case Grid::k4x4: return launch_gemm<F, 4, 4, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     case Grid::k2x8: return launch_gemm<F, 2, 8, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k2x6: return launch_gemm<F, 2, 6, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
+    case Grid::k2x5: return launch_gemm<F, 2, 5, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     case Grid::k2x4: return launch_gemm<F, 2, 4, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     default:
       if constexpr (EP == Epi::Residual)

@@ -13,10 +13,12 @@ from ondeviceinfer_amd.weight_quantization import backend as wq
 pytestmark = pytest.mark.gpu
 
 
-# (m, n, k): W4 on 64 columns x 4 tiles (129, 448), both n edges (partial last
-# slice: 34800 = 2175 tiles); 128-row two-tile grid (1345, 1500; 5112 ends
-# inside a tile); 64-row one-tile grid (200, 449); two-tile 64-row grid.
-SHAPES = [(129, 34816, 256), (448, 34800, 128), (1345, 5120, 384), (1500, 5112, 256), (200, 5120, 640),
+# (m, n, k), one tile height after the other: 2 tiles x 80 rows (129; 673 =
+# 8 x 80 + 33), 4 x 96 (448 ends inside a block, 34800 inside a slice; 577 =
+# 6 x 96 + 1), 4 x 112 (777, 785 takes 128), 2 x 96 (1056 = 11 x 96), 2 x 128
+# (1345, 1500; 5112 ends inside a tile), 1 x 64, 2 x 64, 4 x 64.
+SHAPES = [(129, 34816, 256), (673, 7168, 384), (448, 34800, 128), (577, 17400, 256), (777, 34816, 128),
+          (785, 34816, 128), (1056, 5112, 256), (1345, 5120, 384), (1500, 5112, 256), (200, 5120, 640),
           (449, 4040, 256), (700, 5120, 256)]
 
 
