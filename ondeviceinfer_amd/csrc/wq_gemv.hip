@@ -1,4 +1,4 @@
-// Decode / small-batch kernels (M <= 64): HBM-streaming MFMA GEMV.
+// Decode kernels (M <= 4) and the skinny kernels (M <= 64 beside wq_mid.hip): HBM-streaming MFMA GEMV.
 //
 // Work unit: one 16-row tile x one 128-k block = one 1 KiB coalesced load
 // (W4 tile layout) or two 16 B-per-lane loads (INT8 row-major).  A workgroup

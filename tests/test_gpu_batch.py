@@ -1,4 +1,4 @@
-"""GPU parity of the small-batch W4A16 kernel (wq_batch.hip: 12 <= M <= 32 on
+"""GPU parity of the small-batch W4A16 kernel (wq_mid.hip: 12 <= M <= 32 on
 narrow N, activations shared in LDS, k split over workgroups) against the
 CPU oracle, through the backend and the C ABI.
 
