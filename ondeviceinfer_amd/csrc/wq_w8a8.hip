@@ -14,6 +14,7 @@
 #include "wq_status.h"
 
 #include <math.h>
+#include <type_traits>
 
 namespace wq {
 namespace {
@@ -691,6 +692,138 @@ int launch_m8_plan(const int8_t* qx, const float* sx, int M, int K, const int8_t
   }
 }
 
+// Long batches over INT8 tiles: 256 x 256 output tiles, both operands in LDS.
+//
+// The 128 x 128 tiles of the kernel above stop at every 128-k block for its
+// copies (vmcnt(0), barrier, first fragment reads) and read each x fragment for
+// two MFMAs.  Here eight waves (wm, wn) of 128 rows x 64 columns share stages of
+// x (32 KiB, rows as above) and weights (32 KiB; the tile layout already is the
+// order fragments are read in) in a two-stage ring, copied buffer -> LDS a whole
+// block ahead; the 4 + 8 fragments of a 64-k step are read while the 32 MFMAs of
+// the step before run, across the block's barrier too.  A block takes 1.7-2.0 us
+// whether 4 or 256 workgroups run and however the reads are placed or the slots
+// ordered, i.e. about 32 cycles per MFMA: bound by issue to the matrix cores.
+// Workgroups resident on one XCD take neighbouring row blocks of one column
+// slice.  One workgroup per compute unit (128 KiB of LDS).
+// MI355X, us before -> now (without the quantizer): 5120->7168 M = 2048 / 4096
+// 112.9 / 181.9 -> 80.8 / 161.7, 5120^2 M = 3000 114 -> 81, 5120->17408 M = 1500 /
+// 4096 184 / 463 -> 158 / 399, 5120->34816 M = 4096 968 -> 777 (1.88 POP/s),
+// 17408->5120 M = 3000 291 -> 228.
+constexpr int kBigTiles = 16, kBigRows = 256;            // of a workgroup
+constexpr int kBigXBytes = kBigRows * kI8RowBytes;       // x of a stage
+constexpr int kBigStageBytes = kBigXBytes + kBigTiles * (int)kW8TileBlockBytes;
+
+template <int LO, int N>
+__device__ __forceinline__ void big_read_x(uint4_t (&b)[8], uint32_t a) {
+  if constexpr (N > 0) {
+    b[LO] = i8_lds_read_off<LO * 16 * kI8RowBytes>(a);
+    big_read_x<LO + 1, N - 1>(b, a);
+  }
+}
+// All LDS reads done, tied to the fragments so that no use moves above it.
+__device__ __forceinline__ void big_wait(uint4_t (&a)[4], uint4_t (&b)[8]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]),
+                 "+v"(b[4]), "+v"(b[5]), "+v"(b[6]), "+v"(b[7]));
+}
+
+__global__ __launch_bounds__(512, 2) void w8a8_gemm256_kernel(const int8_t* __restrict__ qx, const float* __restrict__ sx,
+                                                              int M, int K, const int8_t* __restrict__ qw,
+                                                              const float* __restrict__ sw,
+                                                              const half_t* __restrict__ bias, int N,
+                                                              half_t* __restrict__ y) {
+  __shared__ __attribute__((aligned(1024))) uint8_t xs[2 * kBigStageBytes];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wn = wave & 3, wm = wave >> 2, i = lane & 15, kb = lane >> 4;
+  const int ntile = (N + 15) >> 4, nblk = K / kI8Blk, mblk = (M + kBigRows - 1) / kBigRows;
+  // XCD x (flat id mod 8) takes the x-th run of workgroups, row block fastest.
+  const int g = (int)gridDim.x, q8 = g >> 3, r8 = g & 7, xcd = (int)blockIdx.x & 7;
+  const int id = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+  const int tile0 = id / mblk * kBigTiles, m0 = id % mblk * kBigRows;
+
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(qx + (size_t)m0 * K, (int64_t)(M - m0) * K);
+  const __amdgpu_buffer_rsrc_t rw = buf_rsrc(qw + (size_t)tile0 * nblk * kW8TileBlockBytes,
+                                             (int64_t)(ntile - tile0) * nblk * kW8TileBlockBytes);
+  // x instruction J = 4 wave + j: rows 8 J .. 8 J + 7, lane L chunk
+  // i8_swz(row, L % 8) of row 8 J + L / 8; weight instruction: piece j & 1 of
+  // tile 2 wave + j / 2.
+  uint32_t xvo[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xvo[j] = (uint32_t)((lane >> 3) * K + 16 * i8_swz(8 * j + (lane >> 3), lane & 7));
+  constexpr uint32_t kPastEnd = 0x80000000u;
+  auto fetch = [&](int blk, int st) {   // past the last block: zeros
+    uint8_t* stage = xs + st * kBigStageBytes;
+    const bool live = blk < nblk;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int J = 4 * wave + j;
+      lds_load16(rx, xvo[j & 1], live ? (uint32_t)(8 * J) * (uint32_t)K + (uint32_t)(blk * kI8Blk) : kPastEnd,
+                 stage + J * 1024);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = 2 * wave + (j >> 1);
+      lds_load16(rw, (uint32_t)lane * 16,
+                 live ? (uint32_t)(t * nblk + blk) * (uint32_t)kW8TileBlockBytes + (uint32_t)(j & 1) * 1024 : kPastEnd,
+                 stage + kBigXBytes + t * kW8TileBlockBytes + (j & 1) * 1024);
+    }
+  };
+
+  int4v_t acc[4][8];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) acc[t][mt] = int4v_t{0, 0, 0, 0};
+  const uint32_t lds = (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)xs);
+  const uint32_t xa = lds + (uint32_t)((wm * 128 + i) * kI8RowBytes);
+  const uint32_t wa = lds + (uint32_t)(kBigXBytes + wn * 4 * kW8TileBlockBytes + lane * 16);
+
+  uint4_t a0[4], b0[8], a1[4], b1[8];   // fragments of the two 64-k steps
+  auto read = [&](auto step, uint32_t so, uint4_t (&a)[4], uint4_t (&b)[8]) {
+    constexpr int s = decltype(step)::value;
+    a[0] = i8_lds_read_off<s * 1024>(wa + so);
+    a[1] = i8_lds_read_off<s * 1024 + 2048>(wa + so);
+    a[2] = i8_lds_read_off<s * 1024 + 4096>(wa + so);
+    a[3] = i8_lds_read_off<s * 1024 + 6144>(wa + so);
+    big_read_x<0, 8>(b, xa + so + (uint32_t)(i8_swz(i, 4 * s + kb) * 16));
+  };
+  auto math = [&](const uint4_t (&a)[4], const uint4_t (&b)[8]) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t][mt] = mfma_i8(a[t], b[mt], acc[t][mt]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  fetch(0, 0);
+  fetch(1, 1);
+  __builtin_amdgcn_s_waitcnt(8 | (0x7 << 4) | (0xF << 8));   // stage 0 landed, stage 1's eight copies may be in flight
+  __builtin_amdgcn_s_barrier();
+  read(std::integral_constant<int, 0>{}, 0, a0, b0);
+  for (int blk = 0; blk < nblk; ++blk) {
+    const uint32_t so = (uint32_t)((blk & 1) * kBigStageBytes);
+    big_wait(a0, b0);
+    read(std::integral_constant<int, 1>{}, so, a1, b1);
+    math(a0, b0);
+    big_wait(a1, b1);
+    __builtin_amdgcn_s_waitcnt(0);    // this wave's part of the next stage landed ...
+    __builtin_amdgcn_s_barrier();     // ... everyone's, and everyone has read this stage
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(blk + 2, blk & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    read(std::integral_constant<int, 0>{}, (uint32_t)kBigStageBytes - so, a0, b0);
+    math(a1, b1);
+  }
+  big_wait(a0, b0);                 // the run-out's reads and copies
+  __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+      m8_store(acc[t][mt], m0 + wm * 128 + mt * 16 + i, (tile0 + wn * 4 + t) * 16 + 4 * kb, M, N, sx, sw, bias, y);
+}
+
 constexpr int kW8A8GemvMaxM = 16;
 // Largest k of the W8A8 GEMM: its x and weight offsets are 32-bit (127 rows
 // of k bytes, 64 weight rows of k bytes); longer rows run the GEMV kernel 16
@@ -755,6 +888,17 @@ int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t 
     const bool two_tiles = tiled && big_m && (ntile + 7) / 8 * mblocks >= 512;
     const int nt = two_tiles ? 2 : (ntile + 15) / 16 * mblocks >= 256 ? 4 : 1;
     WQ_REQUIRE(mblocks <= 65535, WQ_ERR_UNSUPPORTED, "too many rows for the W8A8 GEMM grid");
+    // 256 x 256 tiles where their rounds of 256 workgroups cost less: one costs
+    // 3.0 to 3.15 rounds of the 128 x 128 tiles (72-86 against 26-28 us at
+    // K = 5120, 63-67 against 20-22 us per 5120 of K = 17408).  Just past the
+    // line the other way: 5120^2 M = 4096 (2 against 5 rounds) 152 against 128 us,
+    // 5120->17408 M = 777 (2 against 4) 148 against 118.
+    const int64_t big_wgs = (ntile + kBigTiles - 1) / kBigTiles * ((m + kBigRows - 1) / kBigRows);
+    if (two_tiles && 31 * ((big_wgs + 255) / 256) < 10 * (((ntile + 7) / 8 * mblocks + 255) / 256)) {
+      hipLaunchKernelGGL(w8a8_gemm256_kernel, dim3((unsigned)big_wgs), dim3(512), 0, as_stream(stream), qx, x_scale,
+                         (int)m, (int)k, qweight, w_scale, b, (int)n, yy);
+      return check_launch("w8a8_gemm256");
+    }
     const dim3 grid((unsigned)((ntile + 4 * nt - 1) / (4 * nt)), (unsigned)mblocks);
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), qx, x_scale, (int)m, (int)k, qweight,

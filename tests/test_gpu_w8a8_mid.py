@@ -81,3 +81,23 @@ def test_w8a8_quantize_non_finite_rows():
     assert np.array_equal(qx[2], row)
     row[5] = -127
     assert np.array_equal(qx[1], row)
+
+
+@pytest.mark.parametrize('m,n,k,bias', [(4000, 4040, 256, False), (3900, 4088, 128, True), (2000, 8190, 384, True),
+                                        (2048, 7168, 640, False)])
+def test_w8a8_256_tiles_exact(gpu, m, n, k, bias):
+    """256 x 256 tiles (long batches over INT8 tiles; ragged rows and columns, one to five blocks): sampled rows equal
+    the integer oracle and every row the row-major GEMM, bit for bit (exact integer sums, one scaling order)."""
+    rng = np.random.default_rng(m + n + k)
+    qx, qw = (rng.integers(-127, 128, s, dtype=np.int8) for s in ((m, k), (n, k)))
+    sx, sw = (rng.uniform(1e-3, 1e-2, s).astype(np.float32) for s in (m, n))
+    b = rng.standard_normal(n).astype(np.float16) if bias else None
+    td = [None if v is None else torch.from_numpy(v).to(gpu) for v in (qx, sx, qw, sw, b)]
+    y = _native.w8a8_linear(td[0], td[1], _native.w8_repack(td[2]), td[3], td[4])
+    assert torch.equal(y, _native.w8a8_linear(*td))
+    rows = [0, 1, 127, 128, 255, 256, m - 17, m - 1]
+    acc = qx[rows].astype(np.int64) @ qw.astype(np.int64).T
+    want = acc.astype(np.float32) * sx[rows][:, None] * sw[None]
+    if bias:
+        want = want + b.astype(np.float32)
+    assert np.array_equal(y.cpu().numpy()[rows], want.astype(np.float16))
