@@ -101,9 +101,8 @@ int wq_w4_decode_rows(const int32_t* weight_packed, const float* weight_scale,
  * GEMV (m <= 4), the kernel of 5 to 64 rows and the deep-ring GEMM on the
  * smallest prefill grids (m > 64 on narrow n).  The counters sit in a fixed
  * 16 KiB region at the start, so one buffer sized for the largest shape
- * serves every shape.  It must be zero-filled once before first use
- * (5 <= m <= 64 uses counters only at 12 <= m <= 32 with n <= 18432,
- * k <= 8192 and k % 512 == 0; elsewhere any scratch will do); every call
+ * serves every shape.  It must be zero-filled once before first use (for one
+ * shape alone: as many bytes as wq_w4a16_workspace_zeroed says); every call
  * leaves the counters zeroed again, so it can be reused by later calls (and
  * graph replays) on the same stream.  Calls that may run concurrently need
  * separate workspaces.  With a NULL or smaller workspace the linear runs
@@ -112,6 +111,12 @@ int wq_w4_decode_rows(const int32_t* weight_packed, const float* weight_scale,
  * whole k range: the same values up to fp32 summation order).  Replaces
  * marlin_make_workspace_new (backend.py:223). */
 int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t group_size, size_t* bytes);
+
+/* Bytes at the start of this shape's workspace that must be zero before its
+ * first use: the counter region, or 0 where the shape's kernel counts no
+ * arrivals (any scratch will do) or takes no workspace.  No counterpart in
+ * the reference. */
+int wq_w4a16_workspace_zeroed(int64_t m, int64_t n, int64_t k, int64_t group_size, size_t* bytes);
 
 /* y fp16 [m, n] = x fp16 [m, k] . dequant(W)^T with fp32 accumulation.
  * Dispatches on m: MFMA GEMV for small m, LDS-staged MFMA GEMM for large m.

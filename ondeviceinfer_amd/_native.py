@@ -50,6 +50,7 @@ _SIGNATURES = {
     'wq_w4_decode': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P],
     'wq_w4_decode_rows': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P],
     'wq_w4a16_workspace_size': [_I64, _I64, _I64, _I64, _SIZE_P],
+    'wq_w4a16_workspace_zeroed': [_I64, _I64, _I64, _I64, _SIZE_P],
     'wq_w4a16_linear': [_P, _I64, _I64, _P, _P, _I64, _I64, _P, _P, ctypes.c_size_t, _P],
     'wq_w4a16_linear_noalloc': [_P, _I64, _I64, _P, _P, _I64, _I64, _P, _P],
     'wq_w4a16_epilogue_supported': [_I64, _I64, _I64, _I64, ctypes.c_int32],
@@ -287,6 +288,14 @@ def w4a16_workspace_size(m: int, n: int, k: int, group_size: int) -> int:
 
 
 @functools.lru_cache(maxsize=1024)   # a pure function of the shape, asked for on every call
+def w4a16_workspace_zeroed(m: int, n: int, k: int, group_size: int) -> int:
+    """Bytes at the start of this shape's workspace that must be zero before its first use."""
+    b = ctypes.c_size_t()
+    _call('wq_w4a16_workspace_zeroed', m, n, k, group_size, ctypes.byref(b))
+    return b.value
+
+
+@functools.lru_cache(maxsize=1024)   # a pure function of the shape, asked for on every call
 def w8a16_workspace_size(m: int, n: int, k: int) -> int:
     b = ctypes.c_size_t()
     _call('wq_w8a16_workspace_size', m, n, k, ctypes.byref(b))
@@ -318,11 +327,6 @@ def shared_workspace(device: torch.device, nbytes: int, layout: tuple) -> torch.
     return buf
 
 
-def _counts_arrivals(m: int, n: int, k: int) -> bool:
-    """The 5-to-64-row W4 shapes whose split needs zeroed counters (``mid_counts`` in ``csrc/wq_mid.hip``)."""
-    return 12 <= m <= 32 and n <= 18432 and k <= 8192 and k % 512 == 0
-
-
 def w4a16_linear(x: torch.Tensor, tiles: torch.Tensor, meta: torch.Tensor, n: int, group_size: int,
                  out: torch.Tensor | None = None, workspace: torch.Tensor | None = None) -> torch.Tensor:
     """``y[m, n] = x[m, k] . dequant(W)^T`` on the repacked weight."""
@@ -338,13 +342,12 @@ def w4a16_linear(x: torch.Tensor, tiles: torch.Tensor, meta: torch.Tensor, n: in
         if out.data_ptr() % 16:
             raise ValueError('out must be 16-byte aligned')
     if workspace is None and (nbytes := w4a16_workspace_size(m, n, k, group_size)):
-        if 4 < m <= 64 and not _counts_arrivals(m, n, k):
+        if not w4a16_workspace_zeroed(m, n, k, group_size):
             # Split partials only (no counters): any scratch of this call's own.
             workspace = x.new_empty(nbytes, dtype=torch.uint8)
         else:
-            # M > 4, counted splits and the deep-ring GEMM's: their counters
-            # sit in a fixed region at the front and are zero after every
-            # call, so all such shapes share one buffer.
+            # M > 4: the counters sit in a fixed region at the front and are
+            # zero after every call, so all such shapes share one buffer.
             workspace = shared_workspace(device, nbytes, ('w4a16', m, n, k, group_size) if m <= 4 else ('w4a16-split',))
     ws_ptr, ws_bytes = None, 0
     if workspace is not None:

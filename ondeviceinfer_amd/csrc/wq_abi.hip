@@ -22,6 +22,7 @@ int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uin
                   void* ws, size_t ws_bytes, hipStream_t st);
 size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
+bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k);
 int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
                      half_t* y, void* ws, size_t ws_bytes, hipStream_t s);
 int launch_w8_skinny(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
@@ -93,6 +94,16 @@ extern "C" int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t 
   if (mid > need) need = mid;
   if (gemm > need) need = gemm;
   *bytes = need;
+  return WQ_OK;
+}
+
+extern "C" int wq_w4a16_workspace_zeroed(int64_t m, int64_t n, int64_t k, int64_t group_size, size_t* bytes) {
+  size_t need = 0;
+  WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");
+  if (int st = wq_w4a16_workspace_size(m, n, k, group_size, &need)) return st;
+  // Of the kernels with a workspace only the one of 5 to 64 rows has plans without counters.
+  const bool counters = need > 0 && (w4_mid_workspace_bytes(m, n, k) == 0 || w4_mid_has_counters(m, n, k));
+  *bytes = counters ? kSplitCounterBytes : 0;
   return WQ_OK;
 }
 

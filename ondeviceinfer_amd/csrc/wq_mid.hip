@@ -456,6 +456,11 @@ int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* me
 
 }  // namespace
 
+// Whether a W4 shape's workspace carries arrival counters.
+bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k) {
+  return mid_ws_bytes(true, m, n, k) > 0 && mid_counts(true, m, n, k);
+}
+
 size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(true, m, n, k); }
 size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(false, m, n, k); }
 

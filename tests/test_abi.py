@@ -81,3 +81,21 @@ def test_prefill_k_split_workspace_follows_the_chain_length():
     assert _native.w4a16_workspace_size(700, 1000, 8320, 128) == counters + 352 * 4 * per_split_tile
     # M = 257: 64-row tiles (400 workgroups), no deep ring, no split
     assert _native.w4a16_workspace_size(257, 5120, 17408, 128) == 0
+
+
+def test_the_library_says_which_workspaces_start_zeroed():
+    """The bytes a caller zero-fills come from the library's own plan (no GPU
+    needed): the counter region where a kernel counts arrivals, else none, and
+    no copy of that rule in the Python binding."""
+    counters = 16384
+    for m, n, k, zeroed in ((1, 5120, 17408, counters),     # decode GEMV, k split
+                            (1, 5120, 5120, 0),             # decode GEMV, whole k: no workspace
+                            (24, 7168, 5120, counters),     # short chains of 12 to 32 rows: the last arriver sums
+                            (40, 7168, 5120, 0),            # a second launch sums
+                            (56, 5120, 17408, 0),
+                            (128, 5120, 17408, counters),   # deep-ring GEMM, k split
+                            (4096, 5120, 5120, 0)):
+        assert _native.w4a16_workspace_zeroed(m, n, k, 128) == zeroed, (m, n, k)
+        assert zeroed <= _native.w4a16_workspace_size(m, n, k, 128)
+    assert not hasattr(_native, '_counts_arrivals')
+    assert _status('wq_w4a16_workspace_zeroed', 1, 0, 128, 128, None) == _native.WQ_ERR_INVALID_ARGUMENT
