@@ -40,6 +40,12 @@ extern "C" {
 const char* wq_last_error(void);
 int wq_abi_version(void);
 
+/* A number for the graph capture `stream` takes part in (a different one for
+ * every capture), 0 when it is not being captured: a caller that keeps
+ * workspaces gives each captured graph its own, since the graph may later run
+ * beside anything.  No counterpart in the reference (it captures no graphs). */
+int wq_stream_capture_id(void* stream, uint64_t* id);
+
 /* ---------------------------------------------------------------- W4 (uint4, G-grouped) */
 
 /* Sizes of the gfx950 tile layout for an [n, k] pack-quantized weight.

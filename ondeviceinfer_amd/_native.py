@@ -49,6 +49,7 @@ _SIGNATURES = {
     'wq_w4_dequant': [_P, _P, _I64, _I64, _I64, _P, _P],
     'wq_w4_decode': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P],
     'wq_w4_decode_rows': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P],
+    'wq_stream_capture_id': [_P, ctypes.POINTER(ctypes.c_uint64)],
     'wq_w4a16_workspace_size': [_I64, _I64, _I64, _I64, _SIZE_P],
     'wq_w4a16_workspace_zeroed': [_I64, _I64, _I64, _I64, _SIZE_P],
     'wq_w4a16_linear': [_P, _I64, _I64, _P, _P, _I64, _I64, _P, _P, ctypes.c_size_t, _P],
@@ -303,27 +304,51 @@ def w8a16_workspace_size(m: int, n: int, k: int) -> int:
 
 
 _workspaces: dict = {}
+_captured: dict = {}          # capture id -> its workspaces, of the last few captures
+_captured_lock = threading.Lock()
+_MAX_CAPTURES = 4
 
 
-def shared_workspace(device: torch.device, nbytes: int, layout: tuple) -> torch.Tensor | None:
-    """Zero-filled workspace for callers that do not bring their own.
+def _capture_id(stream: int) -> int:
+    """The id of the capture ``stream`` takes part in, 0 outside one (the default stream is never captured)."""
+    if stream == 0:
+        return 0
+    b = ctypes.c_uint64()
+    _call('wq_stream_capture_id', stream, ctypes.byref(b))
+    return b.value
 
-    One buffer per (device, layout), never freed (a graph may have captured
-    its address).  ``layout`` names the operation and the shape that fix where
-    its counters and partials lie (e.g. ``('w4a16', n, k, group)``): the
-    kernels return the counters to zero after every call but leave partials
-    behind, so buffers are shared only between calls with the same layout,
-    and only when those calls are ordered on one stream (concurrent streams
-    need their own workspace: pass ``workspace=``).
+
+def shared_workspace(device: torch.device, nbytes: int, layout: tuple, zeroed: int | None = None) -> torch.Tensor | None:
+    """Workspace for callers that do not bring their own, its first ``zeroed``
+    bytes (all by default) zero before the first use.
+
+    One buffer per (device, stream, layout).  ``layout`` names the operation
+    and the shape that fix where its counters and partials lie (e.g.
+    ``('w4a16', n, k, group)``): the kernels return the counters to zero after
+    every call but leave partials behind, so calls share a buffer only if they
+    have the same layout and are ordered on one stream.  A call under capture
+    takes a buffer of that capture's own, cleared at the graph's start: the
+    graph may be replayed on any stream, beside eager calls and other graphs.
+    It comes from the graph's memory pool, so this module keeps it only while
+    the capture may still ask for it (the last ``_MAX_CAPTURES`` captures).
     """
     if nbytes <= 0:
         return None
-    key = (device.type, device.index) + tuple(layout)
-    buf = _workspaces.get(key)
+    stream = _stream(device)
+    key = (device.type, device.index, stream) + tuple(layout)
+    capture = _capture_id(stream)
+    if capture:
+        with _captured_lock:
+            while capture not in _captured and len(_captured) >= _MAX_CAPTURES:
+                del _captured[next(iter(_captured))]
+            buffers = _captured.setdefault(capture, {})
+    else:
+        buffers = _workspaces
+    buf = buffers.get(key)
     if buf is None or buf.numel() < nbytes:
-        buf = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-        _workspaces.setdefault(('retired',) + key, []).append(_workspaces.get(key))
-        _workspaces[key] = buf
+        buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        buf[:nbytes if zeroed is None else zeroed].zero_()
+        buffers[key] = buf
     return buf
 
 
@@ -342,13 +367,14 @@ def w4a16_linear(x: torch.Tensor, tiles: torch.Tensor, meta: torch.Tensor, n: in
         if out.data_ptr() % 16:
             raise ValueError('out must be 16-byte aligned')
     if workspace is None and (nbytes := w4a16_workspace_size(m, n, k, group_size)):
-        if not w4a16_workspace_zeroed(m, n, k, group_size):
+        zeroed = w4a16_workspace_zeroed(m, n, k, group_size)
+        if not zeroed:
             # Split partials only (no counters): any scratch of this call's own.
             workspace = x.new_empty(nbytes, dtype=torch.uint8)
         else:
             # M > 4: the counters sit in a fixed region at the front and are
             # zero after every call, so all such shapes share one buffer.
-            workspace = shared_workspace(device, nbytes, ('w4a16', m, n, k, group_size) if m <= 4 else ('w4a16-split',))
+            workspace = shared_workspace(device, nbytes, ('w4a16', m, n, k, group_size) if m <= 4 else ('w4a16-split',), zeroed)
     ws_ptr, ws_bytes = None, 0
     if workspace is not None:
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()

@@ -85,6 +85,19 @@ extern "C" const char* wq_last_error(void) { return g_last_error; }
 
 extern "C" int wq_abi_version(void) { return WQ_ABI_VERSION; }
 
+extern "C" int wq_stream_capture_id(void* stream, uint64_t* id) {
+  WQ_REQUIRE(id, WQ_ERR_INVALID_ARGUMENT, "null id output");
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  const hipError_t e = hipStreamGetCaptureInfo(as_stream(stream), &status, &capture);
+  if (e != hipSuccess) {
+    set_error("hipStreamGetCaptureInfo failed: %s", hipGetErrorString(e));
+    return WQ_ERR_HIP;
+  }
+  *id = status == hipStreamCaptureStatusNone ? 0 : (uint64_t)capture + 1;
+  return WQ_OK;
+}
+
 extern "C" int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t group_size, size_t* bytes) {
   if (int st = linear_shape_check(m, n, k)) return st;
   WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");

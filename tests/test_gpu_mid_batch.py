@@ -102,3 +102,44 @@ def test_mid_splits_run_on_two_streams_at_once_and_under_capture(gpu):
     p = layer['p._prepared']
     small = _native.w8a16_linear(xs[0], p.qweight, p.scale, workspace=torch.empty(16, dtype=torch.uint8, device=gpu))
     check_parity(host(small), host(refs[0]).astype(np.float32), 'skinny fallback')
+
+
+@pytest.mark.parametrize('m,n', [(24, 7168), (128, 1024)])
+def test_counted_splits_run_on_two_streams_at_once_and_under_capture(gpu, m, n):
+    """The W4 splits with arrival counters (24 rows, and the deep-ring GEMM at
+    128): calls on two streams that overlap, and replays of two captured graphs
+    beside each other and beside eager calls, equal the calls made one by one."""
+    weights, _ = synth.w4_case(n, 5120, 1, seed=n + m, name='p.weight')
+    layer = {key: dev(v, gpu) for key, v in weights.items()}
+    w = wq.CompressedLinearBackend('marlin')
+    w.prepare(layer, 'p.weight')
+    assert _native.w4a16_workspace_zeroed(m, n, 5120, 128) > 0
+    gen = torch.Generator(device=gpu).manual_seed(4)
+    xs = [torch.randn(m, 5120, generator=gen, device=gpu).half() for _ in range(2)]
+    refs = [w.linear(x, layer, 'p.weight').clone() for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    outs = [[], []]
+    for _ in range(8):
+        for s, x, o in zip(streams, xs, outs):
+            with torch.cuda.stream(s):
+                o.append(w.linear(x, layer, 'p.weight'))
+    torch.cuda.synchronize()
+    for o, ref in zip(outs, refs):
+        assert all(torch.equal(y, ref) for y in o)
+    graphs, ys = [], []
+    for x in xs:   # both on one capture stream, as torch captures by default
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=streams[0]):
+            ys.append([w.linear(x, layer, 'p.weight') for _ in range(3)])
+        graphs.append(g)
+    for _ in range(4):
+        for g, s, y in zip(graphs, streams, ys):
+            with torch.cuda.stream(s):
+                for t in y:
+                    t.zero_()
+                g.replay()
+        beside = [w.linear(x, layer, 'p.weight') for x in xs]   # on the default stream
+        torch.cuda.synchronize()
+        for y, b, ref in zip(ys, beside, refs):
+            assert torch.equal(b, ref) and all(torch.equal(t, ref) for t in y)

@@ -156,3 +156,34 @@ def test_greedy_generate_rejects_bad_inputs():
         greedy_generate(_CountingModel(), torch.tensor([1, 2]), max_new_tokens=2, cache=None)
     with pytest.raises(NotImplementedError, match='batch size 1'):
         greedy_generate(_CountingModel(), torch.tensor([[1], [2]]), max_new_tokens=2, cache=None)
+
+
+def test_workspaces_are_not_shared_between_streams_or_captures(monkeypatch):
+    """Calls that may overlap (other streams, captured graphs) get other
+    counters and partials; calls ordered on one stream share theirs."""
+    from ondeviceinfer_amd import _native
+    now = {'stream': 1, 'capture': 0}
+    monkeypatch.setattr(_native, '_stream', lambda device: now['stream'])
+    monkeypatch.setattr(_native, '_capture_id', lambda stream: now['capture'], raising=False)
+    monkeypatch.setattr(_native, '_workspaces', {})
+    monkeypatch.setattr(_native, '_captured', {}, raising=False)
+
+    def ask(stream, capture=0, nbytes=4096, layout=('w4a16-split',)):
+        now.update(stream=stream, capture=capture)
+        return _native.shared_workspace(torch.device('cpu'), nbytes, layout)
+
+    first = ask(1)
+    assert first.numel() == 4096 and not first.any()
+    assert ask(1) is first and ask(1, nbytes=64) is first
+    assert ask(2) is not first and ask(1, layout=('other',)) is not first
+    graph = ask(3, capture=7)
+    assert ask(3, capture=7) is graph
+    others = [ask(1), ask(3), ask(3, capture=8), ask(4, capture=7)]   # eager, another graph, a forked stream of this one
+    assert all(buf.data_ptr() != graph.data_ptr() for buf in others)
+    assert ask(1) is first and ask(1, nbytes=8192).numel() == 8192
+    for capture in range(10, 30):
+        ask(3, capture=capture)
+    assert len(_native._captured) <= _native._MAX_CAPTURES
+    assert ask(1, nbytes=0) is None
+    part = _native.shared_workspace(torch.device('cpu'), 4096, ('part',), zeroed=64)
+    assert part.numel() == 4096 and not part[:64].any()
