@@ -313,6 +313,20 @@ int wq_w8a8_linear_ws(const int8_t* qx, const float* x_scale, int64_t m, int64_t
                       int32_t tiled, const float* w_scale, int64_t n, const uint16_t* bias, uint16_t* y,
                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* ---------------------------------------------------------------- plans */
+
+#define WQ_FORMAT_W4A16 0
+#define WQ_FORMAT_W8A16 1 /* over INT8 tiles */
+#define WQ_FORMAT_W8A8 2  /* over INT8 tiles */
+
+/* The kernel and tile grid that a linear of this shape runs when it has its
+ * workspace, as a short text in `text` (cut to text_bytes): "gemv", "skinny",
+ * "mid PxS" (wave pairs x k splits), "deep NTxMTxS", "gemm NTxMT" (weight tiles
+ * per wave x 16-row chunks), "gemm 256x256".  epilogue: 0, or the mode of
+ * wq_w4a16_linear_epilogue / wq_w8a16_linear_epilogue.  k % 128 == 0.  For
+ * reports and tests; nothing is launched.  No counterpart in the reference. */
+int wq_linear_plan(int32_t format, int32_t epilogue, int64_t m, int64_t n, int64_t k, char* text, size_t text_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -50,6 +50,7 @@ _SIGNATURES = {
     'wq_w4_decode': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P],
     'wq_w4_decode_rows': [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P],
     'wq_stream_capture_id': [_P, ctypes.POINTER(ctypes.c_uint64)],
+    'wq_linear_plan': [ctypes.c_int32, ctypes.c_int32, _I64, _I64, _I64, ctypes.c_char_p, ctypes.c_size_t],
     'wq_w4a16_workspace_size': [_I64, _I64, _I64, _I64, _SIZE_P],
     'wq_w4a16_workspace_zeroed': [_I64, _I64, _I64, _I64, _SIZE_P],
     'wq_w4a16_linear': [_P, _I64, _I64, _P, _P, _I64, _I64, _P, _P, ctypes.c_size_t, _P],
@@ -180,6 +181,16 @@ def _check(t: torch.Tensor, dtype: torch.dtype, shape: tuple, name: str) -> None
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+_FORMATS = {'w4a16': 0, 'w8a16': 1, 'w8a8': 2}
+
+
+def linear_plan(fmt: str, m: int, n: int, k: int, epilogue: int = 0) -> str:
+    """The kernel and tile grid a linear of this shape runs (``wq_linear_plan``); INT8 weights as tiles."""
+    text = ctypes.create_string_buffer(32)
+    _call('wq_linear_plan', _FORMATS[fmt], epilogue, m, n, k, text, len(text))
+    return text.value.decode()
 
 
 # ----------------------------------------------------------------------------- W4

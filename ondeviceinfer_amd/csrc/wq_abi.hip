@@ -23,6 +23,9 @@ int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uin
 size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k);
+bool mid_plan_text(bool w4, int64_t m, int64_t n, int64_t k, char* text, size_t bytes);
+void gemm_plan_text(bool w4, int64_t m, int64_t n, int64_t k, int epilogue, char* text, size_t bytes);
+void w8a8_plan_text(int64_t m, int64_t n, int64_t k, char* text, size_t bytes);
 int launch_w4_skinny(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G,
                      half_t* y, void* ws, size_t ws_bytes, hipStream_t s);
 int launch_w8_skinny(const half_t* x, int M, int K, const int8_t* q, const half_t* scale, const half_t* bias, int N,
@@ -355,6 +358,32 @@ extern "C" int wq_w8a16_linear_tiled(const uint16_t* x, int64_t m, int64_t k, co
                                      void* workspace, size_t workspace_bytes, void* stream) {
   return w8a16_linear_impl(x, m, k, reinterpret_cast<const int8_t*>(tiles), scale, n, bias, y, workspace,
                            workspace_bytes, stream, 1);
+}
+
+extern "C" int wq_linear_plan(int32_t format, int32_t epilogue, int64_t m, int64_t n, int64_t k, char* text,
+                              size_t text_bytes) {
+  if (int st = linear_shape_check(m, n, k)) return st;
+  WQ_REQUIRE(format >= WQ_FORMAT_W4A16 && format <= WQ_FORMAT_W8A8 && text && text_bytes > 0 && m > 0 && k % 128 == 0,
+             WQ_ERR_INVALID_ARGUMENT, "need a format, m > 0, k %% 128 == 0 and a text buffer");
+  const bool w4 = format == WQ_FORMAT_W4A16;
+  if (epilogue != 0) {
+    const bool fits = format != WQ_FORMAT_W8A8 && (w4 ? w4_epilogue_fits(m, n, k, kW4BlockK, epilogue)
+                                                      : w8_epilogue_fits(m, n, k, epilogue));
+    WQ_REQUIRE(fits, WQ_ERR_UNSUPPORTED, "epilogue %d does not apply to this shape", (int)epilogue);
+    gemm_plan_text(w4, m, n, k, epilogue, text, text_bytes);
+  } else if (format == WQ_FORMAT_W8A8) {
+    w8a8_plan_text(m, n, k, text, text_bytes);
+  } else if (m <= 4) {
+    snprintf(text, text_bytes, "gemv");
+  } else if (mid_plan_text(w4, m, n, k, text, text_bytes)) {
+  } else if (w4 && w4_gemm_small_fits(m, n) && k <= kGemmMaxK) {
+    snprintf(text, text_bytes, "deep small");
+  } else if (m <= kSkinnyMaxM || k > kGemmMaxK) {
+    snprintf(text, text_bytes, "skinny");
+  } else {
+    gemm_plan_text(w4, m, n, k, 0, text, text_bytes);
+  }
+  return WQ_OK;
 }
 
 // ---------------------------------------------------------------------------

@@ -829,6 +829,19 @@ size_t w4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return deep_ws_bytes<1, 2>((int)M, (int)N, (int)K);
 }
 
+// The grid of a W4 (or INT8-tile) shape, given its workspace; epilogue 0 none,
+// 1 SiluPair, 2 Residual.
+void gemm_plan_text(bool w4, int64_t M, int64_t N, int64_t K, int epilogue, char* text, size_t bytes) {
+  const bool deep = gemm_takes_deep(M, N, true);
+  const int S = w4 && deep && epilogue == 0 ? deep_splits<1, 2>((int)M, (int)N, (int)K) : 1;
+  const Grid grid = S > 1 ? Grid::kDeep : gemm_grid(M, N, w4, epilogue == 0 && deep, epilogue == 1 ? 2 : 1);
+  for (const GridCost& g : kGridCosts)
+    if (g.grid == grid) {
+      if (grid == Grid::kDeep) snprintf(text, bytes, "deep %dx%dx%d", g.nt, g.mt, S);
+      else snprintf(text, bytes, "gemm %dx%d", g.nt, g.mt);
+    }
+}
+
 // Whether a W4 (or INT8-tile) shape has a fused epilogue: 0 where the deep
 // ring may serve it; mode 1 (SiluPair) also needs gate and up tiles within one
 // wave (N % 32 == 0, and 128-wide slices that fill the machine) and the up

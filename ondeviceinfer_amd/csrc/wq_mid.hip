@@ -456,6 +456,14 @@ int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* me
 
 }  // namespace
 
+// Writes the plan of a shape this file takes; false otherwise.
+bool mid_plan_text(bool w4, int64_t m, int64_t n, int64_t k, char* text, size_t bytes) {
+  if (!mid_takes(w4, m, n, k)) return false;
+  const MidSplit p = mid_plan(w4, m, n, k);
+  snprintf(text, bytes, "mid %dx%d", p.p, p.s);
+  return true;
+}
+
 // Whether a W4 shape's workspace carries arrival counters.
 bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k) {
   return mid_ws_bytes(true, m, n, k) > 0 && mid_counts(true, m, n, k);

@@ -825,10 +825,54 @@ __global__ __launch_bounds__(512, 2) void w8a8_gemm256_kernel(const int8_t* __re
 }
 
 constexpr int kW8A8GemvMaxM = 16;
-// Largest k of the W8A8 GEMM: its x and weight offsets are 32-bit (127 rows
-// of k bytes, 64 weight rows of k bytes); longer rows run the GEMV kernel 16
-// rows at a time.
+// Largest k of the W8A8 GEMM: a workgroup reads its 128 x rows and up to 64
+// weight rows of k bytes each through one buffer apiece, whose record count is
+// capped at 2^31 - 1 bytes; longer rows run the GEMV kernel 16 rows at a time.
 constexpr int64_t kW8A8GemmMaxK = 1 << 23;
+static_assert(128 * kW8A8GemmMaxK <= 0x7fffffff, "GEMM x and weight offsets must fit the 31-bit buffer range");
+// The 256 x 256 tiles read 256 rows of each, so their last block at k = 2^23
+// would end past that cap and come back as zeros: one 128-k block less.
+constexpr int64_t kBigMaxK = kW8A8GemmMaxK - kI8Blk;
+static_assert(kBigRows * kBigMaxK <= 0x7fffffff && kBigTiles * 16 * kBigMaxK <= 0x7fffffff,
+              "256 x 256 tile offsets must fit the 31-bit buffer range");
+
+// The kernel and grid of a shape.
+struct W8A8Route {
+  enum Kernel { kGemv, kGemm, kGemm256, kMid } kernel;
+  M8Plan plan;             // kMid
+  int nt, mt;              // kGemm: weight tiles per wave, 16-row chunks of x
+  int64_t mblocks, wgs256; // row blocks of kGemm, workgroups of kGemm256
+};
+
+W8A8Route w8a8_route(int64_t m, int64_t n, int64_t k, bool tiled, size_t ws_bytes) {
+  W8A8Route r{W8A8Route::kGemv, m8_plan(m, n, k), 0, 0, 0, 0};
+  if (r.plan.mc > 0 && (r.plan.m.s == 1 || ws_bytes >= r.plan.bytes())) {
+    r.kernel = W8A8Route::kMid;
+    return r;
+  }
+  if (m <= kW8A8GemvMaxM || k % kI8Blk != 0 || k > kW8A8GemmMaxK) return r;
+  // GEMM: 128-row x tiles for long batches, 32-row ones otherwise; four
+  // weight tiles per wave while that still leaves a full machine of
+  // workgroups, else one.  Over INT8 tiles, long batches take two tiles
+  // per wave while that gives 512 workgroups (M = 4096: 5120^2 197 ->
+  // 159 us, 5120->17408 513 -> 454 us, 17408->5120 466 -> 410 us).
+  const int64_t ntile = (n + 15) / 16;
+  const bool big_m = m >= 256;
+  r.kernel = W8A8Route::kGemm;
+  r.mblocks = big_m ? (m + 127) / 128 : (m + 31) / 32;
+  r.mt = big_m ? 8 : 2;
+  const bool two_tiles = tiled && big_m && (ntile + 7) / 8 * r.mblocks >= 512;
+  r.nt = two_tiles ? 2 : (ntile + 15) / 16 * r.mblocks >= 256 ? 4 : 1;
+  // 256 x 256 tiles where their rounds of 256 workgroups cost less: one costs
+  // 3.0 to 3.15 rounds of the 128 x 128 tiles (72-86 against 26-28 us at
+  // K = 5120, 63-67 against 20-22 us per 5120 of K = 17408).  Just past the
+  // line the other way: 5120^2 M = 4096 (2 against 5 rounds) 152 against 128 us,
+  // 5120->17408 M = 777 (2 against 4) 148 against 118.
+  r.wgs256 = (ntile + kBigTiles - 1) / kBigTiles * ((m + kBigRows - 1) / kBigRows);
+  if (two_tiles && k <= kBigMaxK && 31 * ((r.wgs256 + 255) / 256) < 10 * (((ntile + 7) / 8 * r.mblocks + 255) / 256))
+    r.kernel = W8A8Route::kGemm256;
+  return r;
+}
 
 }  // namespace
 }  // namespace wq
@@ -873,53 +917,39 @@ int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t 
   const half_t* b = reinterpret_cast<const half_t*>(bias);
   half_t* yy = reinterpret_cast<half_t*>(y);
   const int64_t nsteps = k / kI8Step, ntile = (n + 15) / 16;
-  const M8Plan plan = m8_plan(m, n, k);
-  if (plan.mc > 0 && (plan.m.s == 1 || (ws != nullptr && ws_bytes >= plan.bytes())))
-    return (plan.m.p == 4 ? launch_m8_plan<4> : launch_m8_plan<5>)(qx, x_scale, (int)m, (int)k, qweight, w_scale, b,
-                                                                  (int)n, yy, plan, ws, wl8, as_stream(stream));
-  if (m > kW8A8GemvMaxM && k % kI8Blk == 0 && k <= kW8A8GemmMaxK) {
-    // GEMM: 128-row x tiles for long batches, 32-row ones otherwise; four
-    // weight tiles per wave while that still leaves a full machine of
-    // workgroups, else one.  Over INT8 tiles, long batches take two tiles
-    // per wave while that gives 512 workgroups (M = 4096: 5120^2 197 ->
-    // 159 us, 5120->17408 513 -> 454 us, 17408->5120 466 -> 410 us).
-    const bool big_m = m >= 256;
-    const int64_t mblocks = big_m ? (m + 127) / 128 : (m + 31) / 32;
-    const bool two_tiles = tiled && big_m && (ntile + 7) / 8 * mblocks >= 512;
-    const int nt = two_tiles ? 2 : (ntile + 15) / 16 * mblocks >= 256 ? 4 : 1;
-    WQ_REQUIRE(mblocks <= 65535, WQ_ERR_UNSUPPORTED, "too many rows for the W8A8 GEMM grid");
-    // 256 x 256 tiles where their rounds of 256 workgroups cost less: one costs
-    // 3.0 to 3.15 rounds of the 128 x 128 tiles (72-86 against 26-28 us at
-    // K = 5120, 63-67 against 20-22 us per 5120 of K = 17408).  Just past the
-    // line the other way: 5120^2 M = 4096 (2 against 5 rounds) 152 against 128 us,
-    // 5120->17408 M = 777 (2 against 4) 148 against 118.
-    const int64_t big_wgs = (ntile + kBigTiles - 1) / kBigTiles * ((m + kBigRows - 1) / kBigRows);
-    if (two_tiles && 31 * ((big_wgs + 255) / 256) < 10 * (((ntile + 7) / 8 * mblocks + 255) / 256)) {
-      hipLaunchKernelGGL(w8a8_gemm256_kernel, dim3((unsigned)big_wgs), dim3(512), 0, as_stream(stream), qx, x_scale,
-                         (int)m, (int)k, qweight, w_scale, b, (int)n, yy);
-      return check_launch("w8a8_gemm256");
-    }
-    const dim3 grid((unsigned)((ntile + 4 * nt - 1) / (4 * nt)), (unsigned)mblocks);
+  const W8A8Route r = w8a8_route(m, n, k, tiled, ws != nullptr ? ws_bytes : 0);
+  if (r.kernel == W8A8Route::kMid)
+    return (r.plan.m.p == 4 ? launch_m8_plan<4> : launch_m8_plan<5>)(qx, x_scale, (int)m, (int)k, qweight, w_scale, b,
+                                                                    (int)n, yy, r.plan, ws, wl8, as_stream(stream));
+  if (r.kernel == W8A8Route::kGemm || r.kernel == W8A8Route::kGemm256)
+    WQ_REQUIRE(r.mblocks <= 65535, WQ_ERR_UNSUPPORTED, "too many rows for the W8A8 GEMM grid");
+  if (r.kernel == W8A8Route::kGemm256) {
+    hipLaunchKernelGGL(w8a8_gemm256_kernel, dim3((unsigned)r.wgs256), dim3(512), 0, as_stream(stream), qx, x_scale,
+                       (int)m, (int)k, qweight, w_scale, b, (int)n, yy);
+    return check_launch("w8a8_gemm256");
+  }
+  if (r.kernel == W8A8Route::kGemm) {
+    const dim3 grid((unsigned)((ntile + 4 * r.nt - 1) / (4 * r.nt)), (unsigned)r.mblocks);
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), qx, x_scale, (int)m, (int)k, qweight,
                          w_scale, b, (int)n, yy, wl8);
     };
-    if (big_m) {
-      if (nt == 4) launch(w8a8_gemm_kernel<4, 8>);
-      else if (nt == 2) launch(w8a8_gemm_kernel<2, 8>);
+    if (r.mt == 8) {
+      if (r.nt == 4) launch(w8a8_gemm_kernel<4, 8>);
+      else if (r.nt == 2) launch(w8a8_gemm_kernel<2, 8>);
       else launch(w8a8_gemm_kernel<1, 8>);
     } else {
-      if (nt == 4) launch(w8a8_gemm_kernel<4, 2>); else launch(w8a8_gemm_kernel<1, 2>);
+      if (r.nt == 4) launch(w8a8_gemm_kernel<4, 2>); else launch(w8a8_gemm_kernel<1, 2>);
     }
     return check_launch("w8a8_gemm");
   }
   // Decode kernel: about eight 64-k steps per wave (one round of loads).
   int ksw = (int)((nsteps + 7) / 8);
   ksw = ksw < 1 ? 1 : (ksw > 16 ? 16 : ksw);
-  for (int64_t r = 0; r < m; r += kW8A8GemvMaxM) {   // batches beyond 16 rows only when k % 128 != 0 or k > 2^23
-    const int64_t mr = m - r < kW8A8GemvMaxM ? m - r : kW8A8GemvMaxM;
-    hipLaunchKernelGGL(w8a8_gemv_kernel, dim3((unsigned)ntile), dim3(64 * ksw), 0, as_stream(stream), qx + r * k,
-                       x_scale + r, (int)mr, (int)k, qweight, w_scale, b, (int)n, yy + r * n, wl8);
+  for (int64_t m0 = 0; m0 < m; m0 += kW8A8GemvMaxM) {   // batches beyond 16 rows only when k % 128 != 0 or k > 2^23
+    const int64_t mr = m - m0 < kW8A8GemvMaxM ? m - m0 : kW8A8GemvMaxM;
+    hipLaunchKernelGGL(w8a8_gemv_kernel, dim3((unsigned)ntile), dim3(64 * ksw), 0, as_stream(stream), qx + m0 * k,
+                       x_scale + m0, (int)mr, (int)k, qweight, w_scale, b, (int)n, yy + m0 * n, wl8);
     const int rc = check_launch("w8a8_gemv");
     if (rc != WQ_OK) return rc;
   }
@@ -927,6 +957,18 @@ int w8a8_linear_impl(const int8_t* qx, const float* x_scale, int64_t m, int64_t 
 }
 
 }  // namespace
+
+namespace wq {
+void w8a8_plan_text(int64_t m, int64_t n, int64_t k, char* text, size_t bytes) {
+  const W8A8Route r = w8a8_route(m, n, k, true, SIZE_MAX);
+  switch (r.kernel) {
+    case W8A8Route::kMid: snprintf(text, bytes, "mid %dx%d", r.plan.m.p, r.plan.m.s); break;
+    case W8A8Route::kGemm256: snprintf(text, bytes, "gemm 256x256"); break;
+    case W8A8Route::kGemm: snprintf(text, bytes, "gemm %dx%d", r.nt, r.mt); break;
+    default: snprintf(text, bytes, "gemv"); break;
+  }
+}
+}  // namespace wq
 
 extern "C" int wq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k, size_t* bytes) {
   WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");

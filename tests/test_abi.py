@@ -99,3 +99,16 @@ def test_the_library_says_which_workspaces_start_zeroed():
         assert zeroed <= _native.w4a16_workspace_size(m, n, k, 128)
     assert not hasattr(_native, '_counts_arrivals')
     assert _status('wq_w4a16_workspace_zeroed', 1, 0, 128, 128, None) == _native.WQ_ERR_INVALID_ARGUMENT
+
+
+def test_w8a8_256_tiles_stop_where_their_reads_leave_the_buffer_range():
+    """256 rows of k bytes end at 2^31 for k = 2^23, one byte past the 31-bit
+    record count of a buffer (the last reads would come back as zeros): that k
+    takes the 128-row tiles, one 128-k block less the 256 x 256 ones."""
+    m = n = 3584
+    assert _native.linear_plan('w8a8', m, n, (1 << 23) - 128) == 'gemm 256x256'
+    assert _native.linear_plan('w8a8', m, n, 1 << 23) == 'gemm 2x8'
+    assert _native.linear_plan('w8a8', m, n, (1 << 23) + 128) == 'gemv'
+    assert _native.linear_plan('w8a8', 2048, 7168, 5120) == 'gemm 256x256'
+    with pytest.raises(ValueError):
+        _native.linear_plan('w8a8', 2048, 7168, 5100)
