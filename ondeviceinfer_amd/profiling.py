@@ -13,7 +13,17 @@ import torch
 _ENABLED = os.environ.get('ONDEVICEINFER_NVTX', '0') == '1'
 
 
-_OFF = contextlib.nullcontext()
+class _Off(contextlib.ContextDecorator):
+    """Does nothing; re-entrant, and a decorator like the range it stands for."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return None
+
+
+_OFF = _Off()
 
 
 @contextlib.contextmanager

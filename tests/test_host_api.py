@@ -187,3 +187,20 @@ def test_workspaces_are_not_shared_between_streams_or_captures(monkeypatch):
     assert ask(1, nbytes=0) is None
     part = _native.shared_workspace(torch.device('cpu'), 4096, ('part',), zeroed=64)
     assert part.numel() == 4096 and not part[:64].any()
+
+
+@pytest.mark.parametrize('enabled', [False, True])
+def test_nvtx_range_is_a_context_and_a_decorator(monkeypatch, enabled):
+    from ondeviceinfer_amd import profiling
+    monkeypatch.setattr(profiling, '_ENABLED', enabled)
+    with profiling.nvtx_range('outer') as value, profiling.nvtx_range('inner'):
+        assert value is None
+
+    @profiling.nvtx_range('call')
+    def double(x):
+        return 2 * x
+
+    assert double(3) == 6 and double(4) == 8
+    with pytest.raises(KeyError):
+        with profiling.nvtx_range('raises'):
+            raise KeyError('x')
