@@ -381,27 +381,6 @@ MidSplit mid_plan(bool w4, int64_t M, int64_t N, int64_t K) {
                    2 * mc * 16 * 256, 1, mc);
 }
 
-// The shapes this file takes, from both sides' measurements.  W4: from 12
-// rows on, and from 5 rows where the k chain is long or N is wide (17408->5120
-// M = 8 20.5 -> 16.5 us, 5120->17408 22.5 -> 18.5; fused QKV M = 8 8.2 against
-// 10.2 the other way); from 2048 tiles on only chains of at least 32 blocks
-// (shorter ones keep the skinny kernels and, above 16 rows, the deep-ring
-// GEMM, whose rows equal those of longer batches bit for bit).  At 33 to 35
-// rows short chains stay on the skinny kernels: their workspace query answers
-// 0 bytes just past 32 rows, which callers may rely on.  INT8: from 33 rows on,
-// and weights of at least 10000 tile blocks (20 MB; 5120->1024 M = 8 6.6 us
-// against 8.6, 2048->4040 5.2 against 8.2 the other way) or, from 17 rows,
-// chains of at least 32 blocks (5120->1024 M = 24 12.9 -> 9.3 us, 2048->4040
-// 8.2 against 9.1).
-bool mid_takes(bool w4, int64_t M, int64_t N, int64_t K) {
-  if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return false;
-  const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
-  if (!w4) return M > 32 || ntile * nblk >= 10000 || (M > 16 && nblk >= 32);
-  if (ntile >= 2048) return nblk >= 32;
-  if (M < 12) return nblk >= 64 || ntile >= 1024;
-  return nblk >= 64 || M < 33 || M > 35;
-}
-
 // Whether the last arriver sums (W4, mid_kernel's ws_cnt): 12 to 32 rows on up
 // to 1152 tiles and k chains of 4 to 64 blocks (a multiple of four), the
 // shapes whose workspace carried zeroed counters before this kernel.
@@ -410,9 +389,47 @@ bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
   return w4 && M >= 12 && M <= 32 && (N + 15) / 16 <= 1152 && nblk <= 64 && nblk % 4 == 0;
 }
 
-size_t mid_ws_bytes(bool w4, int64_t M, int64_t N, int64_t K) {
-  if (!mid_takes(w4, M, N, K)) return 0;
-  return mid_partial_bytes(mid_plan(w4, M, N, K), 1, (int)((M + 15) / 16));
+// The shapes this file takes: those whose plan is estimated below the skinny
+// kernels' time.  W4: the skinny kernels take rounds of 256 workgroups (two
+// tiles a wave, four from 1024 tiles on) whose time is a chain of k blocks,
+//   rounds x blocks x (0.034 + 0.108 per 16-row chunk + 0.006 per row) us
+// and about twice that at four tiles; the constants are fitted so that the
+// measured faster side wins, over k = 512..17408, N = 512..34816, M = 5..64
+// (2700 points: the chosen side is 0.2 % off the faster one on average, 18 %
+// at most; one threshold per row range was 7.9 % off, and 1.3 to 2 times on
+// short narrow chains and at 33 to 35 rows).  Both sides, skinny against this
+// file, us: 512->512 M = 16 3.3 / 4.9, 1024->2048 M = 36 5.8 / 8.0, 2048->6144
+// M = 33 8.4 / 9.7; 2048->12288 M = 33 14.7 / 11.9, 5120->1024 M = 33 15.2 /
+// 8.9, 5120->7168 M = 8 / 12 / 24 9.4 / 10.3 / 14.5 against 10.0 / 10.1 / 11.3,
+// 5120->17408 M = 34 36.5 / 23.9, 17408->5120 M = 8 20.4 / 15.8.
+// From 2048 tiles on and 17 rows the other side is the deep-ring GEMM: only
+// chains of at least 32 blocks leave it (5120->34816 M = 24 / 56 37 / 50 ->
+// 31 / 41 us).  Shorter ones would gain as well (2048->34816 M = 24 / 48 17.0 /
+// 23.1 against 15.0 / 16.5) but keep the deep ring, whose rows equal those of a
+// longer call bit for bit; the long chains' rows no longer do.
+// INT8: from 33 rows on, and weights of at least 10000 tile blocks (20 MB;
+// 5120->1024 M = 8 6.6 us against 8.6, 2048->4040 5.2 against 8.2 the other
+// way) or, from 17 rows, chains of at least 32 blocks (5120->1024 M = 24 12.9
+// -> 9.3 us, 2048->4040 8.2 against 9.1).
+// Returns the plan, or one without groups for the other shapes.
+MidSplit mid_route(bool w4, int64_t M, int64_t N, int64_t K) {
+  constexpr MidSplit kNone{0, 0, 0};
+  if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return kNone;
+  const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
+  if (!w4) return M > 32 || ntile * nblk >= 10000 || (M > 16 && nblk >= 32) ? mid_plan(w4, M, N, K) : kNone;
+  if (ntile >= 2048 && M > 16) return nblk >= 32 ? mid_plan(w4, M, N, K) : kNone;
+  const double mc = (double)((M + 15) / 16);
+  const bool four = ntile >= 1024;   // tiles per wave of the skinny kernels (pick_skinny)
+  const int64_t rounds = ((ntile + (four ? 3 : 1)) / (four ? 4 : 2) + 255) / 256;
+  double skinny = (double)(rounds * nblk) * (0.034 + 0.108 * mc + 0.006 * (double)M + (four ? 0.038 + 0.098 * mc : 0.0)) - 2.4;
+  if (skinny <= -0.3) return kNone;   // whatever the plan
+  const MidSplit p = mid_plan(w4, M, N, K);
+  if (p.s > 1) skinny -= mid_counts(w4, M, N, K) ? -0.3 : 1.3;   // the partial sums, in the same launch or a second
+  return p.us < skinny ? p : kNone;
+}
+
+size_t mid_route_bytes(const MidSplit& p, int64_t M) {
+  return p.groups == 0 ? 0 : mid_partial_bytes(p, 1, (int)((M + 15) / 16));
 }
 
 template <MFmt F, int P, int MC, int D, int MINW>
@@ -445,11 +462,10 @@ int launch_mid_p(const half_t* x, int M, int K, const void* w, const void* meta,
 template <MFmt F>
 int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* bias,
                     half_t* y, void* ws, size_t ws_bytes, int tiled, hipStream_t st) {
-  constexpr bool w4 = F == MFmt::W4;
-  if (!mid_takes(w4, M, N, K)) return -1;
-  const size_t need = mid_ws_bytes(w4, M, N, K);
+  const MidSplit m = mid_route(F == MFmt::W4, M, N, K);
+  if (m.groups == 0) return -1;
+  const size_t need = mid_route_bytes(m, M);
   if (need > 0 && (ws == nullptr || ws_bytes < need)) return -1;
-  const MidSplit m = mid_plan(w4, M, N, K);
   return m.p == 4 ? launch_mid_p<F, 4>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st)
                   : launch_mid_p<F, 5>(x, M, K, w, meta, N, bpg, bias, y, ws, m, tiled, st);
 }
@@ -458,19 +474,18 @@ int launch_mid_auto(const half_t* x, int M, int K, const void* w, const void* me
 
 // Writes the plan of a shape this file takes; false otherwise.
 bool mid_plan_text(bool w4, int64_t m, int64_t n, int64_t k, char* text, size_t bytes) {
-  if (!mid_takes(w4, m, n, k)) return false;
-  const MidSplit p = mid_plan(w4, m, n, k);
-  snprintf(text, bytes, "mid %dx%d", p.p, p.s);
-  return true;
+  const MidSplit p = mid_route(w4, m, n, k);
+  if (p.groups > 0) snprintf(text, bytes, "mid %dx%d", p.p, p.s);
+  return p.groups > 0;
 }
 
 // Whether a W4 shape's workspace carries arrival counters.
 bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k) {
-  return mid_ws_bytes(true, m, n, k) > 0 && mid_counts(true, m, n, k);
+  return mid_route(true, m, n, k).s > 1 && mid_counts(true, m, n, k);
 }
 
-size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(true, m, n, k); }
-size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_ws_bytes(false, m, n, k); }
+size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_route_bytes(mid_route(true, m, n, k), m); }
+size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k) { return mid_route_bytes(mid_route(false, m, n, k), m); }
 
 int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
                   void* ws, size_t ws_bytes, hipStream_t st) {

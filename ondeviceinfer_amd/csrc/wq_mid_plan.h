@@ -8,10 +8,14 @@ namespace wq {
 
 constexpr int kMidTilesPerWave = 2;   // 16-row tiles per wave
 
-// Tile groups of 2 P tiles (P wave pairs per workgroup), S k splits.
+// Tile groups of 2 P tiles (P wave pairs per workgroup), S k splits; us is
+// mid_split's estimate, which leaves out a constant of about 4 us (launch,
+// first loads, parity sum; over 140 shapes x 20 row counts measured times lie
+// within 12 % of estimate + 4.2).
 struct MidSplit {
   int p, s;
   int64_t groups;
+  double us = 0;
 };
 
 inline int64_t mid_groups(int64_t ntile, int p) {
@@ -63,14 +67,16 @@ inline MidSplit mid_split(int64_t ntile, int64_t nst, double w_tile, double x_st
       if (us < best_us) {
         best_us = us;
         best = m;
+        best.us = us;
       }
     }
     if (nst * 3 < 5) {   // a single stage: the loop above has no S to try
       m.s = 1;
-      const double us = (double)((m.groups * nz + 255) / 256) * (p * kMidTilesPerWave * w_tile + x_stage);
+      const double us = (double)((m.groups * nz + 255) / 256) * (p * kMidTilesPerWave * w_tile + x_stage) / 35e3;
       if (p == 4 || us < best_us) {
         best_us = us;
         best = m;
+        best.us = us;
       }
     }
   }

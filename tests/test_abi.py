@@ -112,3 +112,22 @@ def test_w8a8_256_tiles_stop_where_their_reads_leave_the_buffer_range():
     assert _native.linear_plan('w8a8', 2048, 7168, 5120) == 'gemm 256x256'
     with pytest.raises(ValueError):
         _native.linear_plan('w8a8', 2048, 7168, 5100)
+
+
+def test_w4_rows_5_to_64_take_the_kernel_estimated_faster():
+    """Short narrow chains stay on the skinny kernels at every row count (the
+    shared-activation kernel takes 1.3 to 2 times as long there), long or wide
+    ones leave them, and no row count between two others makes an exception."""
+    plan = lambda m, n, k: _native.linear_plan('w4a16', m, n, k).split()[0]
+    rows = range(5, 65)
+    for n, k in ((512, 512), (2048, 1024), (6144, 512), (1024, 1024), (4040, 1024)):
+        assert {plan(m, n, k) for m in rows} == {'skinny'}, (n, k)
+    for n, k in ((5120, 17408), (17408, 5120), (12288, 12288), (1024, 12288)):
+        assert {plan(m, n, k) for m in rows} == {'mid'}, (n, k)
+    for n, k in ((1024, 5120), (5120, 5120), (7168, 5120), (6144, 2048), (12288, 2048)):
+        taken = [plan(m, n, k) == 'mid' for m in rows if not 12 <= m <= 32]   # 12..32: other partial sums
+        assert taken == sorted(taken), (n, k)
+    for m in (33, 34, 35):
+        for n, k in ((1024, 5120), (5120, 5120), (7168, 5120), (17408, 5120), (12288, 2048)):
+            assert plan(m, n, k) == 'mid', (m, n, k)
+    assert plan(33, 34816, 1024) == 'deep' and plan(33, 34816, 5120) == 'mid'

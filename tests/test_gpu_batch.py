@@ -71,7 +71,8 @@ def test_batch_plans_use_the_workspace_and_fall_back_without_it(gpu):
     assert _native.w4a16_workspace_size(m, n, k, 128) > 0
     assert _native.w4a16_workspace_size(m, 17408, k, 128) > 0    # gate / up (1088 tiles)
     assert _native.w4a16_workspace_size(m, 34816, k, 128) == 0   # the fused gate_up keeps the ring kernels
-    assert _native.w4a16_workspace_size(33, n, k, 128) == 0      # beyond M = 32
+    assert _native.w4a16_workspace_size(33, n, k, 128) > 0       # beyond M = 32: partials without counters
+    assert _native.w4a16_workspace_zeroed(33, n, k, 128) == 0
     assert _native.w4a16_workspace_size(11, n, k, 128) == 0      # below M = 12 (skinny kernels)
     assert _native.w4a16_workspace_size(12, n, k, 128) > 0
     _, layer, name, weights, x = prepared(n, k, m, 7, gpu)

@@ -13,7 +13,7 @@ from ondeviceinfer_amd.weight_quantization import backend as wq
 
 pytestmark = pytest.mark.gpu
 
-ROWS = (5, 16, 17, 33, 36, 48, 49, 64)   # both ends of the 16-row chunks (33..35: skinny on short chains)
+ROWS = (5, 16, 17, 33, 36, 48, 49, 64)   # both ends of the 16-row chunks
 
 
 def dev(a, device):
@@ -143,3 +143,25 @@ def test_counted_splits_run_on_two_streams_at_once_and_under_capture(gpu, m, n):
         torch.cuda.synchronize()
         for y, b, ref in zip(ys, beside, refs):
             assert torch.equal(b, ref) and all(torch.equal(t, ref) for t in y)
+
+
+# Shapes the shared-activation kernel does take: an odd block count over a
+# partial last tile group (the last stage half empty) in many splits; groups of
+# 384 = three blocks (stages start inside a group); ten-tile groups in two
+# splits, and unsplit over a partial last group; 33 to 35 rows.
+@pytest.mark.parametrize('m,n,k,g', [(5, 1000, 12416, 128), (17, 1000, 12416, 128), (12, 7168, 5120, 128),
+                                     (33, 1000, 8448, 384), (34, 7168, 5120, 128), (35, 1024, 5120, 256),
+                                     (35, 17408, 2560, 128), (49, 17400, 2432, 128), (64, 5112, 4992, 128),
+                                     (8, 25608, 4224, 128), (16, 25600, 3968, 128)])
+def test_w4_mid_shapes_match_oracle(gpu, m, n, k, g):
+    plan = _native.linear_plan('w4a16', m, n, k)
+    print(f'[mid] m={m} n={n} k={k} g={g}: {plan}', flush=True)
+    assert plan.startswith('mid')
+    weights, x = synth.w4_case(n, k, m, seed=n % 89 + k, group_size=g, name='p.weight')
+    layer = {key: dev(v, gpu) for key, v in weights.items()}
+    backend = wq.CompressedLinearBackend('marlin', group_size=g)
+    backend.prepare(layer, 'p.weight')
+    w32 = qdq.decode_weight(weights, 'p.weight', group_size=g).astype(np.float32)
+    y = backend.linear(dev(x, gpu), layer, 'p.weight')
+    check_parity(host(y), (x.astype(np.float32) @ w32.T).astype(np.float16), plan)
+    assert torch.equal(backend.linear(dev(x, gpu), layer, 'p.weight'), y)
