@@ -321,7 +321,7 @@ int wq_w8a8_linear_ws(const int8_t* qx, const float* x_scale, int64_t m, int64_t
 
 /* The kernel and tile grid that a linear of this shape runs when it has its
  * workspace, as a short text in `text` (cut to text_bytes): "gemv", "skinny",
- * "mid PxS" (wave pairs x k splits), "deep NTxMTxS", "gemm NTxMT" (weight tiles
+ * "mid PxS" (wave pairs x k splits), "batch RxS" (k blocks x splits), "deep NTxMTxS", "gemm NTxMT" (weight tiles
  * per wave x 16-row chunks), "gemm 256x256".  epilogue: 0, or the mode of
  * wq_w4a16_linear_epilogue / wq_w8a16_linear_epilogue.  k % 128 == 0.  For
  * reports and tests; nothing is launched.  No counterpart in the reference. */

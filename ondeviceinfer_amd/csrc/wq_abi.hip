@@ -1,5 +1,6 @@
 // C-ABI entry points for the linear kernels, plus the error channel.
 #include "wq_common.h"
+#include "wq_mid_plan.h"
 #include "wq_status.h"
 
 #include <mutex>
@@ -20,6 +21,9 @@ void set_error(const char* fmt, ...) {
 size_t gemv_workspace_bytes(bool w4, int64_t m, int64_t n, int64_t k);
 int launch_w4_mid(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
                   void* ws, size_t ws_bytes, hipStream_t st);
+int launch_w4_batch(const half_t* x, int M, int K, const uint4_t* tiles, const uint8_t* meta, int N, int G, half_t* y,
+                    void* ws, size_t ws_bytes, hipStream_t st);
+size_t w4_batch_workspace_bytes(int64_t m, int64_t n, int64_t k);
 size_t w4_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 size_t w8_mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 bool w4_mid_has_counters(int64_t m, int64_t n, int64_t k);
@@ -105,9 +109,10 @@ extern "C" int wq_w4a16_workspace_size(int64_t m, int64_t n, int64_t k, int64_t 
   if (int st = linear_shape_check(m, n, k)) return st;
   WQ_REQUIRE(bytes, WQ_ERR_INVALID_ARGUMENT, "null size output");
   size_t need = gemv_workspace_bytes(true, m, n, k);
-  const size_t mid = w4_mid_workspace_bytes(m, n, k);
+  const size_t mid = w4_mid_workspace_bytes(m, n, k), batch = w4_batch_workspace_bytes(m, n, k);
   const size_t gemm = m > kSkinnyMaxM && k <= kGemmMaxK ? w4_gemm_workspace_bytes(m, n, k) : 0;
   if (mid > need) need = mid;
+  if (batch > need) need = batch;
   if (gemm > need) need = gemm;
   *bytes = need;
   return WQ_OK;
@@ -152,6 +157,10 @@ extern "C" int wq_w4a16_linear(const uint16_t* x, int64_t m, int64_t k, const vo
                                  reinterpret_cast<const uint8_t*>(meta), (int)n, (int)group_size, yh, workspace,
                                  workspace_bytes, as_stream(stream));
     if (rc != -1) return rc;
+    const int rb = launch_w4_batch(xh, (int)m, (int)k, reinterpret_cast<const uint4_t*>(tiles),
+                                   reinterpret_cast<const uint8_t*>(meta), (int)n, (int)group_size, yh, workspace,
+                                   workspace_bytes, as_stream(stream));
+    if (rb != -1) return rb;
   }
   if (w4_gemm_small_fits(m, n) && k <= kGemmMaxK)
     return launch_w4_gemm_small(xh, (int)m, (int)k, reinterpret_cast<const uint4_t*>(tiles),
@@ -376,6 +385,8 @@ extern "C" int wq_linear_plan(int32_t format, int32_t epilogue, int64_t m, int64
   } else if (m <= 4) {
     snprintf(text, text_bytes, "gemv");
   } else if (mid_plan_text(w4, m, n, k, text, text_bytes)) {
+  } else if (const W4BatchPlan b = w4 ? w4_batch_route(m, n, k) : W4BatchPlan{}; b.r > 0) {
+    snprintf(text, text_bytes, "batch %dx%d", b.r, b.s);
   } else if (w4 && w4_gemm_small_fits(m, n) && k <= kGemmMaxK) {
     snprintf(text, text_bytes, "deep small");
   } else if (m <= kSkinnyMaxM || k > kGemmMaxK) {

@@ -411,8 +411,10 @@ bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
 // 5120->1024 M = 8 6.6 us against 8.6, 2048->4040 5.2 against 8.2 the other
 // way) or, from 17 rows, chains of at least 32 blocks (5120->1024 M = 24 12.9
 // -> 9.3 us, 2048->4040 8.2 against 9.1).
-// Returns the plan, or one without groups for the other shapes.
-MidSplit mid_route(bool w4, int64_t M, int64_t N, int64_t K) {
+// wq_batch.hip's shapes come off both (w4_batch_plan).
+// Returns the plan, or one without groups for the other shapes; W4 only:
+// best_us the estimated time of the faster of the two sides.
+MidSplit mid_route(bool w4, int64_t M, int64_t N, int64_t K, double* best_us = nullptr) {
   constexpr MidSplit kNone{0, 0, 0};
   if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return kNone;
   const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
@@ -421,12 +423,29 @@ MidSplit mid_route(bool w4, int64_t M, int64_t N, int64_t K) {
   const double mc = (double)((M + 15) / 16);
   const bool four = ntile >= 1024;   // tiles per wave of the skinny kernels (pick_skinny)
   const int64_t rounds = ((ntile + (four ? 3 : 1)) / (four ? 4 : 2) + 255) / 256;
-  double skinny = (double)(rounds * nblk) * (0.034 + 0.108 * mc + 0.006 * (double)M + (four ? 0.038 + 0.098 * mc : 0.0)) - 2.4;
+  const double skinny = (double)(rounds * nblk) * (0.034 + 0.108 * mc + 0.006 * (double)M + (four ? 0.038 + 0.098 * mc : 0.0)) - 2.4;
+  if (best_us) *best_us = 4.2 + skinny;
   if (skinny <= -0.3) return kNone;   // whatever the plan
   const MidSplit p = mid_plan(w4, M, N, K);
-  if (p.s > 1) skinny -= mid_counts(w4, M, N, K) ? -0.3 : 1.3;   // the partial sums, in the same launch or a second
-  return p.us < skinny ? p : kNone;
+  const double split = p.s <= 1 ? 0.0 : mid_counts(w4, M, N, K) ? -0.3 : 1.3;   // partial sums, in the same launch or a second
+  if (best_us) {
+    const double mid = p.us + (p.s > 1 ? 0.9 : 0.0);
+    *best_us = 4.2 + (mid < skinny ? mid : skinny);
+  }
+  return p.us < skinny - split && (best_us || w4_batch_route(M, N, K).r == 0) ? p : kNone;
 }
+
+}  // namespace
+
+W4BatchPlan w4_batch_route(int64_t m, int64_t n, int64_t k) {
+  const W4BatchPlan p = w4_batch_plan(m, n, k);
+  if (p.r == 0) return {};
+  double other = 0;
+  mid_route(true, m, n, k, &other);
+  return p.us < other + 0.7 ? p : W4BatchPlan{};   // 0.7: where the fitted estimates cross on measured times
+}
+
+namespace {
 
 size_t mid_route_bytes(const MidSplit& p, int64_t M) {
   return p.groups == 0 ? 0 : mid_partial_bytes(p, 1, (int)((M + 15) / 16));

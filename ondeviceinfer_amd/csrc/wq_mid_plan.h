@@ -83,4 +83,30 @@ inline MidSplit mid_split(int64_t ntile, int64_t nst, double w_tile, double x_st
   return best;
 }
 
+// wq_batch.hip's plan: R blocks per workgroup in flight, S splits, groups of
+// eight tiles; r == 0 for the shapes it has none for.  us is its time, fitted to
+// 256 shapes of 12 to 32 rows (10 % at most off): a chain of R blocks per 16-row
+// chunk, the partial sums of two splits, and the tiles.
+constexpr int64_t kW4BatchMaxTiles = 1152;
+struct W4BatchPlan {
+  int mc, r, s, groups;
+  double us;
+};
+inline W4BatchPlan w4_batch_plan(int64_t m, int64_t n, int64_t k) {
+  const int64_t ntile = (n + 15) / 16, nblk = k / kW4BlockK;
+  if (m < 12 || m > 32 || k % kW4BlockK != 0 || ntile <= 512 || ntile > kW4BatchMaxTiles || nblk > 20) return {};
+  const int mc = (int)((m + 15) / 16), groups = (int)((ntile + 7) / 8);
+  for (int r : {10, 8, 5, 4}) {
+    const int s = (int)(nblk / r);
+    if (nblk % r != 0 || r * mc * 4 % 8 != 0) continue;   // the x copies split evenly over eight waves
+    if (s > 2 || s * groups > 256) return {};             // more than one round of workgroups
+    return {mc, r, s, groups,
+            1.6 + 0.5 * mc + (0.40 + 0.07 * mc) * r + (s > 1 ? 1.3 + 0.5 * mc : 0.0) + 0.5 * (double)ntile / 1152};
+  }
+  return {};
+}
+
+// The plan where that kernel is estimated the fastest, else r == 0 (wq_mid.hip).
+W4BatchPlan w4_batch_route(int64_t m, int64_t n, int64_t k);
+
 }  // namespace wq

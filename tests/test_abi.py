@@ -127,6 +127,7 @@ def test_w4_rows_5_to_64_take_the_kernel_estimated_faster():
     for n, k in ((1024, 5120), (5120, 5120), (7168, 5120), (6144, 2048), (12288, 2048)):
         taken = [plan(m, n, k) == 'mid' for m in rows if not 12 <= m <= 32]   # 12..32: other partial sums
         assert taken == sorted(taken), (n, k)
+    assert {plan(m, 17408, 1024) for m in range(12, 33)} == {plan(m, 12288, 2048) for m in range(12, 33)} == {'batch'}
     for m in (33, 34, 35):
         for n, k in ((1024, 5120), (5120, 5120), (7168, 5120), (17408, 5120), (12288, 2048)):
             assert plan(m, n, k) == 'mid', (m, n, k)

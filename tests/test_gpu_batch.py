@@ -1,6 +1,7 @@
-"""GPU parity of the small-batch W4A16 kernel (wq_mid.hip: 12 <= M <= 32 on
-narrow N, activations shared in LDS, k split over workgroups) against the
-CPU oracle, through the backend and the C ABI.
+"""GPU parity of the small-batch W4A16 kernels (12 <= M <= 32 on up to 1152
+tiles, activations shared in LDS, k split over workgroups: wq_mid.hip, and
+wq_batch.hip on short chains) against the CPU oracle, through the backend and
+the C ABI.
 
 Bars as in test_gpu_parity.py (``oracle.qdq.parity_ok``).  The k split
 changes the fp32 summation order relative to the skinny kernels, so the two
@@ -61,6 +62,26 @@ def test_batch_kernel_matches_oracle(gpu, n, k, g, sym):
         assert y.shape == (m, n)
         expected = (x[:m].astype(np.float32) @ w32.T).astype(np.float16)
         check_parity(y, expected, f'batch n={n} k={k} g={g} m={m}')
+
+
+# The shapes wq_batch.hip takes: every depth in flight (4, 5, 8, 10 blocks), one and two
+# 16-row chunks, partial last tile groups, two splits, groups of one to four blocks.
+@pytest.mark.parametrize('m,n,k,g', [(16, 17400, 512, 128), (32, 9224, 512, 512), (17, 17400, 640, 128),
+                                     (12, 16520, 1024, 256), (32, 17408, 1024, 128), (24, 18432, 1280, 256),
+                                     (12, 12296, 2048, 512), (32, 11272, 2048, 128), (16, 9224, 2560, 128)])
+def test_short_chain_kernel_matches_oracle(gpu, m, n, k, g):
+    plan = _native.linear_plan('w4a16', m, n, k)
+    print(f'[batch] m={m} n={n} k={k} g={g}: {plan}', flush=True)
+    assert plan.startswith('batch')
+    backend, layer, name, weights, x = prepared(n, k, m, 50 + n % 13, gpu, g)
+    w32 = qdq.decode_weight(weights, name, group_size=g).astype(np.float32)
+    first = backend.linear(dev(x, gpu), layer, name)
+    check_parity(host(first), (x.astype(np.float32) @ w32.T).astype(np.float16), plan)
+    for _ in range(5):
+        assert torch.equal(backend.linear(dev(x, gpu), layer, name), first)
+    p = layer['self_attn.qkv_proj._prepared']
+    small = _native.w4a16_linear(dev(x, gpu), p.tiles, p.meta, n, g, workspace=torch.zeros(16, dtype=torch.uint8, device=gpu))
+    check_parity(host(small), (x.astype(np.float32) @ w32.T).astype(np.float16), 'without its workspace')
 
 
 def test_batch_plans_use_the_workspace_and_fall_back_without_it(gpu):
