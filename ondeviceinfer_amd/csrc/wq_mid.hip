@@ -389,7 +389,7 @@ bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
   return w4 && M >= 12 && M <= 32 && (N + 15) / 16 <= 1152 && nblk <= 64 && nblk % 4 == 0;
 }
 
-// The shapes this file takes: those whose plan is estimated below the skinny
+// The shapes this file takes: those whose plan is estimated below the other
 // kernels' time.  W4: the skinny kernels take rounds of 256 workgroups (two
 // tiles a wave, four from 1024 tiles on) whose time is a chain of k blocks,
 //   rounds x blocks x (0.034 + 0.108 per 16-row chunk + 0.006 per row) us
@@ -407,10 +407,14 @@ bool mid_counts(bool w4, int64_t M, int64_t N, int64_t K) {
 // 31 / 41 us).  Shorter ones would gain as well (2048->34816 M = 24 / 48 17.0 /
 // 23.1 against 15.0 / 16.5) but keep the deep ring, whose rows equal those of a
 // longer call bit for bit; the long chains' rows no longer do.
-// INT8: from 33 rows on, and weights of at least 10000 tile blocks (20 MB;
-// 5120->1024 M = 8 6.6 us against 8.6, 2048->4040 5.2 against 8.2 the other
-// way) or, from 17 rows, chains of at least 32 blocks (5120->1024 M = 24 12.9
-// -> 9.3 us, 2048->4040 8.2 against 9.1).
+// INT8: the same with the INT8 skinny kernels' chain, one tile a wave up to 16
+// rows and two above:
+//   rounds x blocks x (0.124 + 0.0129 per row, from 17 rows 0.407 + 0.0094) us
+// (0.07 % off the faster side on average, 10 % at most; the line on the weight's
+// size and the chain before was 2.5 % off).  Skinny against this file, us:
+// 5120->1024 M = 8 / 24 / 33 6.7 / 12.8 / 18.1 against 8.1 / 9.2 / 10.2, 512->2048
+// M = 33 6.1 / 8.6, 1024->6144 M = 36 7.5 / 9.9, 5120->4040 M = 8 8.1 / 10.1,
+// 2048->17408 M = 5 11.8 / 13.6, 5120->17408 M = 8 26.9 / 22.
 // wq_batch.hip's shapes come off both (w4_batch_plan).
 // Returns the plan, or one without groups for the other shapes; W4 only:
 // best_us the estimated time of the faster of the two sides.
@@ -418,7 +422,14 @@ MidSplit mid_route(bool w4, int64_t M, int64_t N, int64_t K, double* best_us = n
   constexpr MidSplit kNone{0, 0, 0};
   if (M <= 4 || M > 64 || K % kW4BlockK != 0 || K < kW4BlockK || K > kMidMaxK) return kNone;
   const int64_t ntile = (N + 15) / 16, nblk = K / kW4BlockK;
-  if (!w4) return M > 32 || ntile * nblk >= 10000 || (M > 16 && nblk >= 32) ? mid_plan(w4, M, N, K) : kNone;
+  if (!w4) {
+    const int64_t rounds = ((M <= 16 ? ntile : (ntile + 1) / 2) + 255) / 256;
+    const double chain = (double)(rounds * nblk) * (M <= 16 ? 0.124 + 0.0129 * (double)M : 0.407 + 0.0094 * (double)M);
+    const double skinny = chain + 1.94 * (double)((M + 15) / 16) + (M <= 16 ? 0.86 : 0.0) - 9.4;
+    if (skinny <= 0.0) return kNone;
+    const MidSplit p = mid_plan(w4, M, N, K);
+    return p.us + (p.s > 1 ? 1.0 : 0.0) < skinny ? p : kNone;
+  }
   if (ntile >= 2048 && M > 16) return nblk >= 32 ? mid_plan(w4, M, N, K) : kNone;
   const double mc = (double)((M + 15) / 16);
   const bool four = ntile >= 1024;   // tiles per wave of the skinny kernels (pick_skinny)

@@ -132,3 +132,16 @@ def test_w4_rows_5_to_64_take_the_kernel_estimated_faster():
         for n, k in ((1024, 5120), (5120, 5120), (7168, 5120), (17408, 5120), (12288, 2048)):
             assert plan(m, n, k) == 'mid', (m, n, k)
     assert plan(33, 34816, 1024) == 'deep' and plan(33, 34816, 5120) == 'mid'
+
+
+def test_int8_rows_5_to_64_take_the_kernel_estimated_faster():
+    plan = lambda m, n, k: _native.linear_plan('w8a16', m, n, k).split()[0]
+    rows = range(5, 65)
+    for n, k in ((512, 512), (2048, 512), (6144, 512), (4040, 512)):
+        assert {plan(m, n, k) for m in rows} == {'skinny'}, (n, k)
+    for n, k in ((5120, 17408), (17408, 5120), (34816, 5120), (9216, 12288)):
+        assert {plan(m, n, k) for m in rows} == {'mid'}, (n, k)
+    for n, k in ((1024, 5120), (5120, 5120), (6144, 1024), (4040, 5120), (17408, 2048)):
+        taken = [plan(m, n, k) == 'mid' for m in rows]
+        assert taken == sorted(taken), (n, k)
+    assert plan(8, 1024, 5120) == plan(33, 2048, 512) == 'skinny' and plan(24, 1024, 5120) == 'mid'

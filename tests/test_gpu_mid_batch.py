@@ -165,3 +165,19 @@ def test_w4_mid_shapes_match_oracle(gpu, m, n, k, g):
     y = backend.linear(dev(x, gpu), layer, 'p.weight')
     check_parity(host(y), (x.astype(np.float32) @ w32.T).astype(np.float16), plan)
     assert torch.equal(backend.linear(dev(x, gpu), layer, 'p.weight'), y)
+
+
+# INT8 shapes the kernel takes: both ends of the 16-row chunks, an odd block count, partial last tile groups,
+# n not a multiple of 4, many splits, ten-tile groups unsplit and in two splits.
+@pytest.mark.parametrize('m,n,k', [(5, 5112, 17280), (16, 1001, 12416), (17, 1000, 8064), (32, 17408, 4992),
+                                   (33, 1001, 3968), (48, 34816, 640), (49, 2050, 8448), (64, 17408, 1280)])
+def test_w8_mid_shapes_match_oracle_in_both_layouts(gpu, m, n, k):
+    plan = _native.linear_plan('w8a16', m, n, k)
+    print(f'[mid] int8 m={m} n={n} k={k}: {plan}', flush=True)
+    assert plan.startswith('mid')
+    _, q, s, x = synth.int8_case(n, k, m, seed=n % 97 + k)
+    qd, sd, xd = dev(q, gpu), dev(s, gpu), dev(x, gpu)
+    w32 = qdq.dequantize_linear_weight(q, s).astype(np.float32)
+    y = _native.w8a16_linear(xd, _native.w8_repack(qd), sd)
+    assert torch.equal(y, _native.w8a16_linear(xd, qd, sd))
+    check_parity(host(y), (x.astype(np.float32) @ w32.T).astype(np.float16), plan)
