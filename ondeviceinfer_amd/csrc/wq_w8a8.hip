@@ -421,6 +421,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(const int8_t* __restr
 // i.e. 178 MB of weights at M = 8 in 32 us without the quantizer (5.6 TB/s).
 constexpr int kM8Tiles = kMidTilesPerWave;
 constexpr int kM8MaxM = 255;   // from 256 rows the GEMM takes 128-row tiles
+constexpr int kM8GemvMaxM = 16;
 
 // The MC fragments of one k-step (16 rows apart in a stage), read and waited
 // for in one asm block (see i8_lds_read_off for why asm).
@@ -635,30 +636,50 @@ struct M8Plan {
   size_t bytes() const { return mid_partial_bytes(m, nz, mc); }
 };
 
+// What the GEMV (up to 16 rows) or the GEMM on 32-row tiles below would take
+// beside this kernel, us above this kernel's constant part.  GEMV: one round of
+// loads per chain, rounds of 256 workgroups (one per tile), and x read by every
+// tile; GEMM: a chain of k blocks whose cost grows with the workgroups, at one
+// or four tiles a wave (w8a8_route).  Constants fitted so that the measured
+// faster side wins, over k = 512..17408, N = 512..34816, M = 5..255 (4000
+// points: 0.35 % off the faster side on average, 10 % at most on the projection
+// shapes of 5120 and 17408; five thresholds on M, the chain and the tiles were
+// 1.4 % off).
+double m8_other_us(int64_t M, int64_t ntile, int64_t nblk, int mc) {
+  const double b = (double)nblk;
+  if (M <= kM8GemvMaxM)
+    return b * (0.048 + 0.087 * (double)((ntile + 255) / 256) + 0.114 * (double)(ntile * M) / (320.0 * 16)) - 4.3;
+  const int64_t mblocks = (M + 31) / 32, wide = (ntile + 15) / 16 * mblocks;
+  const double x = 0.31 * mc / 8;   // this kernel's row chunks
+  if (wide >= 256) return b * (1.024 + 0.576 * (double)((wide + 255) / 256) - x) - 4.3;
+  return b * (0.544 + 0.224 * (double)((ntile + 3) / 4 * mblocks) / 256 - x) - 4.3;
+}
+
+// Taken where the plan is estimated below the others (with the quantizer left
+// out, us, others against this kernel: N = 1024 M = 8 5.9 / 8.8; 5120^2 M = 8 / 16
+// 10.5 / 11.1, 13.1 / 11.2; 2048->4040 M = 16 5.2 / 9.1; 3328->13000 M = 96 / 200
+// 20.2 / 22.4, 52 / 31; 2048->17408 M = 65 16.9 / 19.9; 5120->17408 M = 128 / 200
+// 53 / 39, 54.6 / 59; 5120->34816 M = 129 / 255 90 / 98, 148 / 116).
 // Row blocks: one up to 128 rows (the weights are read once), except two on
 // narrow N with short k chains, where the rows give the parallelism that more
 // splits would (5120^2 M = 96: 15.2 us for two blocks in three splits, 16.9
 // for one in six).  Depth: three stages while a compute unit holds one
-// workgroup, two (two workgroups fit) beyond.  Not taken: M <= 4, and M <= 16
-// where the GEMV is as fast (short, narrow shapes: N = 1024 M = 8 5.9 us
-// against 8.9; 5120^2 M = 8 10.5 against 10.7; 2048->4040 M = 16 / 40, with the
-// quantizer, 7.8 / 12.4 against 11.9 / 13.8; 3328->13000 M = 96 24.2 against
-// 26.3); above 128 rows the shapes whose
-// GEMM grid already fills the machine (N = 17408 M = 200 53 us against 58).
+// workgroup, two (two workgroups fit) beyond.
 M8Plan m8_plan(int64_t M, int64_t N, int64_t K) {
   M8Plan p{0, 1, 2, {4, 1, 0}};
   const int64_t ntile = (N + 15) / 16, nblk = K / kI8Blk, g8 = (ntile + 7) / 8;
   if (M <= 4 || M > kM8MaxM || K % kI8Blk != 0 || K > (1 << 23)) return p;
-  const bool long_k = nblk >= 64;
-  if (nblk < 20 && ntile * nblk < 10000) return p;
-  if (M <= 16 && !long_k && g8 < 128 && !(M > 8 && g8 >= 32 && ntile * nblk >= 10000)) return p;
-  if (M > 64 && M <= 128 && nblk < 32 && g8 > 64 && g8 <= 128) return p;
-  if (M > 128 && !long_k && (g8 < 40 || (g8 > 128 && g8 < 256))) return p;
-  if (M > 128 || (!long_k && g8 <= 64 && M > (g8 <= 16 ? 32 : 48))) p.nz = 2;
-  const int mc = (int)((M + 16 * p.nz - 1) / (16 * p.nz));
-  p.mc = mc <= 4 ? mc : mc <= 6 ? 6 : 8;
-  p.m = mid_split(ntile, (nblk + 3) / 4, 4 * kW8TileBlockBytes, 4.0 * p.mc * 16 * kI8RowBytes, p.nz, p.mc);
-  p.d = p.m.groups * p.nz * p.m.s <= 256 && p.mc < 8 ? 3 : 2;
+  if (M > 128 && nblk < 64 && ntile < 320) return p;   // two row blocks of few tiles: 5120->2048 M = 192 16.2 against 13.2
+  if (M > 128 || (nblk < 64 && g8 <= 64 && M > (g8 <= 16 ? 32 : 48))) p.nz = 2;
+  const int chunks = (int)((M + 16 * p.nz - 1) / (16 * p.nz));
+  const int mc = chunks <= 4 ? chunks : chunks <= 6 ? 6 : 8;
+  double other = m8_other_us(M, ntile, nblk, mc);
+  if (other + 0.38 * (double)nblk <= 0.0) return p;
+  p.m = mid_split(ntile, (nblk + 3) / 4, 4 * kW8TileBlockBytes, 4.0 * mc * 16 * kI8RowBytes, p.nz, mc);
+  if (M > kM8GemvMaxM && p.m.p == 5) other += 0.38 * (double)nblk;   // ten-tile groups: estimated high by that
+  if (p.m.us + (p.m.s > 1 ? 0.4 : 0.0) >= other) return p;
+  p.mc = mc;
+  p.d = p.m.groups * p.nz * p.m.s <= 256 && mc < 8 ? 3 : 2;
   return p;
 }
 
@@ -824,7 +845,7 @@ __global__ __launch_bounds__(512, 2) void w8a8_gemm256_kernel(const int8_t* __re
       m8_store(acc[t][mt], m0 + wm * 128 + mt * 16 + i, (tile0 + wn * 4 + t) * 16 + 4 * kb, M, N, sx, sw, bias, y);
 }
 
-constexpr int kW8A8GemvMaxM = 16;
+constexpr int kW8A8GemvMaxM = kM8GemvMaxM;
 // Largest k of the W8A8 GEMM: a workgroup reads its 128 x rows and up to 64
 // weight rows of k bytes each through one buffer apiece, whose record count is
 // capped at 2^31 - 1 bytes; longer rows run the GEMV kernel 16 rows at a time.

@@ -145,3 +145,14 @@ def test_int8_rows_5_to_64_take_the_kernel_estimated_faster():
         taken = [plan(m, n, k) == 'mid' for m in rows]
         assert taken == sorted(taken), (n, k)
     assert plan(8, 1024, 5120) == plan(33, 2048, 512) == 'skinny' and plan(24, 1024, 5120) == 'mid'
+
+
+def test_w8a8_rows_5_to_255_take_the_kernel_estimated_faster():
+    plan = lambda m, n, k: _native.linear_plan('w8a8', m, n, k).split()[0]
+    for n, k in ((512, 512), (1024, 2048), (4040, 2048), (9216, 512)):
+        assert 'mid' not in {plan(m, n, k) for m in range(5, 201)}, (n, k)
+    for n, k in ((1024, 17408), (5120, 17408), (7168, 8192)):
+        assert {plan(m, n, k) for m in range(17, 129)} == {'mid'}, (n, k)
+    assert {plan(m, 34816, 5120) for m in range(5, 65)} == {'mid'} and plan(129, 34816, 5120) == 'gemm'
+    assert plan(8, 5120, 5120) == 'gemv' and plan(16, 5120, 5120) == plan(48, 17408, 5120) == 'mid'
+    assert plan(200, 13000, 3328) == 'mid' and plan(96, 13000, 3328) == plan(200, 17408, 5120) == 'gemm'

@@ -52,6 +52,30 @@ def test_w8a8_mid_bit_exact_in_both_layouts(n, k, ms):
         assert np.array_equal(host(y).view(np.uint16), expected[:rows])
 
 
+# Shapes the kernel takes: one to eight 16-row chunks, two row blocks, splits, ten-tile groups unsplit and in two
+# splits, partial last tile groups and stages.
+@pytest.mark.parametrize('m,n,k', [(17, 1001, 8320), (64, 1001, 8320), (96, 1001, 8320), (128, 1001, 8320),
+                                   (255, 1001, 8320), (16, 7176, 5248), (33, 7176, 5248), (192, 7176, 5248),
+                                   (5, 33000, 4224), (49, 17400, 5120), (128, 17400, 5120)])
+def test_w8a8_mid_shapes_bit_exact(m, n, k):
+    plan = _native.linear_plan('w8a8', m, n, k)
+    print(f'[w8a8 mid] m={m} n={n} k={k}: {plan}', flush=True)
+    assert plan.startswith('mid')
+    rng = np.random.default_rng(n + k + m)
+    qx, qw = (rng.integers(-127, 128, s, dtype=np.int8) for s in ((m, k), (n, k)))
+    xs, wsc = ((rng.random(s) * 0.01 + 1e-4).astype(np.float32) for s in (m, n))
+    tiles = _native.w8_repack(dev(qw))
+    got = host(_native.w8a8_linear(dev(qx), dev(xs), tiles, dev(wsc)))
+    lib, y = _native.load(), torch.empty(m, n, dtype=torch.float16, device='cuda:0')
+    td = (dev(qx), dev(xs), dev(wsc))
+    assert lib.wq_w8a8_linear_tiled(td[0].data_ptr(), td[1].data_ptr(), m, k, tiles.tiles.data_ptr(), td[2].data_ptr(),
+                                    n, None, y.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    assert np.array_equal(got.view(np.uint16), host(y).view(np.uint16))   # without the splits' workspace
+    rows, cols = sorted({0, 15, m // 2, m - 1} & set(range(m))), np.r_[0:32, n // 2:n // 2 + 16, n - 40:n]
+    expected = qdq.w8a8_linear_int(qx[rows], xs[rows], qw[cols], wsc[cols], None)
+    assert np.array_equal(got[rows][:, cols].view(np.uint16), expected.view(np.uint16))
+
+
 # 1024 threads a row (m <= 512) with one and three chunks a thread, 256 threads with
 # one, three and nine, and rows too long to stay in registers.
 @pytest.mark.parametrize('m,k', [(7, 2056), (48, 8192), (512, 8200), (2, 24576), (513, 2048), (600, 5120), (530, 17408),
