@@ -27,6 +27,8 @@
 #include "wq_common.h"
 #include "wq_status.h"
 
+#include <algorithm>
+
 namespace wq {
 namespace {
 
@@ -731,15 +733,15 @@ bool gemm_takes_deep(long M, long N, bool w4_or_tiles) {
 // The grid of least estimated time for W4 weights or INT8 tiles (every grid
 // gives the same bits).  On MI355X a grid takes c rounds of 256 workgroups, c
 // = ceil(workgroups / 256), at a cost per round that hardly depends on how
-// many of a compute unit's workgroups run side by side, only on the tile:
-// K = 5120, us per round over M = 100..1500 on N = 5120..34816:
-//          4x8   4x4   2x8   2x4   1x4   deep 1x2   (4x6, 4x7, 2x5, 2x6 in between)
-//   W4     68    41.5  40    22    13.9  11.7
-//   INT8   77    48    45.5  24.5  14.3  12.6
-// A single round leaves each SIMD one wave, with nothing beside its load waits
-// (4x8 W4 92 us instead of 68; narrow tiles about 1.75 times and more), and an
-// odd round of 112- or 128-row tiles, two of which share a compute unit, runs
-// its last one alone.  So rows padded to the tile and rounds left partly empty
+// many of a compute unit's workgroups run side by side, only on the tile: a
+// chain of k blocks and, at its end, the stores, which on INT8 (scales, bias)
+// weigh two to three times what they do on W4.  The table holds what each takes at
+// K = 5120.  A single round leaves each SIMD one wave, with nothing beside its
+// load waits (alone: 1.2 to 2 of a round among others); an odd round of 112- or
+// 128-row tiles, two of which share a compute unit, runs its last one alone; a
+// last round partly empty costs slightly less.  Of the deep ring's 32-row tiles
+// several workgroups fit a compute unit, so past two rounds its time follows
+// the workgroups.  So rows padded to the tile and rounds left partly empty
 // decide, and the tile heights in between give a ragged M a grid that does
 // neither (us, W4 / INT8):
 //   17408->5120 M = 777   2x4 (520 workgroups, three rounds) 199 / 221 -> 2x5 (400, two) 175 / 163
@@ -749,33 +751,42 @@ bool gemm_takes_deep(long M, long N, bool w4_or_tiles) {
 //   fused gate_up M = 777 4x8 271 / 309 -> 4x7 254 / 281;  M = 400  197 / 205 -> 172 / 184 (4x6)
 //   5120->17408 M = 200   67 / 79 -> 59 / 61 (2x5)
 //   5120^2 M = 200        deep 34.4 / 37 -> 1x4 30 / 31; INT8 17408->5120 133 -> 95
-// The widest tile keeps a 3 % lead: it reads the least through L2.
+// Constants fitted to all ten grids' times over k = 512..17408, N = 512..34816,
+// M = 65..4096 (1932 W4 and 2574 INT8 shapes: 0.15 / 1.1 % off the fastest grid
+// on average; slower than the threshold rule's grid by more than 3 % at 2 / 22,
+// 12 % at most; costs without their share of the chain were 1.5 / 2.0 % off, slower
+// at 27 / 62, e.g. INT8 5120->34816 M = 128 105 us on 1x4 against 90 on 2x4).
 struct GridCost {
   Grid grid;
   int nt, mt;
-  float w4, w8, alone;   // us per round (K = 5120), factor of a single round
+  double w4, w4_end, w8, w8_end;   // us of a round at K = 5120, and the part of it that is not the chain
+  double w4_alone, w8_alone;       // factor of a single round
 };
 constexpr GridCost kGridCosts[] = {
-    {Grid::k4x8, 4, 8, 66.0f, 74.7f, 1.4f}, {Grid::k4x7, 4, 7, 60.0f, 68.0f, 1.4f},
-    {Grid::k4x6, 4, 6, 53.8f, 61.4f, 1.4f}, {Grid::k4x4, 4, 4, 41.5f, 48.0f, 1.4f},
-    {Grid::k2x8, 2, 8, 40.0f, 45.5f, 1.4f}, {Grid::k2x6, 2, 6, 31.0f, 35.0f, 1.7f},
-    {Grid::k2x5, 2, 5, 27.0f, 30.5f, 1.75f}, {Grid::k2x4, 2, 4, 22.0f, 24.5f, 1.75f},
-    {Grid::k1x4, 1, 4, 13.9f, 14.3f, 2.2f}, {Grid::kDeep, 1, 2, 11.7f, 12.6f, 1.9f}};
+    {Grid::k4x8, 4, 8, 62.6, 5.1, 70.3, 10.6, 1.67, 1.67}, {Grid::k4x7, 4, 7, 60.0, 4.1, 67.6, 10.2, 1.84, 1.84},
+    {Grid::k4x6, 4, 6, 55.1, 2.8, 66.3, 9.1, 1.38, 1.38}, {Grid::k4x4, 4, 4, 44.4, 1.9, 46.5, 4.6, 1.19, 1.19},
+    {Grid::k2x8, 2, 8, 37.9, 1.9, 43.4, 4.5, 1.38, 1.38}, {Grid::k2x6, 2, 6, 31.1, 1.0, 34.8, 2.8, 1.40, 1.40},
+    {Grid::k2x5, 2, 5, 26.1, 0.68, 28.4, 1.9, 1.65, 1.65}, {Grid::k2x4, 2, 4, 22.3, 0.84, 23.7, 1.5, 1.59, 1.59},
+    {Grid::k1x4, 1, 4, 14.1, 0.17, 14.6, 1.0, 1.90, 1.95}, {Grid::kDeep, 1, 2, 14.2, 0.5, 16.1, 0.4, 1.68, 1.25}};
+constexpr double kW4DeepTwoRounds = 1.86, kW8DeepTwoRounds = 1.6;   // the deep ring's second round
 
 // allow_deep / min_nt: the grids the caller can use (the fused epilogues have
 // no deep ring, and SiluPair pairs tiles within a wave).
-Grid gemm_grid(long M, long N, bool w4, bool allow_deep, int min_nt) {
+Grid gemm_grid(long M, long N, long K, bool w4, bool allow_deep, int min_nt) {
   const long ntile = (N + 15) / 16;
+  const double chain = (double)(K / kW4BlockK) / 40;
   Grid best = Grid::k2x4;
-  float best_us = 1e30f;
+  double best_us = 1e30;
   for (const GridCost& g : kGridCosts) {
     if ((g.grid == Grid::kDeep && !allow_deep) || g.nt < min_nt) continue;
     const long wgs = ((ntile + 4 * g.nt - 1) / (4 * g.nt)) * ((M + 16 * g.mt - 1) / (16 * g.mt));
     const long c = (wgs + 255) / 256;
-    float rounds = (float)c;
-    if (c == 1) rounds = g.alone;
-    else if (g.mt >= 7 && (c & 1)) rounds += 0.15f;
-    const float us = rounds * (w4 ? g.w4 : g.w8);
+    const double full = (double)wgs / 256;
+    double rounds = (double)c - 0.05 * ((double)c - full);
+    if (c == 1) rounds = w4 ? g.w4_alone : g.w8_alone;
+    else if (g.grid == Grid::kDeep) rounds = std::max(full, w4 ? kW4DeepTwoRounds : kW8DeepTwoRounds);
+    else if (g.mt >= 7 && (c & 1)) rounds += 0.16;
+    const double end = w4 ? g.w4_end : g.w8_end, us = rounds * (((w4 ? g.w4 : g.w8) - end) * chain + end);
     if (us < best_us) {
       best_us = us;
       best = g.grid;
@@ -794,7 +805,7 @@ int launch_gemm_auto(const half_t* x, int M, int K, const void* w, const void* m
     // every whole-k grid of these shapes.
     const bool split = F == GFmt::W4 && deep && bias == nullptr && ws != nullptr && deep_splits<1, 2>(M, N, K) > 1 &&
                        ws_bytes >= deep_ws_bytes<1, 2>(M, N, K);
-    switch (split ? Grid::kDeep : gemm_grid(M, N, F == GFmt::W4, deep, 1)) {
+    switch (split ? Grid::kDeep : gemm_grid(M, N, K, F == GFmt::W4, deep, 1)) {
       case Grid::k4x8: return launch_gemm<F, 4, 8>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k4x7: return launch_gemm<F, 4, 7>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
       case Grid::k4x6: return launch_gemm<F, 4, 6>(x, M, K, w, meta, N, bpg, bias, y, s, w8_tiled);
@@ -834,7 +845,7 @@ size_t w4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 void gemm_plan_text(bool w4, int64_t M, int64_t N, int64_t K, int epilogue, char* text, size_t bytes) {
   const bool deep = gemm_takes_deep(M, N, true);
   const int S = w4 && deep && epilogue == 0 ? deep_splits<1, 2>((int)M, (int)N, (int)K) : 1;
-  const Grid grid = S > 1 ? Grid::kDeep : gemm_grid(M, N, w4, epilogue == 0 && deep, epilogue == 1 ? 2 : 1);
+  const Grid grid = S > 1 ? Grid::kDeep : gemm_grid(M, N, K, w4, epilogue == 0 && deep, epilogue == 1 ? 2 : 1);
   for (const GridCost& g : kGridCosts)
     if (g.grid == grid) {
       if (grid == Grid::kDeep) snprintf(text, bytes, "deep %dx%dx%d", g.nt, g.mt, S);
@@ -863,7 +874,7 @@ template <GFmt F, Epi EP>
 int launch_gemm_epi(const half_t* x, int M, int K, const void* w, const void* meta, int N, int bpg, const half_t* res,
                     half_t* y, hipStream_t s) {
   constexpr int tiled = F == GFmt::W8;
-  switch (gemm_grid(M, N, F == GFmt::W4, false, EP == Epi::SiluPair ? 2 : 1)) {
+  switch (gemm_grid(M, N, K, F == GFmt::W4, false, EP == Epi::SiluPair ? 2 : 1)) {
     case Grid::k4x8: return launch_gemm<F, 4, 8, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     case Grid::k4x7: return launch_gemm<F, 4, 7, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);
     case Grid::k4x6: return launch_gemm<F, 4, 6, EP>(x, M, K, w, meta, N, bpg, nullptr, y, s, tiled, res);

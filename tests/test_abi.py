@@ -156,3 +156,23 @@ def test_w8a8_rows_5_to_255_take_the_kernel_estimated_faster():
     assert {plan(m, 34816, 5120) for m in range(5, 65)} == {'mid'} and plan(129, 34816, 5120) == 'gemm'
     assert plan(8, 5120, 5120) == 'gemv' and plan(16, 5120, 5120) == plan(48, 17408, 5120) == 'mid'
     assert plan(200, 13000, 3328) == 'mid' and plan(96, 13000, 3328) == plan(200, 17408, 5120) == 'gemm'
+
+
+def test_every_prefill_grid_is_reached_and_tested():
+    """The GPU test's shapes run the grids it names, cover the cost table's
+    nine plain grids, and have each fused epilogue on every grid it exists on."""
+    from test_gpu_gemm_grids import EVERY_GRID
+    assert list(EVERY_GRID) == ['1x4', '2x4', '2x5', '2x6', '2x8', '4x4', '4x6', '4x7', '4x8']
+    for grid, shapes in EVERY_GRID.items():
+        for fmt in ('w4a16', 'w8a16'):
+            for shape in shapes:
+                assert _native.linear_plan(fmt, *shape) == f'gemm {grid}', (fmt, shape)
+            modes = {e for e in (_native.EPI_SILU_MUL, _native.EPI_RESIDUAL) for m, n, k in shapes
+                     if (_native.w4a16_epilogue_supported(m, n, k, 128, e) if fmt == 'w4a16'
+                         else _native.w8a16_epilogue_supported(m, n, k, e))
+                     and _native.linear_plan(fmt, m, n, k, e) == f'gemm {grid}'}
+            assert modes == ({2} if grid == '1x4' else {1, 2}), (fmt, grid, modes)
+    # Costs follow the whole round: narrow tiles on short chains, the wide ones' lead on long ones.
+    assert _native.linear_plan('w8a16', 128, 34816, 5120) == 'gemm 2x4'
+    assert _native.linear_plan('w4a16', 4096, 17408, 5120) == _native.linear_plan('w8a16', 4096, 34816, 5120) == 'gemm 4x8'
+    assert _native.linear_plan('w4a16', 65, 5120, 1280) == 'deep 1x2x1'

@@ -1,7 +1,9 @@
-"""Prefill GEMM grids (wq_gemm.hip): row counts at the edges of the 64- and
-128-row tiles on each grid give the rows of the 64-wide grid bit for bit (one
+"""Prefill GEMM grids (wq_gemm.hip): row counts around the edges of the tiles
+give, on every grid, the rows of a longer call on another grid bit for bit (one
 k order on every grid), the fused epilogues equal the plain GEMM plus the
-elementwise op, and sampled rows hold the oracle's bar (``parity_ok``)."""
+elementwise op, and sampled rows hold the oracle's bar (``parity_ok``).
+``EVERY_GRID`` names the grid each of its shapes runs (checked against the
+library, here and on the CPU in ``test_abi.py``)."""
 import numpy as np
 import pytest
 import torch
@@ -13,13 +15,20 @@ from ondeviceinfer_amd.weight_quantization import backend as wq
 pytestmark = pytest.mark.gpu
 
 
-# (m, n, k), one tile height after the other: 2 tiles x 80 rows (129; 673 =
-# 8 x 80 + 33), 4 x 96 (448 ends inside a block, 34800 inside a slice; 577 =
-# 6 x 96 + 1), 4 x 112 (777, 785 takes 128), 2 x 96 (1056 = 11 x 96), 2 x 128
-# (1345, 1500; 5112 ends inside a tile), 1 x 64, 2 x 64, 4 x 64.
+# (m, n, k) on short chains: a last row block of one row (129 = 128 + 1, 449, 577, 785,
+# 1345, 673 of 32), columns that end inside a slice (34800, 17400) or a tile (5112, 4040).
 SHAPES = [(129, 34816, 256), (673, 7168, 384), (448, 34800, 128), (577, 17400, 256), (777, 34816, 128),
           (785, 34816, 128), (1056, 5112, 256), (1345, 5120, 384), (1500, 5112, 256), (200, 5120, 640),
           (449, 4040, 256), (700, 5120, 256)]
+
+
+# The grid (weight tiles per wave x 16-row chunks) of every entry of the cost table, plain and with both epilogues
+# where they apply; each with a ragged last row block, and one whose columns end inside a tile.
+EVERY_GRID = {'1x4': [(707, 2048, 640)], '2x4': [(577, 5120, 640), (774, 4040, 640)],
+              '2x5': [(769, 5120, 640), (775, 5112, 640)], '2x6': [(845, 7168, 640)],
+              '2x8': [(1043, 7168, 1920), (1529, 5112, 1920)], '4x4': [(1537, 5120, 3328), (1542, 5112, 3328)],
+              '4x6': [(1465, 7168, 3328)], '4x7': [(1782, 7168, 1280), (1765, 7160, 1280)],
+              '4x8': [(2164, 7168, 1280)]}
 
 
 def same(a, b):
@@ -66,10 +75,20 @@ def test_grids_agree_and_hold_the_oracle(gpu, fmt, m, n, k):
         assert same(plain(x), _native.w8a16_linear(x, q, s))   # row-major: its own grids
     y = plain(x)
     check(y, x, w32, (fmt, m, n, k))
-    # The same rows inside a longer call, which takes the widest grid.
+    # The same rows inside a longer call (most on another grid).
     longer = plain(torch.cat([x, torch.randn(4096 - m, k, generator=gen, device=gpu).half()]))
     assert same(y, longer[:m])
     if takes(_native.EPI_RESIDUAL):
         assert same(fused(_native.EPI_RESIDUAL, res), res + y)
     if takes(_native.EPI_SILU_MUL):
         assert same(fused(_native.EPI_SILU_MUL), _native.silu_mul(y))
+
+
+@pytest.mark.parametrize('grid,m,n,k', [(grid, *shape) for grid, shapes in EVERY_GRID.items() for shape in shapes])
+@pytest.mark.parametrize('fmt', ['w4', 'int8'])
+def test_every_grid_agrees_and_holds_the_oracle(gpu, fmt, grid, m, n, k):
+    name = {'w4': 'w4a16', 'int8': 'w8a16'}[fmt]
+    assert _native.linear_plan(name, m, n, k) == f'gemm {grid}'
+    if fmt == 'w4' and grid != '4x8':   # INT8 is compared with the row-major weight's own grids
+        assert _native.linear_plan(name, 4096, n, k) != f'gemm {grid}'
+    test_grids_agree_and_hold_the_oracle(gpu, fmt, m, n, k)
