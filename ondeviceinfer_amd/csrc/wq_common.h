@@ -126,53 +126,26 @@ __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t vo
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_base, 16, voff, soff, 0, 0);
 }
 
-// 16-byte LDS read issued as inline asm, for kernels that fill LDS with the
-// direct copies above: the compiler cannot tell such a copy into the next
-// stage from a read of the current one and waits for all of them (vmcnt(0))
-// before any LDS read it can see, which serializes the copy with the math.
-// These reads are invisible to it; lds_wait_first_half / lds_wait_rest must
-// complete them before use.
-__device__ __forceinline__ uint4_t lds_read16_asm(const uint8_t* p) {
-  const uint32_t a = (uint32_t)(size_t)((const __attribute__((address_space(3))) uint8_t*)p);
-  uint4_t v;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(a));
-  return v;
-}
-
-// For MT reads issued in order: wait until the first MT/2 have landed (LDS
-// reads return in order), then until all have; each wait is tied to the
-// fragments it completes so that no use moves above it.
-template <int MT>
-__device__ __forceinline__ void lds_wait_first_half(uint4_t (&b)[MT]) {
-  static_assert(MT == 1 || MT == 2 || MT == 4 || MT == 8 || MT == 16, "fragment count");
-  if constexpr (MT == 1) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b[0]));   // a single read: all of it
-  } else if constexpr (MT == 16) {
-    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]),
-                 "+v"(b[6]), "+v"(b[7]));
-  } else if constexpr (MT == 8) {
-    asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
-  } else if constexpr (MT == 4) {
-    asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(b[0]), "+v"(b[1]));
-  } else {
-    asm volatile("s_waitcnt lgkmcnt(1)" : "+v"(b[0]));
-  }
-}
-template <int MT>
-__device__ __forceinline__ void lds_wait_rest(uint4_t (&b)[MT]) {
-  static_assert(MT == 1 || MT == 2 || MT == 4 || MT == 8 || MT == 16, "fragment count");
-  if constexpr (MT == 1) {
-    // completed by lds_wait_first_half
-  } else if constexpr (MT == 16) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b[8]), "+v"(b[9]), "+v"(b[10]), "+v"(b[11]), "+v"(b[12]), "+v"(b[13]),
-                 "+v"(b[14]), "+v"(b[15]));
-  } else if constexpr (MT == 8) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b[4]), "+v"(b[5]), "+v"(b[6]), "+v"(b[7]));
-  } else if constexpr (MT == 4) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b[2]), "+v"(b[3]));
-  } else {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b[1]));
-  }
+// Kernels that fill LDS with the direct copies above read it with inline asm:
+// the compiler cannot tell such a copy into the next stage from a read of the
+// current one and waits for all of them (vmcnt(0)) before any LDS read it can
+// see, which serializes the copy with the math.  Reads in asm are invisible to
+// it, so each must be completed by a wait like this one before use.  LDS reads
+// return in order.
+// Wait until at most LEFT of the LDS reads issued are outstanding, tied to the
+// fragments [LO, HI) it completes so that no use moves above it.
+template <int MT, int LO, int HI, int LEFT>
+__device__ __forceinline__ void lds_wait_frags(uint4_t (&b)[MT]) {
+  static_assert(HI - LO >= 1 && HI - LO <= 4, "fragment count");
+  if constexpr (HI - LO == 1)
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[LO]) : "i"(LEFT));
+  else if constexpr (HI - LO == 2)
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[LO]), "+v"(b[LO + 1]) : "i"(LEFT));
+  else if constexpr (HI - LO == 3)
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]) : "i"(LEFT));
+  else
+    asm volatile("s_waitcnt lgkmcnt(%4)"
+                 : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]), "+v"(b[LO + 3]) : "i"(LEFT));
 }
 
 __device__ __forceinline__ half2_t as_h2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }

@@ -60,7 +60,7 @@ struct WRegs<GFmt::W8, NT> {
 // The MT B-fragments of one k-step: fragment mt is row mt*16 + i of the
 // stage, so its address is a per-lane base plus the immediate mt*16 rows
 // (no address arithmetic per read).  Inline asm for the reason given at
-// lds_read16_asm.
+// lds_wait_frags.
 template <int OFF>
 __device__ __forceinline__ uint4_t lds_read16_off(uint32_t a) {
   uint4_t v;
@@ -74,22 +74,6 @@ __device__ __forceinline__ void lds_read_frags(uint4_t (&b)[MT], uint32_t a) {
     lds_read_frags<MT, LO + 1, HI>(b, a);
   }
 }
-// Wait until at most LEFT of the LDS reads issued are outstanding, tied to the
-// fragments [LO, HI) it completes so that no use moves above it.
-template <int MT, int LO, int HI, int LEFT>
-__device__ __forceinline__ void lds_wait_frags(uint4_t (&b)[MT]) {
-  static_assert(HI - LO >= 1 && HI - LO <= 4, "fragment count");
-  if constexpr (HI - LO == 1)
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b[LO]) : "i"(LEFT));
-  else if constexpr (HI - LO == 2)
-    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b[LO]), "+v"(b[LO + 1]) : "i"(LEFT));
-  else if constexpr (HI - LO == 3)
-    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]) : "i"(LEFT));
-  else
-    asm volatile("s_waitcnt lgkmcnt(%4)"
-                 : "+v"(b[LO]), "+v"(b[LO + 1]), "+v"(b[LO + 2]), "+v"(b[LO + 3]) : "i"(LEFT));
-}
-
 // One 128-k block of a wave's NT x MT tile: per 32-k step, MT B-fragments
 // from the LDS stage and NT A-fragments dequantized from the block's weight
 // registers, tile-outer so that tile t+1 is dequantized (VALU) while tile t's

@@ -185,7 +185,7 @@ constexpr int kI8RowBytes = kI8Blk;      // one int8 x row per stage
 // as in the W4 GEMM: a read the compiler can see makes it wait for every
 // outstanding buffer -> LDS copy (vmcnt(0)) first, the next stage's included,
 // which serializes the copies with the math; these reads are completed by
-// lds_wait_first_half / lds_wait_rest.
+// lds_wait_frags.
 template <int OFF>
 __device__ __forceinline__ uint4_t i8_lds_read_off(uint32_t a) {
   uint4_t v;
@@ -283,14 +283,14 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(const int8_t* __restr
       const int c = 4 * step + kb;   // 16-byte chunk of this lane's k range
       uint4_t b[MT];
       i8_read_frags<MT>(b, stage + (uint32_t)(i8_swz(i, c) * 16));
-      lds_wait_first_half<MT>(b);
+      lds_wait_frags<MT, 0, MT / 2, MT - MT / 2>(b);
 #pragma unroll
-      for (int mt = 0; mt < (MT + 1) / 2; ++mt)
+      for (int mt = 0; mt < MT / 2; ++mt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t][mt] = mfma_i8(w[t][step], b[mt], acc[t][mt]);
-      lds_wait_rest<MT>(b);
+      lds_wait_frags<MT, MT / 2, MT, 0>(b);
 #pragma unroll
-      for (int mt = (MT + 1) / 2; mt < MT; ++mt)
+      for (int mt = MT / 2; mt < MT; ++mt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t][mt] = mfma_i8(w[t][step], b[mt], acc[t][mt]);
     }
@@ -361,14 +361,14 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(const int8_t* __restr
         const int c = 4 * step + kb;   // 16-byte chunk of this lane's k range
         uint4_t b[MT];
         i8_read_frags<MT>(b, stage + (uint32_t)(i8_swz(i, c) * 16));
-        lds_wait_first_half<MT>(b);
+        lds_wait_frags<MT, 0, MT / 2, MT - MT / 2>(b);
 #pragma unroll
-        for (int mt = 0; mt < (MT + 1) / 2; ++mt)
+        for (int mt = 0; mt < MT / 2; ++mt)
 #pragma unroll
           for (int t = 0; t < NT; ++t) acc[t][mt] = mfma_i8(cur[t][step], b[mt], acc[t][mt]);
-        lds_wait_rest<MT>(b);
+        lds_wait_frags<MT, MT / 2, MT, 0>(b);
 #pragma unroll
-        for (int mt = (MT + 1) / 2; mt < MT; ++mt)
+        for (int mt = MT / 2; mt < MT; ++mt)
 #pragma unroll
           for (int t = 0; t < NT; ++t) acc[t][mt] = mfma_i8(cur[t][step], b[mt], acc[t][mt]);
       }
