@@ -16,7 +16,10 @@ After the prefill and ``--warmup`` untimed steps, ``--steps`` steps are timed;
 ``value`` = steps / seconds (tok/s), compared with the reference's published
 26.358 tok/s (AWQ-INT4 + Marlin, RTX 3090, same workload).
 
-Also in the same JSON line:
+Also measured, in the same JSON line except for the per-case tables (``prefill``,
+``prefill_attention``, ``batch_sweep``, ``int8``, ``kernel_validation``,
+``decode_step_kernels``), which go to stderr and, with ``--report FILE``, to a
+file together with the rest:
 * ``gemv_pass``: the 280 per-projection decode GEMVs of one token
   (q, k, v, o, gate, up, down x 40 layers) replayed as one graph; GB/s of
   algorithmic bytes ``N*K/2 + N*(K/128)*2.5 + 2MK + 2MN``;
@@ -862,12 +865,23 @@ def kernel_sections(torch, native, model, runtime, cfg, args, device, capacity: 
     del src, dst
 
 
+# The per-case tables, about 20 KB: a reader of stdout that keeps only a tail of it (or a bounded line) would lose
+# the headline with them, so they go to stderr and to --report.
+TABLES = ('prefill', 'prefill_attention', 'batch_sweep', 'int8', 'kernel_validation', 'decode_step_kernels')
+
+
+def split_tables(result: dict) -> tuple[dict, dict]:
+    """(the stdout line, the tables) of a result."""
+    return ({k: v for k, v in result.items() if k not in TABLES}, {k: result[k] for k in TABLES if k in result})
+
+
 def main() -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument('--gpus', type=int, default=1)
     ap.add_argument('--steps', type=int, default=127, help='timed decode tokens')
     ap.add_argument('--warmup', type=int, default=5, help='untimed decode tokens before the timed ones')
     ap.add_argument('--layers', type=int, default=40)
+    ap.add_argument('--report', metavar='FILE', help='also write the whole result, tables included, to FILE')
     ap.add_argument('--no-cpu-baseline', action='store_true')
     ap.add_argument('--no-extras', action='store_true', help='skip the GEMV pass, kernel and prefill sections')
     args = ap.parse_args()
@@ -1001,15 +1015,12 @@ def main() -> int:
         log('cpu baseline')
         result['cpu_baseline'] = cpu_baseline(torch, native, device, args.layers)
 
-    # Bulky per-case tables first, the decode summary last: a reader that keeps
-    # only the tail of stdout still sees the step's kernels, the GEMV pass, the
-    # roofline and the CPU baseline.
-    last = ('decode_step_kernels', 'int8_e2e', 'e2e_w4_lm_head', 'prefill_seconds', 'prefill_tok_s',
-            'bytes_per_token', 'effective_gbs', 'pct_hbm_peak_effective', 'peak_allocated_gib',
-            'reference_peak_allocated_gib', 'gemv_pass', 'roofline', 'cpu_baseline')
-    ordered = {k: v for k, v in result.items() if k not in last}
-    ordered.update((k, result[k]) for k in last if k in result)
-    print(json.dumps(ordered), flush=True)
+    line, tables = split_tables(result)
+    log('tables ' + json.dumps(tables))
+    if args.report:
+        with open(args.report, 'w') as f:
+            json.dump(result, f)
+    print(json.dumps(line), flush=True)
     return 0
 
 

@@ -84,3 +84,14 @@ def test_in_step_time_is_bounded_by_the_kernels_own_time():
     broken = {k: {'us': 1.3, 'per_step': v['per_step']} for k, v in RECORDS.items()}
     assert bench.in_step_us(broken, (gu,), 40, own_us=21.5) is None
     assert bench.in_step_us(RECORDS, (gu,), 40, own_us=8.0) is None                   # more than 2x
+
+
+def test_the_stdout_line_holds_the_headline_without_the_tables():
+    contract = {'metric': 'm', 'value': 396.0, 'unit': 'tok/s', 'n_gpus': 1, 'steps': 20, 'warmup': 5, 'ms_per_step': 2.5,
+                'higher_is_better': True, 'scaling': 'weak', 'vs_baseline': 15.0, 'dtype': 'fp16', 'data': 'synthetic',
+                'config': {'workload': 'x'}}
+    result = {**contract, 'kernel_validation': {'rows': [[0.0] * 12] * 84}, 'batch_sweep': [{'us': 1.0}] * 30,
+              'decode_step_kernels': [{'op': 'x' * 200}] * 10, 'roofline': {'frac': 0.6}}
+    line, tables = bench.split_tables(result)
+    assert list(line)[:len(contract)] == list(contract) and {**line, **tables} == result
+    assert 'roofline' in line and set(tables) <= set(bench.TABLES) and not set(line) & set(bench.TABLES)
