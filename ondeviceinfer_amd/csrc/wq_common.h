@@ -92,8 +92,9 @@ constexpr int kNtPolicy = 2;   // non-temporal: data streamed once
 // 16x16x32 fragment read takes slot (2 kb + (w & 1) + 8 (w >> 1)) ^ i of row i
 // in k-step w.  ds_read_b128 serves lanes of neighbouring kb together, whose
 // slots have to differ below 128 bytes: with 4 kb + w, the order of the W4
-// tiles, half of the LDS cycles were bank conflicts, with this order none are (W4
-// 5120^2 M = 700 45.9 -> 45.4 us, fused gate_up M = 4096 1213 -> 1204).
+// tiles, half of the LDS cycles were bank conflicts, with this order none are.
+// The W4 GEMM's times moved by less than two runs of one build differ (under
+// 1 %: the matrix cores bound it), the INT8 form reads this way as well.
 __device__ __forceinline__ int frag_slot(int i, int kb, int w) { return (2 * kb + (w & 1) + 8 * (w >> 1)) ^ i; }
 
 // The chunk of row r that slot s holds: W4 tiles take k = 32 kb + 8 w (chunk

@@ -21,9 +21,10 @@
 // The tile shape follows the grid size (launch_gemm_auto); grids whose
 // blocks are too short to hide a load run a deep-ring form with several
 // blocks in flight (wq_gemm_deep_kernel), with the same block math; from
-// M = 4096 on, W4 row blocks are assigned to XCDs (gemm_coords).  The W4
-// kernel can also finish the Qwen3 MLP's elementwise ops in its epilogue
-// (Epi: silu(gate) * up over a fused [gate | up] weight, or a residual add).
+// M = 4096 on, the row blocks of W4 grids that have a multiple of 8 of them
+// are assigned to XCDs (gemm_coords).  Either format can also finish the Qwen3
+// MLP's elementwise ops in its epilogue (Epi: silu(gate) * up over a fused
+// [gate | up] weight, or a residual add).
 #include "wq_common.h"
 #include "wq_status.h"
 
@@ -627,9 +628,11 @@ __global__ __launch_bounds__(256) void wq_gemm_deep_kernel(const half_t* __restr
   gemm_store<F, NT, MT>(acc, tile0, ntile, m0, M, N, i, kb, wmeta, bias, y);
 }
 
-// Row blocks owned per XCD (gemm_coords) from M = 4096 on, for W4 (M = 4096:
-// fused gate_up 1274 -> 1241 us, down 681 -> 665 us; at M = 2048 it slows the
-// down projection, and the W8 GEMM gains nothing); 0 = launch order.
+// Row blocks owned per XCD (gemm_coords) from M = 4096 on, for W4 grids whose
+// row blocks divide by 8 (128-row tiles at M = 4096: fused gate_up 1274 -> 1241
+// us; at M = 2048 it slows the down projection, and the W8 GEMM gains nothing);
+// 0 = launch order.  q/o and down at M = 4096 run 112-row tiles in launch order,
+// 37 row blocks: 207 and 655 us against 218 and 697 on 128-row tiles with it.
 template <GFmt F>
 int xcd_rows(int M, unsigned grid_y) {
   return F == GFmt::W4 && M >= 4096 && grid_y % 8 == 0 ? (int)grid_y / 8 : 0;

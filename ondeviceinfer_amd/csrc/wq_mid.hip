@@ -27,16 +27,18 @@
 // rows keep the last arriver (mid_counts): they finish before the host has
 // queued a second launch (fused QKV M = 24 called from Python 11.5 us against
 // 13.3).
-// MI355X, graphs of distinct weights, us, previous kernels -> this one:
-//   W4 17408->5120    M = 8 / 24 / 40 / 56   20.5 / 35.8 / 49.7 / 65.1 -> 16.5 / 18.6 / 22.1 / 25.7
-//   W4 5120->7168     M = 24 / 40 / 56       13.0 / 18.1 / 23.2 -> 11.8 / 14.4 / 16.7
-//   W4 5120->17408    M = 8 / 24 / 40 / 56   22.5 / 27.5 / 40.0 / 56.2 -> 18.5 / 20.8 / 24.2 / 28.1
-//   W4 5120->34816    M = 8 / 24 / 40 / 56   27.9 / 35.9 / 49.3 / 50.6 -> 26.7 / 30.6 / 35.2 / 41.2
-//   INT8 17408->5120  M = 8 / 24 / 56        32.0 / 37.2 / 66.2 -> 20.4 / 21.7 / 30.6
-//   INT8 5120->17408  M = 8 / 24 / 56        25.5 / 36.4 / 71.3 -> 22.0 / 24.4 / 30.9
-//   INT8 5120->34816  M = 8 / 24 / 56        41.1 / 59.0 / 118 -> 33.4 / 35.8 / 47.1
-// i.e. 93 MB of W4 weights at M = 8 in 26.7 us (3.5 TB/s) and 178 MB of INT8
-// in 33.4 us (5.3 TB/s); what remains is about 6 us of launch, first load and
+// MI355X, graphs of distinct weights, us, the skinny kernels (W4 12..32 rows up
+// to 1152 tiles: wq_batch.hip, 17..64 rows from 2048 tiles on: the deep-ring
+// GEMM) -> this one:
+//   W4 17408->5120    M = 8 / 24 / 40 / 56   20.1 / 35.9 / 49.3 / 64.8 -> 15.9 / 18.7 / 21.6 / 24.9
+//   W4 5120->7168     M = 24 / 40 / 56       12.4 / 17.5 / 23.5 -> 11.7 / 14.0 / 16.2
+//   W4 5120->17408    M = 8 / 24 / 40 / 56   21.6 / 27.3 / 39.1 / 55.2 -> 17.4 / 21.0 / 23.9 / 27.2
+//   W4 5120->34816    M = 8 / 24 / 40 / 56   28.7 / 37.5 / 49.9 / 51.2 -> 27.5 / 31.4 / 35.6 / 40.4
+//   INT8 17408->5120  M = 8 / 24 / 56        31.4 / 37.8 / 66.7 -> 20.6 / 21.9 / 29.2
+//   INT8 5120->17408  M = 8 / 24 / 56        25.0 / 37.7 / 71.2 -> 21.7 / 24.4 / 28.3
+//   INT8 5120->34816  M = 8 / 24 / 56        46.6 / 62.4 / 120 -> 35.0 / 37.5 / 48.4
+// i.e. 93 MB of W4 weights at M = 8 in 27.5 us (3.4 TB/s) and 178 MB of INT8
+// in 35.0 us (5.1 TB/s); what remains is about 6 us of launch, first load and
 // partial sum, then 16 B per cycle and compute unit of weights and x.
 #include "wq_common.h"
 #include "wq_mid_plan.h"

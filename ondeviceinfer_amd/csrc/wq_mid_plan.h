@@ -42,11 +42,11 @@ inline size_t mid_partial_bytes(const MidSplit& m, int64_t nz, int mc) {
 //   six splits 1 us, their bytes out and back at 4 MB/us.
 // P = 4 or 5: eight or ten tiles a workgroup.  Ten is for grids of more than
 // 128 groups of eight, whose rounds it can even out: 5120->34816 (2176 tiles)
-// takes 218 workgroups in one round instead of 272 in two (W8A8 M = 48 48.3 ->
-// 34.9 us, INT8 M = 40 54 -> 41.8, W4 M = 40 43 -> 35.7), 5120->17408 in two
-// splits the same (W8A8 M = 48 27.6 -> 24.7 us).  On narrow N ten waves lost to
-// eight at the same bytes (W4 17408->5120 M = 8, seven splits: 18.2 us against
-// 15.0 with eight waves in six).
+// takes 218 workgroups in one round instead of 272 in two (us, eight -> ten:
+// W8A8 M = 48 51.5 -> 39.2, INT8 M = 40 55.7 -> 41.0, W4 M = 40 43 -> 36.5),
+// 5120->17408 in two splits the same (W8A8 M = 48 28.7 -> 26.0, INT8 M = 24 27.8
+// -> 24.1, W4 M = 56 30.7 -> 27.1; W4 M = 24 20.4 -> 20.7).  On narrow N ten waves
+// lost to eight at the same bytes (W4 17408->5120 M = 8 18.5 us against 15.8).
 // Beyond 64 rows ten waves' registers would spill.
 // w_tile / x_stage: bytes of one tile's weights and of the workgroup's x in one
 // stage; nst stages; nz row blocks; mc 16-row chunks.

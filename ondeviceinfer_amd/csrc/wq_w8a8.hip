@@ -413,12 +413,13 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(const int8_t* __restr
 // ahead; the two halves meet in LDS, S > 1 k ranges through int32 partials that
 // a second launch adds and scales.  The sums are exact integers, so every plan
 // gives the same bits.
-// MI355X, graphs of distinct weights, us with the quantizer, before -> now:
-//   17408->5120  M = 8 / 24 / 56 / 96 / 200   37.4 / 62.2 / 62.8 / 62.9 / 71.8 -> 24.4 / 25.8 / 29.9 / 34.1 / 48.3
-//   5120->17408  M = 8 / 24 / 56              27.2 / 32.2 / 37.6 -> 24.7 / 26.2 / 30.7
-//   5120->34816  M = 8 / 24 / 56              45.4 / 44.5 / 67.5 -> 36.4 / 38.1 / 43.6
-//   5120->5120   M = 16 / 56 / 96             17.1 / 23.9 / 24.1 -> 14.7 / 19.4 / 20.9
-// i.e. 178 MB of weights at M = 8 in 32 us without the quantizer (5.6 TB/s).
+// MI355X, graphs of distinct weights, us without the quantizer, GEMV or 32-row
+// GEMM -> this kernel:
+//   17408->5120  M = 8 / 24 / 56 / 96 / 200   31.3 / 52.9 / 53.2 / 53.8 / 60.7 -> 20.5 / 21.5 / 24.3 / 28.3 / 42.0
+//   5120->17408  M = 8 / 24 / 56              23.6 / 26.8 / 31.7 -> 21.6 / 22.4 / 27.3
+//   5120->34816  M = 8 / 24 / 56              42.9 / 41.5 / 63.6 -> 35.0 / 36.8 / 41.3
+//   5120->5120   M = 16 / 56 / 96             12.7 / 18.5 / 18.5 -> 11.1 / 15.9 / 16.1
+// i.e. 178 MB of weights at M = 8 in 35 us (5.1 TB/s).
 constexpr int kM8Tiles = kMidTilesPerWave;
 constexpr int kM8MaxM = 255;   // from 256 rows the GEMM takes 128-row tiles
 constexpr int kM8GemvMaxM = 16;
