@@ -338,7 +338,7 @@ def shared_workspace(device: torch.device, nbytes: int, layout: tuple, zeroed: i
     ``('w4a16', n, k, group)``): the kernels return the counters to zero after
     every call but leave partials behind, so calls share a buffer only if they
     have the same layout and are ordered on one stream.  A call under capture
-    takes a buffer of that capture's own, cleared at the graph's start: the
+    takes a buffer of that capture's own, cleared where the graph first uses it: the
     graph may be replayed on any stream, beside eager calls and other graphs.
     It comes from the graph's memory pool, so this module keeps it only while
     the capture may still ask for it (the last ``_MAX_CAPTURES`` captures).
