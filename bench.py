@@ -872,7 +872,12 @@ TABLES = ('prefill', 'prefill_attention', 'batch_sweep', 'int8', 'kernel_validat
 
 def split_tables(result: dict) -> tuple[dict, dict]:
     """(the stdout line, the tables) of a result."""
-    return ({k: v for k, v in result.items() if k not in TABLES}, {k: result[k] for k in TABLES if k in result})
+    line = {k: v for k, v in result.items() if k not in TABLES}
+    tables = {k: result[k] for k in TABLES if k in result}
+    if 'shapes' in (line.get('cpu_baseline') or {}):
+        line['cpu_baseline'] = {k: v for k, v in line['cpu_baseline'].items() if k != 'shapes'}
+        tables['cpu_baseline_shapes'] = result['cpu_baseline']['shapes']
+    return line, tables
 
 
 def main() -> int:

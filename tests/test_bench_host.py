@@ -95,3 +95,7 @@ def test_the_stdout_line_holds_the_headline_without_the_tables():
     line, tables = bench.split_tables(result)
     assert list(line)[:len(contract)] == list(contract) and {**line, **tables} == result
     assert 'roofline' in line and set(tables) <= set(bench.TABLES) and not set(line) & set(bench.TABLES)
+    result['cpu_baseline'] = {'value': 0.04, 'kind': 'port', 'shapes': [{'op': 'x'}] * 5}
+    line, tables = bench.split_tables(result)
+    assert line['cpu_baseline'] == {'value': 0.04, 'kind': 'port'} and len(tables['cpu_baseline_shapes']) == 5
+    assert len(result['cpu_baseline']['shapes']) == 5
